@@ -55,6 +55,11 @@ struct FanTables {
     std::vector<double> h_view, h_p, h_zero;
     std::vector<float> h_pf, h_gam, h_colw, h_xf;
     DevBuf d_view, d_p, d_zero, d_pf, d_gam, d_colw, d_xf;
+    // exact adjoint, built on its first use: bin index over the detector, ray records
+    uint64_t adj_key = 0;
+    std::vector<int> h_lut;
+    double lut_lo = 0, lut_scale = 0;
+    DevBuf d_lut, d_rays;
 };
 
 struct ParTables {
@@ -167,6 +172,12 @@ ctr_status fail(ctr_ctx *ctx, ctr_status st, const char *fmt, ...)
     do {                                                                                                \
         hipError_t e_ = (expr);                                                                         \
         if (e_ != hipSuccess) return fail((ctx), CTR_EHIP, "%s: %s", #expr, hipGetErrorString(e_));     \
+    } while (0)
+
+#define TRY(expr)                          \
+    do {                                   \
+        ctr_status s_ = (expr);            \
+        if (s_ != CTR_OK) return s_;       \
     } while (0)
 
 int parse_fault()
@@ -722,6 +733,49 @@ FanParams fan_params(ctr_ctx *ctx, const ctr_fan_geom *g, unsigned flags)
     return P;
 }
 
+// Tables of the exact fan adjoint, once per geometry: the bin index (first bin
+// at or above each of 4 n_p positions over the detector) and the ray records.
+// Records take 16 bytes per ray; beyond 2^26 rays (1 GiB) the kernel forms them
+// as it goes.
+ctr_status fan_adjoint_tables(ctr_ctx *ctx, const ctr_fan_geom *g, FanParams &P)
+{
+    FanTables &T = ctx->fan;
+    const int np = g->n_p;
+    const bool asc = g->p[np - 1] >= g->p[0];
+    const size_t nray = (size_t)g->n_beta * np;
+    const bool table = nray <= ((size_t)1 << 26);
+    const double lo = asc ? g->p[0] : g->p[np - 1], hi = asc ? g->p[np - 1] : g->p[0];
+    const int cells = std::min(4 * (size_t)np, (size_t)1 << 16);
+    P.asc = asc;
+    P.lut_n = cells;
+    if (T.adj_key != T.key || !T.d_lut.ptr) {
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));   // queued work may still read the old tables
+        T.adj_key = 0;
+        const double h = hi > lo ? (hi - lo) / cells : 1.0;
+        T.lut_lo = (double)(float)lo;
+        T.lut_scale = (double)(float)(1.0 / h);
+        T.h_lut.resize((size_t)cells + 1);
+        int c = 0;
+        for (int k = 0; k <= cells; ++k) {
+            const double edge = k == cells ? std::numeric_limits<double>::infinity() : T.lut_lo + k / T.lut_scale;
+            while (k > 0 && c < np && (asc ? g->p[c] : g->p[np - 1 - c]) < edge) ++c;
+            T.h_lut[k] = c;
+        }
+        TRY(upload(ctx, T.d_lut, T.h_lut.data(), sizeof(int) * T.h_lut.size()));
+        if (table) {
+            TRY(buf_reserve(ctx, T.d_rays, nray * sizeof(double2)));
+            TRY(check_launch(ctx, launch_fan_ray_table(P, (double2 *)T.d_rays.ptr, ctx->stream), "fan ray records"));
+        }
+        T.adj_key = T.key;
+    }
+    P.lut_lo = (float)T.lut_lo;
+    P.lut_scale = (float)T.lut_scale;
+    P.lut_eps = (float)(1e-3 + 1e-6 * (hi - lo));
+    P.lut = (const int *)T.d_lut.ptr;
+    if (table) P.rays = (const double2 *)T.d_rays.ptr;
+    return CTR_OK;
+}
+
 uint64_t par_key(const ctr_par_geom *g)
 {
     uint64_t h = 1469598103934665603ull;
@@ -1058,12 +1112,6 @@ size_t nrayp(const ctr_par_geom *g) { return (size_t)g->n_theta * g->n_t; }
 size_t nvoxc(const ctr_curved_geom *g) { return (size_t)g->nt * g->ns * g->nz; }
 size_t nrayc(const ctr_curved_geom *g) { return (size_t)g->n_beta * g->n_gamma * g->n_xi; }
 
-#define TRY(expr)                          \
-    do {                                   \
-        ctr_status s_ = (expr);            \
-        if (s_ != CTR_OK) return s_;       \
-    } while (0)
-
 ctr_status cone_filter_impl(ctr_ctx *ctx, const ctr_cone_geom *g, int filter, const float *in, float *out)
 {
     if (g->n_p > 2048) return fail(ctx, CTR_ETOOBIG, "ramp filter supports at most 2048 detector columns");
@@ -1308,7 +1356,8 @@ void ctr_ctx_destroy(ctr_ctx *ctx)
     for (auto &b : ctx->ws) buf_free(b);
     for (DevBuf *b : {&ctx->cone.d_view, &ctx->cone.d_p, &ctx->cone.d_xi, &ctx->cone.d_bp, &ctx->cone.d_pf,
                       &ctx->cone.d_xf, &ctx->cone.d_zq, &ctx->fan.d_view, &ctx->fan.d_p, &ctx->fan.d_zero, &ctx->fan.d_pf,
-                      &ctx->fan.d_gam, &ctx->fan.d_colw, &ctx->fan.d_xf, &ctx->taps.d, &ctx->taps.d_spec, &ctx->foot_bp.buf, &ctx->foot_adj.buf})
+                      &ctx->fan.d_gam, &ctx->fan.d_colw, &ctx->fan.d_xf, &ctx->fan.d_lut,
+                      &ctx->fan.d_rays, &ctx->taps.d, &ctx->taps.d_spec, &ctx->foot_bp.buf, &ctx->foot_adj.buf})
         buf_free(*b);
     if (ctx->own) (void)hipStreamDestroy(ctx->own);
     delete ctx;
@@ -1583,6 +1632,7 @@ ctr_status ctr_fan_bp_adjoint(ctr_ctx *ctx, const ctr_fan_geom *g, const float *
     TRY(stage_in(ctx, dev, kWsIn, proj, nray2(g), &dp));
     TRY(stage_out(ctx, dev, (flags & CTR_ACCUMULATE) != 0, kWsOut, img, nvox2(g), &di));
     FanParams P = fan_params(ctx, g, flags);
+    TRY(fan_adjoint_tables(ctx, g, P));
     TRY(check_launch(ctx, launch_fan_adjoint(P, dp, di, nullptr, 0, ctx->stream), "fan adjoint"));
     return finish_out(ctx, dev, di, img, nvox2(g));
 }
@@ -2081,7 +2131,8 @@ ctr_status ctr_sirt2d(ctr_ctx *ctx, const ctr_fan_geom *g, const float *b, float
     TRY(sirt_opts_check(ctx, opts));
     TRY(fan_tables(ctx, g));
     const RayParams R = fan_ray_params(ctx, g);
-    const FanParams P = fan_params(ctx, g, 0);
+    FanParams P = fan_params(ctx, g, 0);
+    TRY(fan_adjoint_tables(ctx, g, P));
     auto fp = [&](const float *xx, const float *bb, float *rr, double *part, int *nblk) {
         RayParams Rx = R;
         TRY(fp_transposed(ctx, Rx, xx, ctx->ws[kWsT], ctx->stream));

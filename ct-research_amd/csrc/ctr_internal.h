@@ -177,6 +177,13 @@ struct FanParams {
     int accumulate;
     int quirks;
     int equiangular;
+    // exact adjoint: lut[k] is the first bin, counted in ascending position, at
+    // or above lut_lo + k / lut_scale (k = 0 .. lut_n); asc: the detector ascends;
+    // lut_eps: the margin in mm that covers the float arithmetic of a look-up
+    int asc, lut_n;
+    float lut_lo, lut_scale, lut_eps;
+    const int *lut;
+    const double2 *rays;    // [nb][np] ray records (launch_fan_ray_table), or null
 };
 
 // ---- launchers (return hipError_t of the launch) --------------------------
@@ -305,6 +312,7 @@ hipError_t noalloc_scratch(int device, void **ptr);
 hipError_t launch_filter_tables(int filter, double d, int n, int L, double *taps, double *spec, hipStream_t st);
 
 hipError_t launch_fan_bp_ref(const FanParams &P, const float *proj, float *img, hipStream_t st);
+hipError_t launch_fan_ray_table(const FanParams &P, double2 *rays, hipStream_t st);
 hipError_t launch_fan_adjoint(const FanParams &P, const float *proj, float *img, const SirtUpdate *upd,
                               int ones_input, hipStream_t st);
 hipError_t launch_fan_fbp_bp(const FanParams &P, const float *filt, float *img, hipStream_t st);
