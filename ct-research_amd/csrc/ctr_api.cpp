@@ -607,9 +607,24 @@ ctr_status fp_transposed(ctr_ctx *ctx, RayParams &R, const float *vol, DevBuf &b
     if (!enable) return CTR_OK;
     ctr_status s = buf_reserve(ctx, buf, (size_t)R.nt * R.ns * R.nz * sizeof(float));
     if (s != CTR_OK) return s;
-    s = check_launch(ctx, launch_transpose_st(vol, (float *)buf.ptr, R.nt, R.ns, R.nz, st), "volume transpose");
+    s = check_launch(ctx, launch_transpose_st(vol, (float *)buf.ptr, nullptr, R.nt, R.ns, R.nz, st), "volume transpose");
     if (s != CTR_OK) return s;
     R.volT = (const float *)buf.ptr;
+    return CTR_OK;
+}
+
+// The 2-D projector's image: a copy of it followed by its transpose, so that
+// every ray of a wavefront reads along its own axis from one buffer.  Images
+// above 2^28 pixels (whose pair would pass the 32-bit offsets) keep the 3-D
+// kernel and its transposed copy.
+ctr_status fp_flat(ctr_ctx *ctx, RayParams &R, const float *img, DevBuf &buf, hipStream_t st)
+{
+    const size_t n = (size_t)R.nt * R.ns;
+    if (n > ((size_t)1 << 28)) return fp_transposed(ctx, R, img, buf, st);
+    TRY(buf_reserve(ctx, buf, 2 * n * sizeof(float)));
+    float *pair = (float *)buf.ptr;
+    TRY(check_launch(ctx, launch_transpose_st(img, pair + n, pair, R.nt, R.ns, 1, st), "image transpose"));
+    R.flat = pair;
     return CTR_OK;
 }
 
@@ -1601,7 +1616,7 @@ ctr_status ctr_fan_fp(ctr_ctx *ctx, const ctr_fan_geom *g, const float *img, flo
     TRY(stage_in(ctx, dev, kWsIn, img, nvox2(g), &di));
     TRY(stage_out(ctx, dev, false, kWsOut, proj, nray2(g), &dp));
     RayParams R = fan_ray_params(ctx, g);
-    TRY(fp_transposed(ctx, R, di, ctx->ws[kWsT], ctx->stream));
+    TRY(fp_flat(ctx, R, di, ctx->ws[kWsT], ctx->stream));
     TRY(check_launch(ctx, launch_ray_fp(R, di, dp, ctx->stream), "fan forward projection"));
     return finish_out(ctx, dev, dp, proj, nray2(g));
 }
@@ -1698,7 +1713,7 @@ ctr_status ctr_par_fp(ctr_ctx *ctx, const ctr_par_geom *g, const float *img, flo
     TRY(stage_in(ctx, dev, kWsIn, img, npix(g), &di));
     TRY(stage_out(ctx, dev, false, kWsOut, proj, nrayp(g), &dp));
     RayParams R = par_ray_params(ctx, g);
-    TRY(fp_transposed(ctx, R, di, ctx->ws[kWsT], ctx->stream));
+    TRY(fp_flat(ctx, R, di, ctx->ws[kWsT], ctx->stream));
     TRY(check_launch(ctx, launch_ray_fp(R, di, dp, ctx->stream), "parallel forward projection"));
     return finish_out(ctx, dev, dp, proj, nrayp(g));
 }
@@ -2135,7 +2150,7 @@ ctr_status ctr_sirt2d(ctr_ctx *ctx, const ctr_fan_geom *g, const float *b, float
     TRY(fan_adjoint_tables(ctx, g, P));
     auto fp = [&](const float *xx, const float *bb, float *rr, double *part, int *nblk) {
         RayParams Rx = R;
-        TRY(fp_transposed(ctx, Rx, xx, ctx->ws[kWsT], ctx->stream));
+        TRY(fp_flat(ctx, Rx, xx, ctx->ws[kWsT], ctx->stream));
         return check_launch(ctx, launch_ray_fp_residual(Rx, xx, bb, rr, part, nblk, ctx->stream), "SIRT residual");
     };
     auto ones = [&](float *vinv) {
@@ -3087,7 +3102,7 @@ ctr_status ctr_sirt3d_batched(ctr_ctx *ctx, const ctr_sirt_problem *pr, int n, c
                 const BatchProblem &q = B.probs[p];
                 hipStream_t t = B.ws[p % nstreams];
                 if (q.R.volT)
-                    TRY(check_launch(ctx, launch_transpose_st(q.xp, (float *)q.vt.ptr, q.R.nt, q.R.ns, q.R.nz, t),
+                    TRY(check_launch(ctx, launch_transpose_st(q.xp, (float *)q.vt.ptr, nullptr, q.R.nt, q.R.ns, q.R.nz, t),
                                      "volume transpose"));
                 int nblk = 0;
                 TRY(check_launch(ctx, launch_ray_fp_residual(q.R, q.xp, q.bp, (float *)q.r.ptr, (double *)q.part.ptr,
@@ -3107,7 +3122,7 @@ ctr_status ctr_sirt3d_batched(ctr_ctx *ctx, const ctr_sirt_problem *pr, int n, c
             for (int p = 0; p < n; ++p) {
                 const BatchProblem &q = B.probs[p];
                 if (q.R.volT)
-                    TRY(check_launch(ctx, launch_transpose_st(q.xp, (float *)q.vt.ptr, q.R.nt, q.R.ns, q.R.nz, s),
+                    TRY(check_launch(ctx, launch_transpose_st(q.xp, (float *)q.vt.ptr, nullptr, q.R.nt, q.R.ns, q.R.nz, s),
                                      "volume transpose"));
             }
             TRY(check_launch(ctx, launch_ray_fp_residual_batched(dfp, n, fp_max, s), "batched residual"));

@@ -29,6 +29,8 @@ struct RayParams {
                             // central ray runs mostly along t (neighbouring rays then differ in s)
     int parallel;           // parallel beam: ray (view, p) is the line through centre + p (cos, sin)
                             // along (-sin, cos); view[4b+2..3] unused
+    const float *flat;      // 2-D image (one slice, one detector row at its height: fan, parallel beam):
+                            // the image [nt*ns] followed by its transpose, at most 2^29 floats together
     int residual_norm;      // the SIRT residual pass stores r times the ray norm (the cone
                             // adjoint's input form); the fan adjoint reads r itself
     int skip_empty;         // a slab's second and third voxels are read only by lanes whose
@@ -372,7 +374,8 @@ hipError_t launch_diff_sums(const float *x, const float *ref, size_t n, double *
 
 // Utilities.
 hipError_t launch_fill(float *dst, float value, size_t n, hipStream_t st);
-hipError_t launch_transpose_st(const float *in, float *out, int nt, int ns, int nz, hipStream_t st);   // [z][t][s] <- [z][s][t]
+// out [z][t][s] from in [z][s][t]; copy: null, or where in itself goes as well
+hipError_t launch_transpose_st(const float *in, float *out, float *copy, int nt, int ns, int nz, hipStream_t st);
 hipError_t launch_reciprocal_eps(float *v, size_t n, float eps, hipStream_t st);   // v <- 1/(v+eps)
 // Deterministic sum of n (a, b) pairs into out2[0..1].  Above kReduceDirect
 // pairs it runs in two stages and writes up to kReduceSlack stage pairs after

@@ -482,12 +482,221 @@ __global__ __launch_bounds__(kBX *kBY) void k_ray_fp_residual_batched(const FpJo
     fp_residual_block(jobs[p].vol, jobs[p].b, jobs[p].r, jobs[p].partials, g, bx, by, ib, (size_t)local);
 }
 
+// ---------------------------------------------------------------------------
+// 2-D images (one slice, one detector row: fan and parallel beams).  The
+// crossings, segments and float operations are those of trace_ray without the
+// third axis, in the same order (a residual history of SIRT shows a rounding of
+// another kind at 1e-8), laid out for what a 2-D problem lacks, rays and
+// wavefronts:
+//   - a wavefront holds 64 neighbouring rays of the one detector row (the
+//     16 x 4 layout of the cone beam would leave 48 of its lanes empty);
+//   - each ray walks the slabs of the axis with its own shorter step, so it
+//     meets at most one crossing of the other axis in a slab (two that coincide
+//     but for rounding are taken in two slabs, the second segment a rounding
+//     short) and none has to walk crossing by crossing;
+//   - rays read the image or its transpose, whichever has their other axis
+//     fastest, from one buffer that holds both;
+//   - the weights and offsets of kFlatUnroll slabs are formed ahead of their
+//     loads, so that many gathers are in flight at three wavefronts per SIMD.
+// 256^2 / 360 views / 512 bins, residual pass: 144 us in the cone beam's
+// kernel, 37 us here, bound by VALU issue (15 instructions a slab) and by the
+// gathers' latency in turn; without the second layout, rays of the other axis
+// in a wavefront cost 65 us.
+// ---------------------------------------------------------------------------
+constexpr int kFlatUnroll = 8, kFlatWaves = 4;
+
+__device__ __forceinline__ float trace_ray_flat(const RayParams &g, int ib, int ip, bool valid, float &chord)
+{
+    RayWalk w;
+    const bool go = valid && ray_walk(g, ib, ip, 0, false, w);
+    chord = go ? (float)w.lam_end : 0.0f;
+    if (__ballot(go) == 0) return 0.0f;
+    const int npix = g.nt * g.ns;
+    __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)g.flat, 0, (int)((unsigned)npix * 8u), kBufDword3);
+    const bool lane_t = w.at.stride != 0 && (w.as.stride == 0 || w.at.step <= w.as.step);
+    const AxisSetup aD = lane_t ? w.at : w.as;
+    const AxisSetup aA = lane_t ? w.as : w.at;
+    const int sgnD = aD.stride > 0 ? 1 : -1, sgnA = aA.stride > 0 ? 1 : (aA.stride < 0 ? -1 : 0);
+    const unsigned sA = (unsigned)sgnA * 4u, sD = (unsigned)(sgnD * (lane_t ? g.ns : g.nt)) * 4u;
+    const unsigned idx0 = lane_t ? (unsigned)(npix + w.at.i0 * g.ns + w.as.i0) : (unsigned)w.idx0;
+
+    // trace_ray's 16 neighbouring rays that do not all have the view's axis as
+    // their shorter one walk crossing by crossing, with one segment behind the
+    // last counted crossing; the others cut that segment at lcnt
+    const bool along_t = fabs(g.view[4 * ib + 0]) > fabs(g.view[4 * ib + 1]);
+    const AxisSetup &vD = along_t ? w.at : w.as, &vA = along_t ? w.as : w.at;
+    const bool odd = go && !(vD.stride != 0 && (vA.n == 0 || vA.step >= 1.001 * vD.step));
+    const unsigned long long of_group = 0xffffull << (__lane_id() & 48);
+    const bool one_tail = (__ballot(odd) & of_group) != 0 ||
+                          ((__ballot(go && vD.stride > 0) & of_group) != 0 && (__ballot(go && vD.stride < 0) & of_group) != 0);
+
+    // slab index relative to the first slab of the wavefront's rays of the same
+    // axis and direction, so that these read one image row together
+    const int kind = (lane_t ? 2 : 0) + (sgnD > 0 ? 1 : 0), from = sgnD * aD.i0;
+    int istart = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const bool same = go && kind == c;
+        if (__ballot(same) == 0) continue;
+        const int m = wave_min_int(same ? from : 0x7fffffff);
+        istart = same ? m : istart;
+    }
+    const int o = go ? from - istart : (1 << 30);
+    const int uend = __builtin_amdgcn_readfirstlane(wave_max_int(go ? o + aD.n : -1));
+    const int nD = go ? aD.n : 0;
+
+    const float inf = __builtin_huge_valf();
+    const float D0 = go ? (float)aD.next0 : inf, dD = go ? (float)aD.step : 0.0f;
+    const float A0 = go && aA.n > 0 ? (float)aA.next0 : inf, dA = go ? (float)aA.step : 0.0f;
+    const float lend = go ? (float)w.lam_end : 0.0f;
+    const float near_end = __builtin_bit_cast(float, max(__builtin_bit_cast(int, lend) - 8, 0));
+    const float lcnt = one_tail ? lend : near_end, most = one_tail ? (float)aA.n : inf;
+    const int last = one_tail ? nD : -1;   // the slab that ends at the exit, whatever its plane's float parameter
+    unsigned off = idx0 * 4u;
+    float pA = A0, cA = 0.0f, s = 0.0f, sum = 0.0f;
+    const float ninf = opaque_ninf();
+    float w1[kFlatUnroll], w2[kFlatUnroll], v1[kFlatUnroll], v2[kFlatUnroll];
+    unsigned o1[kFlatUnroll];
+    for (int u = 0; u <= uend; u += kFlatUnroll) {
+        const int k0 = u - o;
+        const float kf = (float)k0;
+        // all slabs of the block lie on every ray and end before its last
+        // counted crossing: no clamps, no masks
+        const bool inner = k0 >= 0 && k0 + kFlatUnroll - 1 < nD && fmaf(kf + (float)(kFlatUnroll - 1), dD, D0) <= near_end;
+        if (__ballot(!inner) == 0) {
+#pragma unroll
+            for (int q = 0; q < kFlatUnroll; ++q) {
+                const float e = fmaf(kf + (float)q, dD, D0);
+                const bool hasA = pA < e;
+                const float p1 = min_nc(pA, e, ninf);
+                w1[q] = p1 - s;
+                w2[q] = e - p1;
+                o1[q] = off;
+                off += (hasA ? sA : 0u) + sD;
+                cA = hasA ? cA + 1.0f : cA;
+                pA = fmaf(cA, dA, A0);
+                s = e;
+            }
+#pragma unroll
+            for (int q = 0; q < kFlatUnroll; ++q) {
+                v1[q] = load_vox(rs, o1[q]);
+                v2[q] = load_vox(rs, o1[q] + sA);
+            }
+#pragma unroll
+            for (int q = 0; q < kFlatUnroll; ++q) {
+                sum = fmaf(w1[q], v1[q], sum);
+                sum = fmaf(w2[q], v2[q], sum);
+            }
+        } else {
+            // a slab outside the ray gets weights of 0 and offsets past the
+            // image, which read 0; the segment behind the last counted
+            // crossing, if there is one, follows its slab's other two
+            float w3[kFlatUnroll];
+            unsigned o2[kFlatUnroll], o3[kFlatUnroll];
+#pragma unroll
+            for (int q = 0; q < kFlatUnroll; ++q) {
+                const bool act = go && (unsigned)(k0 + q) <= (unsigned)nD;
+                const float plane = min_nc(fmaf(kf + (float)q, dD, D0), lend, ninf);
+                const float e = k0 + q == last ? lend : plane;
+                const float ec = min_nc(e, lcnt, ninf);
+                const bool hasA = act && pA < ec && cA < most;
+                const float p1 = hasA ? pA : ec;
+                w1[q] = act ? p1 - s : 0.0f;
+                w2[q] = act ? ec - p1 : 0.0f;
+                w3[q] = act ? e - ec : 0.0f;
+                o1[q] = act ? off : 0xFFFFFFFCu;
+                o2[q] = act ? off + sA : 0xFFFFFFFCu;
+                o3[q] = off + (hasA ? sA : 0u);
+                cA = hasA ? cA + 1.0f : cA;
+                pA = fmaf(cA, dA, A0);
+                off = act ? o3[q] + sD : off;
+                s = act ? e : s;
+            }
+#pragma unroll
+            for (int q = 0; q < kFlatUnroll; ++q) {
+                v1[q] = load_vox(rs, o1[q]);
+                v2[q] = load_vox(rs, o2[q]);
+            }
+#pragma unroll
+            for (int q = 0; q < kFlatUnroll; ++q) {
+                sum = fmaf(w1[q], v1[q], sum);
+                sum = fmaf(w2[q], v2[q], sum);
+                if (w3[q] != 0.0f) sum = fmaf(w3[q], load_vox(rs, o3[q]), sum);
+            }
+        }
+    }
+    return sum;
+}
+
+// Wavefront `wave` of the launch: 64 columns of one view.
+__device__ __forceinline__ bool flat_item(const RayParams &g, int &ib, int &ip)
+{
+    const int chunks = (g.np + 63) / 64;
+    const long item = (long)blockIdx.x * kFlatWaves + __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    ib = (int)(item / chunks);
+    ip = (int)(item - (long)ib * chunks) * 64 + (int)threadIdx.x;
+    return ib < g.nb;
+}
+
+__global__ __launch_bounds__(64 * kFlatWaves) void k_ray_fp_flat(float *__restrict__ proj, RayParams g)
+{
+    int ib, ip;
+    if (!flat_item(g, ib, ip)) return;
+    float chord;
+    const float acc = trace_ray_flat(g, ib, ip, ip < g.np, chord);
+    if (ip < g.np) proj[(size_t)ib * g.np + ip] = acc;
+}
+
+// The residual pass (fp_residual_block) of a 2-D problem.
+__global__ __launch_bounds__(64 * kFlatWaves) void k_ray_fp_residual_flat(const float *__restrict__ b,
+                                                                          float *__restrict__ r,
+                                                                          double *__restrict__ partials, RayParams g)
+{
+    __shared__ double red[2][kFlatWaves];
+    int ib, ip;
+    double e2 = 0.0, e1 = 0.0;
+    if (flat_item(g, ib, ip)) {
+        float chord;
+        const float acc = trace_ray_flat(g, ib, ip, ip < g.np, chord);
+        if (ip < g.np) {
+            const size_t ray = (size_t)ib * g.np + ip;
+            const float e = b[ray] - acc;
+            r[ray] = e / (chord + 1e-9f);
+            e2 = (double)e * (double)e;
+            e1 = fabs((double)e);
+        }
+    }
+    e2 = wave_sum(e2);
+    e1 = wave_sum(e1);
+    if (threadIdx.x == 0) {
+        red[0][threadIdx.y] = e2;
+        red[1][threadIdx.y] = e1;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && threadIdx.y == 0) {
+        double s2 = 0.0, s1 = 0.0;
+        for (int w = 0; w < kFlatWaves; ++w) {
+            s2 += red[0][w];
+            s1 += red[1][w];
+        }
+        partials[2 * (size_t)blockIdx.x] = s2;
+        partials[2 * (size_t)blockIdx.x + 1] = s1;
+    }
+}
+
+unsigned flat_blocks(const RayParams &g)
+{
+    const long items = (long)((g.np + 63) / 64) * g.nb;
+    return (unsigned)((items + kFlatWaves - 1) / kFlatWaves);
+}
+
 dim3 fp_grid(const RayParams &g) { return dim3((g.np + kBX - 1) / kBX, (g.nx + kBY - 1) / kBY, g.nb); }
 
 }  // namespace
 
 int ray_fp_blocks(const RayParams &g)
 {
+    if (g.flat) return (int)flat_blocks(g);
     const dim3 grid = fp_grid(g);
     return (int)(grid.x * grid.y * grid.z);
 }
@@ -508,6 +717,10 @@ hipError_t launch_sysmat_fill(const RayParams &g, const long long *row_ptr, int 
 
 hipError_t launch_ray_fp(const RayParams &g, const float *vol, float *proj, hipStream_t st)
 {
+    if (g.flat) {
+        hipLaunchKernelGGL(k_ray_fp_flat, dim3(flat_blocks(g)), dim3(64, kFlatWaves), 0, st, proj, g);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(k_ray_fp, fp_grid(g), dim3(kBX, kBY), 0, st, vol, proj, g);
     return hipGetLastError();
 }
@@ -515,6 +728,11 @@ hipError_t launch_ray_fp(const RayParams &g, const float *vol, float *proj, hipS
 hipError_t launch_ray_fp_residual(const RayParams &g, const float *vol, const float *b, float *r, double *partials,
                                   int *nblocks, hipStream_t st)
 {
+    if (g.flat) {
+        *nblocks = (int)flat_blocks(g);
+        hipLaunchKernelGGL(k_ray_fp_residual_flat, dim3(flat_blocks(g)), dim3(64, kFlatWaves), 0, st, b, r, partials, g);
+        return hipGetLastError();
+    }
     const dim3 grid = fp_grid(g);
     *nblocks = (int)(grid.x * grid.y * grid.z);
     hipLaunchKernelGGL(k_ray_fp_residual, grid, dim3(kBX, kBY), 0, st, vol, b, r, partials, g);

@@ -112,9 +112,10 @@ __global__ void k_iter_inc(int *iter)
     if (threadIdx.x == 0) iter[0] = iter[0] + 1;
 }
 
-// out[z][t][s] = in[z][s][t]: 32 x 32 tiles through LDS (padded row against bank conflicts).
-__global__ __launch_bounds__(256) void k_transpose_st(const float *__restrict__ in, float *__restrict__ out, int nt,
-                                                      int ns)
+// out[z][t][s] = in[z][s][t]: 32 x 32 tiles through LDS (padded row against
+// bank conflicts); with copy, also copy[z][s][t] = in[z][s][t].
+__global__ __launch_bounds__(256) void k_transpose_st(const float *__restrict__ in, float *__restrict__ out,
+                                                      float *__restrict__ copy, int nt, int ns)
 {
     __shared__ float tile[32][33];
     const int t0 = blockIdx.x * 32, s0 = blockIdx.y * 32;
@@ -122,7 +123,11 @@ __global__ __launch_bounds__(256) void k_transpose_st(const float *__restrict__ 
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 32 x 8
     for (int k = ty; k < 32; k += 8) {
         const int t = t0 + tx, s = s0 + k;
-        if (t < nt && s < ns) tile[k][tx] = in[zo + (size_t)s * nt + t];
+        if (t < nt && s < ns) {
+            const float v = in[zo + (size_t)s * nt + t];
+            tile[k][tx] = v;
+            if (copy) copy[zo + (size_t)s * nt + t] = v;
+        }
     }
     __syncthreads();
     for (int k = ty; k < 32; k += 8) {
@@ -355,9 +360,9 @@ hipError_t launch_reduce_jobs(const ReduceJob *jobs, int njobs, const int *iter,
     return hipGetLastError();
 }
 
-hipError_t launch_transpose_st(const float *in, float *out, int nt, int ns, int nz, hipStream_t st)
+hipError_t launch_transpose_st(const float *in, float *out, float *copy, int nt, int ns, int nz, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_transpose_st, dim3((nt + 31) / 32, (ns + 31) / 32, nz), dim3(256), 0, st, in, out, nt, ns);
+    hipLaunchKernelGGL(k_transpose_st, dim3((nt + 31) / 32, (ns + 31) / 32, nz), dim3(256), 0, st, in, out, copy, nt, ns);
     return hipGetLastError();
 }
 
