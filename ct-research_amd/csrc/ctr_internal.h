@@ -13,6 +13,27 @@ namespace ctr {
 
 constexpr float kInf = __builtin_huge_valf();
 
+// Voxel columns (cells) that the rays of one detector column cross, seen from
+// above (k_ray_cells), for `views` views at a time.
+struct ColumnHead {
+    double lo, len;         // in-plane entry parameter (from the source) and length through the box
+    double inv_rho;         // 1 / in-plane distance from the source to the detector column
+    int n;                  // cells, padded to an even number of blocks; 0: the line misses the box
+    float block, pair;      // bounds on the length of a block and of half a block
+};
+constexpr int kColBlock = 4;
+struct alignas(64) ColumnBlock {
+    float l[kColBlock + 1];     // begin of each cell, relative to the entry; begin of the next block
+    float d[kColBlock];         // lengths: differences of l
+    unsigned off[kColBlock];    // byte offset of the cell in the z-fastest copy
+    unsigned pad[3];
+};
+struct ColumnLists {
+    ColumnHead *head;       // [views][np]
+    ColumnBlock *blocks;    // [views][np][stride / kColBlock]
+    int stride, views;
+};
+
 // Ray-driven Siddon projector (cone; the fan beam is the nz = n_xi = 1 case).
 // Box [0,bt] x [0,bs] x [0,bz] mm, voxel pitch (rt, rs, rz).
 struct RayParams {
@@ -29,6 +50,9 @@ struct RayParams {
                             // central ray runs mostly along t (neighbouring rays then differ in s)
     int parallel;           // parallel beam: ray (view, p) is the line through centre + p (cos, sin)
                             // along (-sin, cos); view[4b+2..3] unused
+    const float *volZ;      // optional [s][t][1 + nz + 1] copy of the volume with a slice of zeros at both
+                            // ends: the projection runs by detector columns (column_plan)
+    ColumnLists cols;
     const float *flat;      // 2-D image (one slice, one detector row at its height: fan, parallel beam):
                             // the image [nt*ns] followed by its transpose, at most 2^29 floats together
     int residual_norm;      // the SIRT residual pass stores r times the ray norm (the cone
@@ -200,6 +224,15 @@ hipError_t scan_counts(const long long *counts, long long *out, int n, void *tmp
 hipError_t launch_ray_fp_residual(const RayParams &g, const float *vol, const float *b, float *r,
                                   double *partials, int *nblocks, hipStream_t st);
 int ray_fp_blocks(const RayParams &g);
+// Whether the cone projection (residual: the SIRT residual pass) runs by
+// detector columns, and the sizes of its volume copy and list workspace;
+// column_bind points g at them.
+struct ColumnPlan {
+    int stride, views;
+    size_t vol_bytes, list_bytes;
+};
+bool column_plan(const RayParams &g, bool residual, ColumnPlan &L);
+void column_bind(RayParams &g, const ColumnPlan &L, float *volz, void *lists);
 
 // Tiling of the voxel-driven backprojection and its per-(tile, view) detector
 // footprint table (int4 per entry, nfoot entries), computed once per geometry.
@@ -376,6 +409,8 @@ hipError_t launch_diff_sums(const float *x, const float *ref, size_t n, double *
 hipError_t launch_fill(float *dst, float value, size_t n, hipStream_t st);
 // out [z][t][s] from in [z][s][t]; copy: null, or where in itself goes as well
 hipError_t launch_transpose_st(const float *in, float *out, float *copy, int nt, int ns, int nz, hipStream_t st);
+// out [s][t][1 + nz + 1] from in [z][s][t], zeros in the first and last slice
+hipError_t launch_z_fastest(const float *in, float *out, int nt, int ns, int nz, hipStream_t st);
 hipError_t launch_reciprocal_eps(float *v, size_t n, float eps, hipStream_t st);   // v <- 1/(v+eps)
 // Deterministic sum of n (a, b) pairs into out2[0..1].  Above kReduceDirect
 // pairs it runs in two stages and writes up to kReduceSlack stage pairs after

@@ -19,6 +19,9 @@
 // the intersection length in mm, as the reference's :311-356.
 #include "ctr_internal.h"
 
+#include <algorithm>
+#include <cstdlib>
+
 namespace ctr {
 namespace {
 
@@ -684,6 +687,415 @@ __global__ __launch_bounds__(64 * kFlatWaves) void k_ray_fp_residual_flat(const 
     }
 }
 
+// ---------------------------------------------------------------------------
+// Cone beam by detector columns.
+//
+// All rays of one detector column (one view, one p) share their path through
+// the (t, s) plane: seen from above they are one line.  k_ray_cells walks that
+// line once in FP64 and lists the voxel columns (cells) it crosses, with the
+// in-plane parameter at which each begins and its length, four cells to a
+// 64-byte block.  k_ray_columns then gives a wavefront 64 neighbouring rows of
+// the detector column and walks the list: a block is the same for the
+// wavefront and comes through the scalar cache in one load, and a lane only
+// keeps track of its slice.  The volume is read from a copy with z fastest,
+// [s][t][1 + nz + 1] with a slice of zeros at both ends, so the wavefront's
+// load of a cell is one run of neighbouring voxels, and a ray that leaves
+// through the top or the bottom reads zeros from there on.
+//
+// Slices change rarely (a cone angle of 12 degrees passes a plane every five
+// voxels), so a lane looks for its next z crossing once per block, or twice
+// where a ray of the wavefront is steep enough to cross two planes in a block:
+// each cell's length splits at the crossing, clamped into the cell, between the
+// old slice and the new one.  Steeper still, the cells are taken one by one,
+// each cut by as many crossings as there are.
+//
+// Crossing parameters and cell bounds are floats relative to the entry point,
+// with one rounding each, as in the slab walk, and lengths are differences of
+// them (lengths rounded one by one would sum up with a bias: 1.2e-6 instead of
+// 3e-8 on a volume of ones).  Per ray and voxel column the loop issues 6.5 VALU
+// instructions and two loads (the slab walk: 32 instructions and three loads
+// per slab of 1.4 voxel columns).
+// ---------------------------------------------------------------------------
+constexpr int kColWaves = 4;
+
+// One wavefront per detector column of view view0 + blockIdx.y: its list and
+// its head.  LDS: C.stride + 1 cell parameters, then C.stride offsets.
+__global__ __launch_bounds__(64) void k_ray_cells(RayParams g, ColumnLists C, int view0)
+{
+    extern __shared__ float cells[];
+    float *sl = cells;
+    unsigned *so = reinterpret_cast<unsigned *>(cells + C.stride + 1);
+    const int ip = blockIdx.x, v = blockIdx.y, ib = view0 + v, lane = threadIdx.x;
+    const size_t col = (size_t)v * g.np + ip;
+    const double sb = g.view[4 * ib + 0], cb = g.view[4 * ib + 1], st = g.view[4 * ib + 2], ss = g.view[4 * ib + 3];
+    const double P = g.p[ip];
+    double dx = P * cb + g.D * sb, dy = P * sb - g.D * cb;
+    const double inv_n = 1.0 / sqrt(dx * dx + dy * dy);
+    dx *= inv_n;
+    dy *= inv_n;
+    double lo = -__builtin_huge_val(), hi = __builtin_huge_val();
+    bool hit = clip_axis(st, dx, g.bt, lo, hi);
+    hit = clip_axis(ss, dy, g.bs, lo, hi) && hit && hi > lo;
+    if (!hit) {
+        if (lane == 0) C.head[col] = ColumnHead{};
+        return;
+    }
+    const AxisSetup at = setup_axis(st, dx, lo, hi, g.rt, g.nt, 1), as = setup_axis(ss, dy, lo, hi, g.rs, g.ns, 1);
+    // slabs of the axis with the shorter step; at most one crossing of the
+    // other axis in a slab, but for rounding, and any number is listed
+    const bool along_t = at.stride != 0 && (as.stride == 0 || at.step <= as.step);
+    const AxisSetup aD = along_t ? at : as, aA = along_t ? as : at;
+    const double len = hi - lo, inv_step = aA.n > 0 ? 1.0 / aA.step : 0.0;
+    const unsigned pitch = (unsigned)(g.nz + 2) * 4u;
+    auto crossings_before = [&](double lam) {
+        const double c = aA.n > 0 ? ceil((lam - aA.next0) * inv_step) : 0.0;
+        return (int)fmin(fmax(c, 0.0), (double)aA.n);
+    };
+    for (int k = lane; k <= aD.n; k += 64) {
+        const double l0 = k == 0 ? 0.0 : aD.next0 + (k - 1) * aD.step, l1 = aD.next0 + k * aD.step;
+        const int c0 = k == 0 ? 0 : crossings_before(l0), c1 = k == aD.n ? aA.n : crossings_before(l1);
+        double begin = l0;
+        for (int c = c0; c <= c1; ++c) {
+            const int iD = aD.i0 + aD.stride * k, iA = aA.i0 + aA.stride * c;
+            sl[k + c] = (float)begin;
+            so[k + c] = (unsigned)(along_t ? iA * g.nt + iD : iD * g.nt + iA) * pitch;
+            begin = aA.next0 + c * aA.step;
+        }
+    }
+    // the list ends in cells of length 0, up to an even number of blocks and one
+    // more that is read ahead
+    const int n = aD.n + aA.n + 1, padded = (n + 2 * kColBlock - 1) / (2 * kColBlock) * (2 * kColBlock);
+    __syncthreads();
+    if (lane <= padded + kColBlock - n) {
+        sl[n + lane] = (float)len;
+        if (lane < padded + kColBlock - n) so[n + lane] = so[n - 1];
+    }
+    __syncthreads();
+    float longest = 0.0f, pair = 0.0f;
+    unsigned *out = reinterpret_cast<unsigned *>(C.blocks + col * (C.stride / kColBlock));
+    for (int e = lane; e < (padded + kColBlock) * 4; e += 64) {   // 16 words a block: l[5], d[4], off[4]
+        const int q = e & 15, i = (e >> 4) * kColBlock;
+        unsigned w = 0;
+        if (q < 5) {
+            w = __builtin_bit_cast(unsigned, sl[i + q]);
+            if (q == 4) {
+                longest = fmaxf(longest, sl[i + 4] - sl[i]);
+                pair = fmaxf(pair, fmaxf(sl[i + 2] - sl[i], sl[i + 4] - sl[i + 2]));
+            }
+        } else if (q < 9) {
+            w = __builtin_bit_cast(unsigned, fmaxf(sl[i + q - 4] - sl[i + q - 5], 0.0f));
+        } else if (q < 13) {
+            w = so[i + q - 9];
+        }
+        out[e] = w;
+    }
+    for (int m = 32; m > 0; m >>= 1) {
+        longest = fmaxf(longest, __shfl_xor(longest, m, 64));
+        pair = fmaxf(pair, __shfl_xor(pair, m, 64));
+    }
+    if (lane == 0)
+        C.head[col] = ColumnHead{lo, len, 1.0 / sqrt(P * P + g.D * g.D), padded, longest * 1.0001f, pair * 1.0001f};
+}
+
+// x clamped into [0, hi]
+__device__ __forceinline__ int clamp_i(int x, int hi)
+{
+    int r;
+    asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(x), "v"(hi));
+    return r;
+}
+
+// v of the lane byte / 4 (mod 64)
+__device__ __forceinline__ float lane_value(int byte, float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(byte, __builtin_bit_cast(int, v)));
+}
+
+// v of lane i, for the whole wavefront
+__device__ __forceinline__ float lane_float(float v, int i)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i));
+}
+
+// State of a lane on its way through the cells of a list.
+struct ColumnLane {
+    float Z0, dZ;   // first z crossing and the step between them
+    int zb, sgn;    // first slice (bytes into a cell) and the step per crossing
+};
+
+// Sum over the blocks of a list, nb of them (even, and one more to read).
+// WINDOW: the cell's 64 slices around the wavefront's rows are loaded as one
+// run, a slice per lane, and handed to the rows by lane permutations; otherwise
+// each row reads its own two.  The window halves the loads, whose address and
+// tag work bounds the loop (7 cycles a load, 4 for 64 lanes at best): 3.0
+// against 3.7 ms for 256^3 / 90 views / 512^2, the rows of a wavefront 40
+// slices apart.  Where they fan out to more than 64 slices two windows would
+// do, which measured 47 ms against 41 for the plain loads at 512^3 / 240 views.
+template <bool WINDOW, int STEP>
+__device__ __forceinline__ float column_sum(__amdgpu_buffer_rsrc_t rs, const ColumnBlock *__restrict__ blk, int nb, int top,
+                                            const ColumnLane &L)
+{
+    // a block on its way: weights of the old and the new slice, loaded values
+    struct Part {
+        float w1[kColBlock], w2[kColBlock], v[kColBlock], u[kColBlock];
+        int io[kColBlock / STEP], in[kColBlock / STEP];
+    };
+    const int lane4 = (int)__lane_id() * 4;
+    float acc = 0.0f, pZ = L.Z0;
+    int za = L.zb, cz = 0;
+    auto load = [&](int z, unsigned cell) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, z, (int)cell, 0));
+    };
+    ColumnBlock next = blk[0];
+    auto issue = [&](Part &q, int i) {
+        const ColumnBlock c = next;
+        next = blk[i + 1];
+        constexpr int H = kColBlock / STEP;
+        float p[H];
+        int zo[H], zn[H];
+#pragma unroll
+        for (int k = 0; k < H; ++k) {
+            p[k] = pZ;
+            zo[k] = za;
+            cz += pZ < c.l[(k + 1) * STEP] ? 1 : 0;
+            pZ = fmaf((float)cz, L.dZ, L.Z0);
+            zn[k] = za = clamp_i(__mul24(cz, L.sgn) + L.zb, top);
+        }
+        if constexpr (!WINDOW) {
+#pragma unroll
+            for (int j = 0; j < kColBlock; ++j) {
+                q.v[j] = load(zo[j / STEP], c.off[j]);
+                q.u[j] = load(zn[j / STEP], c.off[j]);
+            }
+        } else {
+            // the wavefront's slices lie between those of its first and last
+            // row, one more to either side for each step back and one for ties
+            const int e0 = __builtin_amdgcn_readlane(za, 0), e1 = __builtin_amdgcn_readlane(za, 63);
+            const int base = max(min(e0, e1) - 4 * (H + 1), 0);
+#pragma unroll
+            for (int k = 0; k < H; ++k) {
+                q.io[k] = zo[k] - base;
+                q.in[k] = zn[k] - base;
+            }
+#pragma unroll
+            for (int j = 0; j < kColBlock; ++j) q.v[j] = load(lane4, c.off[j] + base);
+        }
+#pragma unroll
+        for (int j = 0; j < kColBlock; ++j) {
+            q.w1[j] = __builtin_amdgcn_fmed3f(p[j / STEP] - c.l[j], 0.0f, c.d[j]);
+            q.w2[j] = c.d[j] - q.w1[j];
+        }
+    };
+    auto sum = [&](const Part &q) {
+        float v1[kColBlock], v2[kColBlock];
+#pragma unroll
+        for (int j = 0; j < kColBlock; ++j) {
+            v1[j] = WINDOW ? lane_value(q.io[j / STEP], q.v[j]) : q.v[j];
+            v2[j] = WINDOW ? lane_value(q.in[j / STEP], q.v[j]) : q.u[j];
+        }
+#pragma unroll
+        for (int j = 0; j < kColBlock; ++j) {
+            acc = fmaf(q.w1[j], v1[j], acc);
+            acc = fmaf(q.w2[j], v2[j], acc);
+        }
+    };
+    Part A, B;
+    issue(A, 0);
+    for (int i = 0; i < nb; i += 2) {
+        issue(B, i + 1);
+        sum(A);
+        issue(A, min(i + 2, nb - 1));
+        sum(B);
+    }
+    return acc;
+}
+
+// Line integrals of the 64 rows of a wavefront through the cells of detector
+// column `col`; chord is the row's length in the volume box.
+__device__ __forceinline__ float trace_column(const RayParams &g, const ColumnHead *__restrict__ heads,
+                                              const ColumnBlock *__restrict__ blocks, size_t stride, size_t col, int ip,
+                                              int ix, bool valid, float &chord)
+{
+    const ColumnHead h = heads[col];
+    chord = 0.0f;
+    if (h.n == 0) return 0.0f;
+    const double slope = g.xi[valid ? ix : g.nx - 1] * h.inv_rho;   // z per in-plane length
+    // first slice, next plane and the step between planes
+    const double inv_rz = 1.0 / g.rz, zin = (g.sz + h.lo * slope) * inv_rz;
+    const double k0 = slope < 0.0 ? ceil(zin) - 1.0 : floor(zin);
+    double z0 = __builtin_huge_val(), dz = 0.0, out = __builtin_huge_val();
+    if (slope != 0.0) {
+        const double inv_s = 1.0 / slope;
+        z0 = ((slope > 0.0 ? k0 + 1.0 : k0) * g.rz - g.sz) * inv_s - h.lo;
+        dz = g.rz * fabs(inv_s);
+        out = (slope > 0.0 ? g.bz - g.sz : -g.sz) * inv_s - h.lo;
+    }
+    const double norm = sqrt(fma(slope, slope, 1.0)), length = fmin(h.len, out);
+    const bool hit = length > 0.0;
+    chord = hit ? (float)(length * norm) : 0.0f;
+    const float Z0 = (float)z0, dZ = (float)dz;
+    const int top = 4 * (g.nz + 1);   // slices 0 and nz + 1 of the copy are zeros
+    const int zb = (int)fmin(fmax(4.0 * (k0 + 1.0), 0.0), (double)top), sgn = slope > 0.0 ? 4 : -4;
+
+    const size_t vbytes = (size_t)g.nt * g.ns * (g.nz + 2) * sizeof(float);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)g.volZ, 0, (int)(vbytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (unsigned)vbytes), kBufDword3);
+    const ColumnBlock *__restrict__ blk = blocks + col * stride;
+    float acc = 0.0f;
+    const int nb = h.n / kColBlock;
+    if (__ballot(dZ != 0.0f && dZ < h.pair) == 0) {
+        // widest run of slices (bytes): the rows fan out from the source until
+        // the line leaves the box or the outermost row its top or bottom, where
+        // its slice stays
+        const float s0 = lane_float((float)slope, 0), s1 = lane_float((float)slope, 63);
+        const float reach = (float)(h.lo + h.len), outer = fmaxf(fabsf(s0), fabsf(s1)) * reach, half = 0.5f * (float)g.bz;
+        const float wide = 4.0f * (fabsf(s1 - s0) * reach * (outer > half ? half / outer : 1.0f) * (float)inv_rz) + 36.0f;
+        const bool narrow = wide <= 4.0f * 63.0f, gentle = __ballot(dZ != 0.0f && dZ < h.block) == 0;
+        const ColumnLane lane{Z0, dZ, zb, sgn};
+        if (gentle)
+            acc = narrow ? column_sum<true, kColBlock>(rs, blk, nb, top, lane)
+                         : column_sum<false, kColBlock>(rs, blk, nb, top, lane);
+        else
+            acc = narrow ? column_sum<true, kColBlock / 2>(rs, blk, nb, top, lane)
+                         : column_sum<false, kColBlock / 2>(rs, blk, nb, top, lane);
+    } else {
+        float pZ = Z0;
+        int za = zb, cz = 0;
+        auto load = [&](int z, unsigned cell) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, z, (int)cell, 0));
+        };
+        for (int i = 0; i < h.n; ++i) {
+            const ColumnBlock &c = blk[i / kColBlock];
+            const int j = i % kColBlock;
+            const float l1 = c.l[j + 1];
+            const unsigned cell = c.off[j];
+            float l = c.l[j];
+            while (pZ < l1) {
+                if (pZ > l) {
+                    acc = fmaf(pZ - l, load(za, cell), acc);
+                    l = pZ;
+                }
+                ++cz;
+                pZ = fmaf((float)cz, dZ, Z0);
+                za = clamp_i(__mul24(cz, sgn) + zb, top);
+            }
+            if (l1 > l) acc = fmaf(l1 - l, load(za, cell), acc);
+        }
+    }
+    return hit ? acc * (float)norm : 0.0f;
+}
+
+// Workgroup -> (64 rows, view, four detector columns).  Consecutive workgroups
+// go to the eight XCDs in turn; an XCD is given tiles of kColTileP x kColTileV
+// (columns, views), 256 workgroups, which is what its 32 CUs hold at a time:
+// neighbouring columns of neighbouring views cross the same cells, so the
+// wavefronts in flight share them in the XCD's L2.  Tiles run over the columns,
+// then the views, rows slowest: one band of slices at a time, which stays in the
+// Infinity Cache.
+constexpr int kColTileP = 16, kColTileV = 16;
+
+struct ColumnTile {
+    int p0, v, row0;   // p0 or v past the end: an empty place of a partial tile
+};
+__host__ __device__ __forceinline__ int column_tiles_p(const RayParams &g)
+{
+    return (g.np + kColWaves * kColTileP - 1) / (kColWaves * kColTileP);
+}
+__host__ __device__ __forceinline__ int column_tiles_v(int views) { return (views + kColTileV - 1) / kColTileV; }
+__device__ __forceinline__ ColumnTile column_tile(const RayParams &g, int views)
+{
+    constexpr int kTile = kColTileP * kColTileV;
+    const int place = blockIdx.x >> 3, tile = place / kTile * 8 + (int)(blockIdx.x & 7), in = place % kTile;
+    const int tp = column_tiles_p(g), tv = column_tiles_v(views);
+    const int ip = tile % tp, rest = tile / tp;
+    return ColumnTile{(ip * kColTileP + in % kColTileP) * kColWaves, rest % tv * kColTileV + in / kColTileP,
+                      rest / tv * 64};
+}
+
+// kResidual: the SIRT residual pass (fp_residual_block) instead of the projection.
+template <bool kResidual>
+__global__ __launch_bounds__(64 * kColWaves, 8) void k_ray_columns(const float *__restrict__ b, float *__restrict__ out,
+                                                                double *__restrict__ partials,
+                                                                const ColumnHead *__restrict__ heads,
+                                                                const ColumnBlock *__restrict__ blocks, RayParams g,
+                                                                int stride, int view0, int views)
+{
+    __shared__ float sums[kColWaves][65], chords[kColWaves][65];
+    __shared__ double red[2][kColWaves];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const ColumnTile B = column_tile(g, views);
+    const int ip = B.p0 + wave;
+    float chord = 0.0f, acc = 0.0f;
+    const bool there = B.p0 < g.np && B.v < views && B.row0 < g.nx;
+    if (there && ip < g.np) {
+        const int ix = B.row0 + lane;
+        acc = trace_column(g, heads, blocks, stride, (size_t)B.v * g.np + ip, ip, ix, ix < g.nx, chord);
+    }
+    // the block's 64 x 4 results, four neighbouring columns of a row per four threads
+    sums[wave][lane] = acc;
+    if (kResidual) chords[wave][lane] = chord;
+    __syncthreads();
+    const int c = threadIdx.x % kColWaves, r = threadIdx.x / kColWaves;
+    const int oc = B.p0 + c, orow = B.row0 + r;
+    double e2 = 0.0, e1 = 0.0;
+    if (there && oc < g.np && orow < g.nx) {
+        const size_t ray = ((size_t)(view0 + B.v) * g.nx + orow) * g.np + oc;
+        if (kResidual) {
+            const float e = b[ray] - sums[c][r];
+            const float rr = e / (chords[c][r] + 1e-9f);
+            out[ray] = g.residual_norm ? rr * ray_norm((float)g.p[oc], (float)g.xi[orow], (float)g.D) : rr;
+            e2 = (double)e * (double)e;
+            e1 = fabs((double)e);
+        } else {
+            out[ray] = sums[c][r];
+        }
+    }
+    if (kResidual) {
+        e2 = wave_sum(e2);
+        e1 = wave_sum(e1);
+        if (lane == 0) {
+            red[0][wave] = e2;
+            red[1][wave] = e1;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double s2 = 0.0, s1 = 0.0;
+            for (int w = 0; w < kColWaves; ++w) {
+                s2 += red[0][w];
+                s1 += red[1][w];
+            }
+            partials[2 * (size_t)blockIdx.x] = s2;
+            partials[2 * (size_t)blockIdx.x + 1] = s1;
+        }
+    }
+}
+
+int column_blocks(const RayParams &g, int views)
+{
+    const long tiles = (long)column_tiles_p(g) * column_tiles_v(views) * ((g.nx + 63) / 64);
+    return (int)((tiles + 7) / 8 * 8 * kColTileP * kColTileV);
+}
+
+// Lists of C.views views at a time, then their rays.
+template <bool kResidual>
+hipError_t launch_columns(const RayParams &g, const float *b, float *out, double *partials, int *nblocks, hipStream_t st)
+{
+    const ColumnLists &C = g.cols;
+    int blocks = 0;
+    for (int v0 = 0; v0 < g.nb; v0 += C.views) {
+        const int views = g.nb - v0 < C.views ? g.nb - v0 : C.views, n = column_blocks(g, views);
+        hipLaunchKernelGGL(k_ray_cells, dim3(g.np, views), dim3(64), (2 * C.stride + 1) * sizeof(float), st, g, C, v0);
+        hipLaunchKernelGGL(k_ray_columns<kResidual>, dim3((unsigned)n), dim3(64 * kColWaves), 0, st, b, out,
+                           partials ? partials + 2 * (size_t)blocks : nullptr, C.head, C.blocks, g, C.stride / kColBlock, v0,
+                           views);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        blocks += n;
+    }
+    if (nblocks) *nblocks = blocks;
+    return hipSuccess;
+}
+
 unsigned flat_blocks(const RayParams &g)
 {
     const long items = (long)((g.np + 63) / 64) * g.nb;
@@ -694,11 +1106,59 @@ dim3 fp_grid(const RayParams &g) { return dim3((g.np + kBX - 1) / kBX, (g.nx + k
 
 }  // namespace
 
+// lists of one pass (16 bytes a cell) stay in the Infinity Cache beside a band of slices
+constexpr size_t kColListBytes = (size_t)256 << 20;
+
+// Where the columns are faster than the slab walk (CTR_FP_COLUMNS = 0 / 1
+// overrides).  A wavefront always pays for 64 rows, so they need about 0.7 of
+// its lanes filled, and the three launches need enough wavefronts.  Slab walk /
+// columns in us (nz, views x columns x rows):
+//   256^3, 90 x 512 x 512     4460 / 2858      56 slices, 360 x 512 x 80   2528 / 3184
+//   128^3, 180 x 192 x 192     608 /  400      50 slices, 180 x 192 x 72    226 /  267
+//    70 slices, 120 x 300 x 100 509 / 397      28 slices, 180 x 192 x 40    125 /  170
+//    64^3, 90 x 96 x 96 (17k wavefronts) 81 / 76,   60 x 52 x 44, 45 x 96 x 80 (9k) 42 / 53
+// The residual pass of SIRT has a second line: its history of residual norms
+// averages the rounding of all rays, which for fewer than 2^22 of them differs
+// between the two kernels by more than 1e-9 of the norm (4e-10 at 3e5 rays a
+// view, 2e-9 at 20000).
+static bool column_use(const RayParams &g, bool residual)
+{
+    if (const char *e = std::getenv("CTR_FP_COLUMNS")) return std::atoi(e) != 0;
+    const size_t chunks = (g.nx + 63) / 64, waves = (size_t)g.nb * g.np * chunks;
+    if (residual && (size_t)g.nb * g.np * g.nx < ((size_t)1 << 22)) return false;
+    return 10 * (size_t)g.nx >= 7 * 64 * chunks && waves >= 12000;
+}
+
+bool column_plan(const RayParams &g, bool residual, ColumnPlan &L)
+{
+    // 32-bit offsets into the z-fastest copy, one workgroup row per view in the list kernel
+    if (g.parallel || (size_t)g.nt * g.ns * (g.nz + 2) > ((size_t)1 << 30)) return false;
+    if (!column_use(g, residual)) return false;
+    L.stride = (g.nt + g.ns + 1 + 2 * kColBlock - 1) / (2 * kColBlock) * (2 * kColBlock) + kColBlock;
+    if (L.stride > 4096) return false;   // the list kernel's LDS
+    const size_t per_view = (size_t)g.np * (L.stride / kColBlock * sizeof(ColumnBlock) + sizeof(ColumnHead));
+    const size_t views = std::max<size_t>(1, kColListBytes / per_view / kColTileV) * kColTileV;
+    L.views = (int)std::min<size_t>({views, (size_t)g.nb, 65535});
+    L.list_bytes = (size_t)L.views * per_view + 256;
+    L.vol_bytes = (size_t)g.nt * g.ns * (g.nz + 2) * sizeof(float);
+    return true;
+}
+
+void column_bind(RayParams &g, const ColumnPlan &L, float *volz, void *lists)
+{
+    g.volZ = volz;
+    g.cols.blocks = (ColumnBlock *)lists;   // 64-byte aligned, before the heads
+    g.cols.head = (ColumnHead *)(g.cols.blocks + (size_t)L.views * g.np * (L.stride / kColBlock));
+    g.cols.stride = L.stride;
+    g.cols.views = L.views;
+}
+
 int ray_fp_blocks(const RayParams &g)
 {
     if (g.flat) return (int)flat_blocks(g);
+    // of either kernel: a caller sizes the partial sums before the plan is bound
     const dim3 grid = fp_grid(g);
-    return (int)(grid.x * grid.y * grid.z);
+    return std::max((int)(grid.x * grid.y * grid.z), kColTileV * column_blocks(g, g.nb));
 }
 
 hipError_t launch_sysmat_count(const RayParams &g, long long *counts, hipStream_t st)
@@ -717,6 +1177,7 @@ hipError_t launch_sysmat_fill(const RayParams &g, const long long *row_ptr, int 
 
 hipError_t launch_ray_fp(const RayParams &g, const float *vol, float *proj, hipStream_t st)
 {
+    if (g.volZ) return launch_columns<false>(g, nullptr, proj, nullptr, nullptr, st);
     if (g.flat) {
         hipLaunchKernelGGL(k_ray_fp_flat, dim3(flat_blocks(g)), dim3(64, kFlatWaves), 0, st, proj, g);
         return hipGetLastError();
@@ -728,6 +1189,7 @@ hipError_t launch_ray_fp(const RayParams &g, const float *vol, float *proj, hipS
 hipError_t launch_ray_fp_residual(const RayParams &g, const float *vol, const float *b, float *r, double *partials,
                                   int *nblocks, hipStream_t st)
 {
+    if (g.volZ) return launch_columns<true>(g, b, r, partials, nblocks, st);
     if (g.flat) {
         *nblocks = (int)flat_blocks(g);
         hipLaunchKernelGGL(k_ray_fp_residual_flat, dim3(flat_blocks(g)), dim3(64, kFlatWaves), 0, st, b, r, partials, g);
@@ -741,6 +1203,12 @@ hipError_t launch_ray_fp_residual(const RayParams &g, const float *vol, const fl
 
 int fp_job_blocks(const RayParams &g, int *gx, int *gy)
 {
+    if (g.volZ) {   // not in the job table: its own launches' partial sums
+        *gx = *gy = 0;
+        int blocks = 0;
+        for (int v0 = 0; v0 < g.nb; v0 += g.cols.views) blocks += column_blocks(g, std::min(g.nb - v0, g.cols.views));
+        return blocks;
+    }
     const dim3 grid = fp_grid(g);
     *gx = (int)grid.x;
     *gy = (int)grid.y;

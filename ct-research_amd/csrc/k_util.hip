@@ -136,6 +136,30 @@ __global__ __launch_bounds__(256) void k_transpose_st(const float *__restrict__ 
     }
 }
 
+// out[s][t][1 + z] = in[z][s][t] for one s per blockIdx.z: 32 x 32 tiles of
+// (t, z) through LDS; the blocks of the first and last slices write the zeros.
+__global__ __launch_bounds__(256) void k_z_fastest(const float *__restrict__ in, float *__restrict__ out, int nt, int ns,
+                                                   int nz, int s0)
+{
+    __shared__ float tile[32][33];
+    const int t0 = blockIdx.x * 32, z0 = blockIdx.y * 32, s = s0 + blockIdx.z;
+    const int x = threadIdx.x & 31, y = threadIdx.x >> 5;   // 32 x 8
+    const size_t plane = (size_t)nt * ns, pitch = (size_t)nz + 2;
+    for (int k = y; k < 32; k += 8) {
+        const int t = t0 + x, z = z0 + k;
+        if (t < nt && z < nz) tile[k][x] = in[z * plane + (size_t)s * nt + t];
+    }
+    __syncthreads();
+    for (int k = y; k < 32; k += 8) {
+        const int t = t0 + k, z = z0 + x;
+        if (t >= nt) continue;
+        float *col = out + ((size_t)s * nt + t) * pitch;
+        if (z < nz) col[1 + z] = tile[x][k];
+        if (z == 0) col[0] = 0.0f;
+        if (z == nz - 1) col[1 + nz] = 0.0f;
+    }
+}
+
 // Per-block (sum x^2, sum x).
 __global__ __launch_bounds__(256) void k_sum_sq_sum(const float *x, size_t n, double *partials)
 {
@@ -363,6 +387,16 @@ hipError_t launch_reduce_jobs(const ReduceJob *jobs, int njobs, const int *iter,
 hipError_t launch_transpose_st(const float *in, float *out, float *copy, int nt, int ns, int nz, hipStream_t st)
 {
     hipLaunchKernelGGL(k_transpose_st, dim3((nt + 31) / 32, (ns + 31) / 32, nz), dim3(256), 0, st, in, out, copy, nt, ns);
+    return hipGetLastError();
+}
+
+hipError_t launch_z_fastest(const float *in, float *out, int nt, int ns, int nz, hipStream_t st)
+{
+    // one launch per 65535 rows s (the grid's third dimension)
+    for (int s0 = 0; s0 < ns; s0 += 65535) {
+        const int n = ns - s0 < 65535 ? ns - s0 : 65535;
+        hipLaunchKernelGGL(k_z_fastest, dim3((nt + 31) / 32, (nz + 31) / 32, n), dim3(256), 0, st, in, out, nt, ns, nz, s0);
+    }
     return hipGetLastError();
 }
 

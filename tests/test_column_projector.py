@@ -1,0 +1,85 @@
+"""The projector by detector columns (forced with CTR_FP_COLUMNS=1) at the
+sizes where its paths end: row counts around a wavefront, single slices, lists
+shorter than a block, rays that leave through the top and the bottom, cones so
+steep that a block of cells holds several z crossings, rows closer and wider
+than the 64-slice window, descending detectors, lines that miss the box.
+
+Tolerance: the bound of the cone projector's tests (float crossing parameters,
+one rounding each): rel-L2 2e-6, largest error 2e-5 of the largest integral."""
+import numpy as np
+import pytest
+
+from conftest import errs, report
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    # name: nt, ns, nz, size, D, views, columns, column pitch, rows, row pitch
+    "row": (20, 18, 12, (20.0, 18.0, 12.0), 60.0, 9, 33, 0.9, 1, 0.7),
+    "rows63": (24, 20, 30, (24.0, 20.0, 30.0), 70.0, 7, 37, 0.8, 63, 0.5),
+    "rows65": (24, 20, 30, (24.0, 20.0, 30.0), 70.0, 18, 70, 0.5, 65, 0.5),
+    "rows130": (33, 40, 64, (33.0, 40.0, 64.0), 110.0, 17, 21, 1.7, 130, 0.55),
+    "one_slice": (16, 16, 1, (16.0, 16.0, 2.0), 50.0, 5, 20, 0.9, 66, 0.05),
+    "one_voxel": (1, 1, 1, (1.0, 1.0, 1.0), 5.0, 8, 9, 0.3, 12, 0.2),
+    "out_of_top": (40, 40, 8, (40.0, 40.0, 4.0), 90.0, 12, 40, 1.2, 64, 0.4),
+    "steep": (30, 30, 30, (30.0, 30.0, 30.0), 40.0, 11, 40, 1.0, 64, 1.0),
+    "very_steep": (24, 24, 96, (24.0, 24.0, 24.0), 30.0, 11, 30, 1.0, 64, 1.2),
+    "wide_rows": (24, 24, 200, (24.0, 24.0, 24.0), 300.0, 9, 30, 1.0, 80, 0.4),
+    "misses": (16, 12, 10, (16.0, 12.0, 10.0), 60.0, 6, 80, 1.0, 20, 1.0),
+    "descending": (20, 24, 16, (20.0, 24.0, 16.0), 70.0, 13, 40, -0.9, 40, -0.6),
+    "thin": (200, 3, 20, (20.0, 6.0, 20.0), 50.0, 8, 50, 0.5, 30, 0.8),
+}
+
+
+def _geom(case, lib):
+    nt, ns, nz, size, D, nb, np_, pp, nx, px = CASES[case]
+    beta = (2 * np.pi / nb * np.arange(1, nb + 1)).astype(np.float32)
+    p = (pp * (np.arange(np_) - (np_ - 1) / 2) + 0.03).astype(np.float32)
+    xi = (px * (np.arange(nx) - (nx - 1) / 2) + 0.02).astype(np.float32)
+    return lib(nt, ns, nz, size, D, beta, p, xi)
+
+
+@pytest.fixture
+def columns(monkeypatch):
+    monkeypatch.setenv("CTR_FP_COLUMNS", "1")
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_column_projector(ctx, oracle, columns, case):
+    import ctr
+    g, og = _geom(case, ctr.ConeGeom), _geom(case, oracle.Cone)
+    vol = np.random.default_rng(len(case)).random(g.nvox).astype(np.float32)
+    print(f"[case] columns {case} {g.vol_shape} {g.proj_shape}", flush=True)
+    e, m = errs(ctx.cone_fp(g, vol), oracle.cone_fp_exact(og, vol))
+    report(f"columns[{case}]", rel_l2=e, max_rel=m)
+    assert e < 2e-6 and m < 2e-5
+
+
+def test_column_projector_of_ones(ctx, oracle, columns):
+    """Lengths telescope: the projection of ones is the chord to the rounding of its ends."""
+    import ctr
+    g, og = _geom("rows130", ctr.ConeGeom), _geom("rows130", oracle.Cone)
+    e, m = errs(ctx.cone_fp(g, np.ones(g.nvox, np.float32)), oracle.cone_rowsum(og))
+    assert e < 2e-7 and m < 1e-6
+
+
+@pytest.mark.parametrize("streams", ["0", "2"])
+def test_column_residual(ctx, monkeypatch, streams):
+    """SIRT on the columns' residual pass: the slab walk's iterates to the
+    rounding of the ray sums, and the batched forms' bits."""
+    import ctr
+    g = _geom("rows130", ctr.ConeGeom)
+    vol = np.random.default_rng(4).random(g.nvox).astype(np.float32)
+    monkeypatch.setenv("CTR_FP_COLUMNS", "0")
+    b = ctx.cone_fp(g, vol)
+    x0, r0, s0 = ctx.sirt3d(g, b, 4)
+    monkeypatch.setenv("CTR_FP_COLUMNS", "1")
+    monkeypatch.setenv("CTR_BATCH_STREAMS", streams)
+    x1, r1, s1 = ctx.sirt3d(g, b, 4)
+    e, m = errs(x1, x0)
+    report("column residual", rel_l2=e, max_rel=m, dres=float(np.abs(r1 - r0).max()))
+    # two float sums of about 100 segments per ray, four iterations
+    assert e < 5e-6 and m < 5e-5 and np.abs(r1 - r0).max() < 1e-6
+    xs, rs = ctx.sirt3d_batched([(g, b), (g, b)], 4)
+    for x, r in zip(xs, rs):
+        assert np.array_equal(x, x1) and np.abs(r - r1).max() < 1e-12
