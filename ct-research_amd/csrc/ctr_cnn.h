@@ -21,7 +21,7 @@ enum CnnEpi {
 // channels-last), 32 output channels; w in the packed forward layout.
 hipError_t launch_conv3d(int cin_pad, int epi, const __bf16 *in, const __bf16 *w, const float *bias,
                          const __bf16 *mask, void *out, const CnnShape &S, hipStream_t st);
-// weight/bias gradient partials [nblk][co*ci*27 + co]; (ci, co) in {(16,32), (32,32), (32,16)}
+// weight/bias gradient partials [nblk][27*co*ci + co] (nblk = wgrad_blocks); (ci, co) in {(16,32), (32,32), (32,16)}
 int wgrad_blocks(const CnnShape &S);
 hipError_t launch_conv3d_wgrad(int ci, int co, const __bf16 *act, const __bf16 *delta, float *partial, int nblk,
                                const CnnShape &S, hipStream_t st);

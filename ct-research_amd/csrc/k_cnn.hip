@@ -17,8 +17,9 @@
 //
 // The backward pass w.r.t. the input is the same convolution with the taps
 // flipped and the channel roles swapped; its epilogue applies the ReLU
-// derivative of the layer below.  The weight gradient is a VALU reduction
-// over LDS-staged tiles (per-block partial sums, reduced deterministically).
+// derivative of the layer below.  The weight gradient is a product over the
+// voxels of LDS-staged, transposed tiles (per-block partial sums, reduced
+// deterministically).
 #include "ctr_cnn.h"
 
 namespace ctr {
@@ -745,108 +746,218 @@ __global__ __launch_bounds__(256) void k_conv3d_out1(const __bf16 *__restrict__ 
 
 // Weight and bias gradient of one layer over a volume:
 //   dW[co][ci][t] += sum_v delta[v][co] * act[v + off(t)][ci],  db[co] += sum_v delta[v][co]
-// Tiles of 32 x 8 voxels of one slice; the activations with their halo
-// (34 x 10 x 3) and the deltas are staged in LDS.  Thread (co, ci block of
-// 4) accumulates 4 x 27 weights over every tile it visits; each block
-// writes its partial sums, reduced afterwards by k_reduce_grad.
-template <int CI, int CO>
-__global__ __launch_bounds__(256) void k_conv3d_wgrad(const __bf16 *__restrict__ act, const __bf16 *__restrict__ delta,
-                                                      float *__restrict__ partial, CnnShape S)
-{
-    constexpr int HX = 34, HY = 10, HZ = 3, HV = HX * HY * HZ;
-    constexpr int CB = CI / 4;                       // ci blocks
-    constexpr int NT = CO * CB;                      // active threads
-    static_assert(NT <= 256, "too many weight blocks");
-    __shared__ __bf16 sa[HV * CI];
-    __shared__ __bf16 sd[256 * CO];
-    const int tid = threadIdx.x;
-    const int co = tid % CO, cb = tid / CO;
-    float acc[4][kTaps], accb = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int t = 0; t < kTaps; ++t) acc[c][t] = 0.0f;
+// a product over the voxels, on v_mfma_f32_16x16x32_bf16: M = 16 output
+// channels, N = 16 input channels, K = the 32 voxels of a tile row.  Both
+// operands want consecutive voxels of one channel per lane, so the tiles of
+// 32 x 4 voxels are transposed on their way into LDS ([row][channel][x], two
+// neighbouring voxels packed per word; a pitch of 40 puts the 16 channels of a
+// fragment on distinct banks).  The nine waves of a block take one (dz, dy)
+// each and its three dx taps: dx = 0 and 2 are the fragment's own words and
+// the words one further, dx = 1 is shifted by half a word.  A block walks its
+// tile along z, so that a slice of activations is staged once for the three
+// slices that use it, with the next slice's loads in flight during the products.
+// Each block writes its partial sums ([tap][co][ci], then [co]), reduced
+// afterwards by k_reduce_grad.
+//
+// 64^3 voxels, 32 -> 32 channels: 461 us with FP32 FMAs (a thread per output
+// channel and four input channels; 14.5 GFLOP at 31 TFLOP/s), bound by LDS and
+// VALU issue with the matrix cores idle; 30 us here, bound by staging and its
+// barriers.
+constexpr int kWgX = 32, kWgY = 4, kWgPitch = 40, kWgThreads = 9 * 64, kWgMaxBlocks = 256;
 
-    const int tiles_x = (S.nx + 31) / 32, tiles_y = (S.ny + 7) / 8;
-    const int ntiles = tiles_x * tiles_y * S.nz;
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int tx = tile % tiles_x, rest = tile / tiles_x;
-        const int ty = rest % tiles_y, z = rest / tiles_y;
-        const int x0 = tx * 32, y0 = ty * 8;
+struct WgradPlan {
+    int zrun, items, blocks;   // slices per item, (tile, run) items, blocks
+};
+WgradPlan wgrad_plan(const CnnShape &S)
+{
+    const long tiles = (long)((S.nx + kWgX - 1) / kWgX) * ((S.ny + kWgY - 1) / kWgY);
+    const long want = (tiles * S.nz + kWgMaxBlocks - 1) / kWgMaxBlocks;
+    WgradPlan p;
+    p.zrun = (int)(want < 1 ? 1 : (want > 16 ? 16 : want));
+    p.items = (int)(tiles * ((S.nz + p.zrun - 1) / p.zrun));
+    p.blocks = p.items < kWgMaxBlocks ? p.items : kWgMaxBlocks;
+    return p;
+}
+
+template <int CI, int CO>
+__global__ __launch_bounds__(kWgThreads) void k_conv3d_wgrad(const __bf16 *__restrict__ act,
+                                                             const __bf16 *__restrict__ delta,
+                                                             float *__restrict__ partial, CnnShape S, int zrun, int items)
+{
+    constexpr int HY = kWgY + 2, MB = CO / 16, NB = CI / 16;
+    constexpr int NPA = (kWgX + 2) / 2 * HY * (CI / 8), NPD = kWgX / 2 * kWgY * (CO / 8);   // voxel pairs x 8 channels
+    constexpr int ROUNDS = (NPA + NPD + kWgThreads - 1) / kWgThreads;
+    __shared__ __align__(16) __bf16 sa[3][HY][CI][kWgPitch];
+    __shared__ __align__(16) __bf16 sd[kWgY][CO][kWgPitch];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int dz = wave / 3, dy = wave % 3, m = lane & 15, kg = lane >> 4;
+    f32x4 acc[3][MB][NB];
+    float bias[MB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+        bias[i] = 0.0f;
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[d][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const int tiles_x = (S.nx + kWgX - 1) / kWgX, tiles_y = (S.ny + kWgY - 1) / kWgY, tiles = tiles_x * tiles_y;
+    for (int item = blockIdx.x; item < items; item += gridDim.x) {
+        const int tile = item % tiles, z0 = item / tiles * zrun, z1 = min(z0 + zrun, S.nz);
+        const int x0 = tile % tiles_x * kWgX, y0 = tile / tiles_x * kWgY;
+        // this thread's voxel pairs of slice zs of the activations (zero
+        // outside the volume) and of slice zd of the deltas
+        uint4 pair[ROUNDS][2];
+        auto fetch = [&](int zs, int zd) {
+#pragma unroll
+            for (int r = 0; r < ROUNDS; ++r) {
+                int e = tid + r * kWgThreads;
+                const bool is_act = e < NPA;
+                const __bf16 *src = is_act ? act : delta;
+                const int ch = is_act ? CI : CO;
+                int x, y, z, c;
+                if (is_act) {
+                    c = e % (CI / 8);
+                    x = x0 - 1 + 2 * (e / (CI / 8) % (kWgX / 2 + 1));
+                    y = y0 - 1 + e / (CI / 8) / (kWgX / 2 + 1);
+                    z = zs;
+                } else {
+                    e -= NPA;
+                    c = e % (CO / 8);
+                    x = x0 + 2 * (e / (CO / 8) % (kWgX / 2));
+                    y = y0 + e / (CO / 8) / (kWgX / 2);
+                    z = e < NPD ? zd : -1;
+                }
+                const bool row = y >= 0 && y < S.ny && z >= 0 && z < S.nz;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    uint4 v = {0, 0, 0, 0};
+                    if (row && x + k >= 0 && x + k < S.nx)
+                        v = *reinterpret_cast<const uint4 *>(src + (((size_t)z * S.ny + y) * S.nx + x + k) * ch + c * 8);
+                    pair[r][k] = v;
+                }
+            }
+        };
+        auto store = [&](int slot, bool deltas) {
+#pragma unroll
+            for (int r = 0; r < ROUNDS; ++r) {
+                int e = tid + r * kWgThreads;
+                __bf16 *dst;
+                if (e < NPA) {
+                    const int c = e % (CI / 8), px = e / (CI / 8) % (kWgX / 2 + 1), y = e / (CI / 8) / (kWgX / 2 + 1);
+                    dst = &sa[slot][y][c * 8][2 * px];
+                } else {
+                    e -= NPA;
+                    if (e >= NPD || !deltas) continue;
+                    const int c = e % (CO / 8), px = e / (CO / 8) % (kWgX / 2), y = e / (CO / 8) / (kWgX / 2);
+                    dst = &sd[y][c * 8][2 * px];
+                }
+                const uint4 p0 = pair[r][0], p1 = pair[r][1];
+                const unsigned w0[4] = {p0.x, p0.y, p0.z, p0.w}, w1[4] = {p1.x, p1.y, p1.z, p1.w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {   // both voxels' low halves, then their high halves
+                    *reinterpret_cast<unsigned *>(dst + 2 * q * kWgPitch) =
+                        __builtin_amdgcn_perm(w1[q], w0[q], 0x05040100u);
+                    *reinterpret_cast<unsigned *>(dst + (2 * q + 1) * kWgPitch) =
+                        __builtin_amdgcn_perm(w1[q], w0[q], 0x07060302u);
+                }
+            }
+        };
+        // slice z of the activations lives in slot (z + 1) mod 3
         __syncthreads();
-        // stage activations with halo (zero outside the volume), 8 channels per step
-        for (int e = tid; e < HV * (CI / 8); e += 256) {
-            const int hv = e / (CI / 8), c8 = e % (CI / 8);
-            const int hx = hv % HX, hy = (hv / HX) % HY, hz = hv / (HX * HY);
-            const int xx = x0 - 1 + hx, yy = y0 - 1 + hy, zz = z - 1 + hz;
-            bf16x8 v;
+        fetch(z0 - 1, -1);
+        store(z0 % 3, false);
+        fetch(z0, -1);
+        store((z0 + 1) % 3, false);
+        fetch(z0 + 1, z0);
+        for (int z = z0; z < z1; ++z) {
+            __syncthreads();   // the previous slice's products are done
+            store((z + 2) % 3, true);
+            __syncthreads();
+            if (z + 1 < z1) fetch(z + 2, z + 1);
+            const int slot = (z + dz) % 3;
 #pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = (__bf16)0.0f;
-            if (xx >= 0 && xx < S.nx && yy >= 0 && yy < S.ny && zz >= 0 && zz < S.nz)
-                v = *reinterpret_cast<const bf16x8 *>(act + (((size_t)zz * S.ny + yy) * S.nx + xx) * CI + c8 * 8);
-            *reinterpret_cast<bf16x8 *>(sa + hv * CI + c8 * 8) = v;
-        }
-        // stage deltas of the 32 x 8 tile (zero outside)
-        for (int e = tid; e < 256 * (CO / 8); e += 256) {
-            const int v = e / (CO / 8), c8 = e % (CO / 8);
-            const int xx = x0 + (v & 31), yy = y0 + (v >> 5);
-            bf16x8 d;
+            for (int y = 0; y < kWgY; ++y) {
+                bf16x8 a[MB];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) d[k] = (__bf16)0.0f;
-            if (xx < S.nx && yy < S.ny)
-                d = *reinterpret_cast<const bf16x8 *>(delta + (((size_t)z * S.ny + yy) * S.nx + xx) * CO + c8 * 8);
-            *reinterpret_cast<bf16x8 *>(sd + v * CO + c8 * 8) = d;
-        }
-        __syncthreads();
-        if (tid < NT) {
-            for (int v = 0; v < 256; ++v) {
-                const float dv = bf2f(sd[v * CO + co]);
-                accb += dv;
-                const int vx = v & 31, vy = v >> 5;
+                for (int i = 0; i < MB; ++i) {
+                    a[i] = *reinterpret_cast<const bf16x8 *>(&sd[y][i * 16 + m][kg * 8]);
+                    if (wave == 4) {
 #pragma unroll
-                for (int t = 0; t < kTaps; ++t) {
-                    const int dz = t / 9, dy = (t / 3) % 3, dx = t % 3;   // halo offsets 0..2
-                    const int hv = (dz * HY + vy + dy) * HX + vx + dx;
-                    const bf16x4 a = *reinterpret_cast<const bf16x4 *>(sa + hv * CI + cb * 4);
+                        for (int q = 0; q < 8; ++q) bias[i] += bf2f(a[i][q]);
+                    }
+                }
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) acc[c][t] = fmaf(dv, bf2f(a[c]), acc[c][t]);
+                for (int j = 0; j < NB; ++j) {
+                    const unsigned *p = reinterpret_cast<const unsigned *>(&sa[slot][y + dy][j * 16 + m][kg * 8]);
+                    const uint4 w = *reinterpret_cast<const uint4 *>(p);
+                    const unsigned w4 = p[4];
+                    const uint4 b1 = {__builtin_amdgcn_alignbit(w.y, w.x, 16), __builtin_amdgcn_alignbit(w.z, w.y, 16),
+                                      __builtin_amdgcn_alignbit(w.w, w.z, 16), __builtin_amdgcn_alignbit(w4, w.w, 16)};
+                    const uint4 b2 = {w.y, w.z, w.w, w4};
+#pragma unroll
+                    for (int i = 0; i < MB; ++i) {
+                        acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], __builtin_bit_cast(bf16x8, w),
+                                                                               acc[0][i][j], 0, 0, 0);
+                        acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], __builtin_bit_cast(bf16x8, b1),
+                                                                               acc[1][i][j], 0, 0, 0);
+                        acc[2][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], __builtin_bit_cast(bf16x8, b2),
+                                                                               acc[2][i][j], 0, 0, 0);
+                    }
                 }
             }
         }
     }
-    // partial layout per block: [CO][CI][27] weights then [CO] bias
     constexpr int NP = CO * CI * kTaps + CO;
     float *P = partial + (size_t)blockIdx.x * NP;
-    if (tid < NT) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+    for (int d = 0; d < 3; ++d)
 #pragma unroll
-            for (int t = 0; t < kTaps; ++t) P[(co * CI + cb * 4 + c) * kTaps + t] = acc[c][t];
-        if (cb == 0) P[CO * CI * kTaps + co] = accb;
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    P[((wave * 3 + d) * CO + i * 16 + kg * 4 + r) * CI + j * 16 + m] = acc[d][i][j][r];
+    if (wave == 4) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+            float t = bias[i];
+            t += __shfl_xor(t, 16, 64);
+            t += __shfl_xor(t, 32, 64);
+            if (kg == 0) P[CO * CI * kTaps + i * 16 + m] = t;
+        }
     }
 }
 
-// Deterministic reduction of per-block gradient partials into the flat
-// parameter layout of one layer ([co][ci][27] weights, then [co] bias):
-// partials use padded channel counts ([co_pad][ci_pad][27] + [co_pad]).
+// Deterministic reduction of per-block gradient partials ([27][co_pad][ci_pad]
+// + [co_pad]) into the flat parameter layout of one layer ([co][ci][27]
+// weights, then [co] bias): 32 values a block, eight threads each, which sum
+// consecutive shares of the partials, and then the shares in order.  One thread
+// per value took 123 us for 512 partials of 27680 values (one load in flight);
+// 5.4 us for 256 now.
 __global__ __launch_bounds__(256) void k_reduce_grad(const float *__restrict__ partial, int nblk, int ci_pad,
                                                      int co_pad, int ci_real, int co_real, float *__restrict__ out,
                                                      int accumulate)
 {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    const int nw = co_real * ci_real * kTaps;
-    if (i >= nw + co_real) return;
-    int src;
-    if (i < nw) {
-        const int co = i / (ci_real * kTaps), rem = i % (ci_real * kTaps);
-        src = (co * ci_pad + rem / kTaps) * kTaps + rem % kTaps;
-    } else {
-        src = co_pad * ci_pad * kTaps + (i - nw);
-    }
-    const size_t np = (size_t)co_pad * ci_pad * kTaps + co_pad;
+    __shared__ float share[8][32];
+    const int v = threadIdx.x & 31, g = threadIdx.x >> 5, i = blockIdx.x * 32 + v;
+    const int nw = co_pad * ci_pad * kTaps, np = nw + co_pad;
+    const int ci = i % ci_pad, co = i < nw ? i / ci_pad % co_pad : i - nw, t = i / ci_pad / co_pad;
+    const bool real = i < np && co < co_real && (i >= nw || ci < ci_real);
     float s = 0.0f;
-    for (int b = 0; b < nblk; ++b) s += partial[(size_t)b * np + src];
-    out[i] = accumulate ? out[i] + s : s;
+    if (real) {
+        const int each = (nblk + 7) / 8, b0 = g * each, b1 = min(b0 + each, nblk);
+#pragma unroll 4
+        for (int b = b0; b < b1; ++b) s += partial[(size_t)b * np + i];
+    }
+    share[g][v] = s;
+    __syncthreads();
+    if (g != 0 || !real) return;
+#pragma unroll
+    for (int k = 1; k < 8; ++k) s += share[k][v];
+    float *o = out + (i < nw ? (co * ci_real + ci) * kTaps + t : co_real * ci_real * kTaps + co);
+    *o = accumulate ? *o + s : s;
 }
 
 // SIRT step s = lambda * vinv * g.
@@ -1018,21 +1129,20 @@ hipError_t launch_conv3d(int cin_pad, int epi, const __bf16 *in, const __bf16 *w
     return hipGetLastError();
 }
 
-int wgrad_blocks(const CnnShape &S)
-{
-    const long tiles = (long)((S.nx + 31) / 32) * ((S.ny + 7) / 8) * S.nz;
-    return (int)(tiles < 512 ? tiles : 512);
-}
+int wgrad_blocks(const CnnShape &S) { return wgrad_plan(S).blocks; }
 
 hipError_t launch_conv3d_wgrad(int ci, int co, const __bf16 *act, const __bf16 *delta, float *partial, int nblk,
                                const CnnShape &S, hipStream_t st)
 {
+    const WgradPlan p = wgrad_plan(S);
+    if (nblk != p.blocks) return hipErrorInvalidValue;
+    const dim3 grid(nblk), block(kWgThreads);
     if (ci == 16 && co == 32)
-        hipLaunchKernelGGL((k_conv3d_wgrad<16, 32>), dim3(nblk), dim3(256), 0, st, act, delta, partial, S);
+        hipLaunchKernelGGL((k_conv3d_wgrad<16, 32>), grid, block, 0, st, act, delta, partial, S, p.zrun, p.items);
     else if (ci == 32 && co == 32)
-        hipLaunchKernelGGL((k_conv3d_wgrad<32, 32>), dim3(nblk), dim3(256), 0, st, act, delta, partial, S);
+        hipLaunchKernelGGL((k_conv3d_wgrad<32, 32>), grid, block, 0, st, act, delta, partial, S, p.zrun, p.items);
     else if (ci == 32 && co == 16)
-        hipLaunchKernelGGL((k_conv3d_wgrad<32, 16>), dim3(nblk), dim3(256), 0, st, act, delta, partial, S);
+        hipLaunchKernelGGL((k_conv3d_wgrad<32, 16>), grid, block, 0, st, act, delta, partial, S, p.zrun, p.items);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
@@ -1041,8 +1151,8 @@ hipError_t launch_conv3d_wgrad(int ci, int co, const __bf16 *act, const __bf16 *
 hipError_t launch_reduce_grad(const float *partial, int nblk, int ci_pad, int co_pad, int ci_real, int co_real,
                               float *out, int accumulate, hipStream_t st)
 {
-    const int n = co_real * ci_real * kTaps + co_real;
-    hipLaunchKernelGGL(k_reduce_grad, dim3((n + 255) / 256), dim3(256), 0, st, partial, nblk, ci_pad, co_pad, ci_real,
+    const int n = co_pad * ci_pad * kTaps + co_pad;
+    hipLaunchKernelGGL(k_reduce_grad, dim3((n + 31) / 32), dim3(256), 0, st, partial, nblk, ci_pad, co_pad, ci_real,
                        co_real, out, accumulate);
     return hipGetLastError();
 }
