@@ -31,7 +31,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kTaps = 27;
-constexpr int kConvZRun = 16;   // consecutive output slices per x-y tile of a conv block
+constexpr int kConvZRun = 16;   // consecutive output slices per x-y tile of a conv block, at most
 // output rows (y) per wave of k_conv3d: 4 for 16 input channels (two waves
 // per SIMD)
 constexpr int conv_rows(int cin) { return cin == 32 ? 8 : 4; }
@@ -43,7 +43,7 @@ __device__ __forceinline__ float bf2f(__bf16 v) { return (float)v; }
 template <int CIN, int EPI>
 __global__ __launch_bounds__(256) void k_conv3d(const __bf16 *__restrict__ in, const __bf16 *__restrict__ wts,
                                                 const float *__restrict__ bias, const __bf16 *__restrict__ mask,
-                                                void *__restrict__ out, CnnShape S)
+                                                void *__restrict__ out, CnnShape S, int zrun)
 {
     constexpr int NQ = CIN / 16;
     constexpr int NW = kTaps * NQ * 32 * 2;   // bf16x8 vectors of the A layout [tap][q][co][16]
@@ -55,14 +55,13 @@ __global__ __launch_bounds__(256) void k_conv3d(const __bf16 *__restrict__ in, c
     const int col = lane & 31, kh = lane >> 5;
     constexpr int R = conv_rows(CIN);   // output rows per wave
     const int tiles_x = (S.nx + 31) / 32, tiles_y = (S.ny + 4 * R - 1) / (4 * R);
-    const int zchunks = (S.nz + kConvZRun - 1) / kConvZRun;
+    const int zchunks = (S.nz + zrun - 1) / zrun;
     const int ncols = tiles_x * tiles_y * zchunks;
-    // a block walks one x-y tile through kConvZRun consecutive slices, so
+    // a block walks one x-y tile through zrun consecutive slices, so
     // the three input slices of an output slice were read by this CU for the
     // previous one (its L2 serves the dz reuse)
     for (int tcol = blockIdx.x; tcol < ncols; tcol += gridDim.x)
-    for (int z = (tcol / (tiles_x * tiles_y)) * kConvZRun,
-             zend = min(S.nz, z + kConvZRun); z < zend; ++z) {
+    for (int z = (tcol / (tiles_x * tiles_y)) * zrun, zend = min(S.nz, z + zrun); z < zend; ++z) {
         const int tx = tcol % tiles_x, ty = (tcol / tiles_x) % tiles_y;
         const int x = tx * 32 + col, y0 = ty * 4 * R + wave * R;
         f32x16 acc[R];
@@ -138,14 +137,15 @@ __global__ __launch_bounds__(256) void k_conv3d(const __bf16 *__restrict__ in, c
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const int c0 = 8 * s + 4 * kh;
-                bf16x4 o;
+                bf16x4 o, mk;
+                if (EPI == kEpiMask) mk = *reinterpret_cast<const bf16x4 *>(mask + vox * 32 + c0);
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
                     float v = acc[g][4 * s + u];
                     if (EPI == kEpiBiasRelu) {
                         v = fmaxf(v + bias[c0 + u], 0.0f);
                     } else if (EPI == kEpiMask) {
-                        v = bf2f(mask[vox * 32 + c0 + u]) > 0.0f ? v : 0.0f;
+                        v = bf2f(mk[u]) > 0.0f ? v : 0.0f;
                     }
                     o[u] = (__bf16)v;
                 }
@@ -221,7 +221,8 @@ __device__ __forceinline__ void shift_rows(bf16x8 halo, const bf16x8 *centre, bf
 // the store after the first step of the second plane: 0.83 -> 0.81 ms.
 constexpr int kC32zRows = 4;   // output rows per wave
 // Output slices per block task (zrun, a launch argument): 64 where that
-// still leaves at least kC32MinTasks tasks, else 32 or 16.  At 256^3, 64
+// still leaves at least kC32MinTasks tasks, else 32 or 16, or fewer where the
+// chip would idle (conv_tasks).  At 256^3, 64
 // against 32: about 2% less time per layer (fewer halo slices per run).
 constexpr int kC32MinTasks = 1024;
 template <int EPI>
@@ -358,6 +359,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 load_slice(zi + 1, nxt);
                 nhal = load_halo(zi + 1);
             }
+            // the mask of the output slice stored below, one 16-byte load per
+            // row in flight during the products before it (a voxel outside the
+            // volume: zero).  64^3, 64 blocks: 120 us with eight 2-byte loads
+            // per row at the store, 57 us
+            bf16x8 mk[R];
+            if (EPI == kEpiMask) {
+                const bool zok = zi - 1 >= z0;
+                const unsigned long long mb = (unsigned long long)(mask + (zok ? zi - 1 : 0) * oplane);
+                const __amdgpu_buffer_rsrc_t mrsrc = __builtin_amdgcn_make_buffer_rsrc(
+                    (void *)(((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(mb >> 32)) << 32) |
+                             (unsigned)__builtin_amdgcn_readfirstlane((unsigned)mb)),
+                    0, __builtin_amdgcn_readfirstlane(zok ? (int)(oplane * sizeof(__bf16)) : 0), 0x00020000);
+#pragma unroll
+                for (int g = 0; g < R; ++g) {
+                    const unsigned off = y0 + g < S.ny ? (unsigned)xoff_out + (unsigned)(y0 + g) * ostride : 0x80000000u;
+                    mk[g] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(mrsrc, off, 0, 0));
+                }
+            }
             const bool zin = zi >= 0 && zi < S.nz;   // uniform: a slice outside the volume contributes zero
             if (zin) {
                 shift_rows<0, R + 2>(hal, cur, sl, sh);
@@ -390,10 +409,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     for (int j = 0; j < 4; ++j) {
                         f32x2 v = {acc[0][g][j >> 1][2 * (j & 1)], acc[0][g][j >> 1][2 * (j & 1) + 1]};
                         if (EPI != kEpiBiasRelu) {
-                            const size_t vox = ((size_t)zo * S.ny + y) * S.nx + x;
 #pragma unroll
-                            for (int e = 0; e < 2; ++e)
-                                v[e] = x < S.nx && bf2f(mask[vox * 32 + 8 * kg + 2 * j + e]) > 0.0f ? v[e] : 0.0f;
+                            for (int e = 0; e < 2; ++e) v[e] = bf2f(mk[g][2 * j + e]) > 0.0f ? v[e] : 0.0f;
                         }
                         o[j] = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
                     }
@@ -445,7 +462,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // consecutive voxels of the padded row, both channels) and, for s = 0 and
 // g < 3, the tap (dz, dy, dx) = (+1, +1, g - 1) of the ninth tap row; the
 // remaining slots have zero weights.
-// A block owns a 16 x 32 tile (8 rows per wave) and walks kC2ZRun output
+// A block owns a 16 x 32 tile (8 rows per wave) and walks up to kC2ZRun output
 // slices: each input slice's 18 x 34 window (with the one-voxel halo; zero
 // outside the volume)
 // is loaded from the two FP32 inputs once, packed to BF16 pairs into a ring
@@ -457,13 +474,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // Rows per wave 2 / 4 / 8 / 16: 0.32 / 0.275 / 0.265 / 0.31 ms.
 constexpr int kC2Rows = 8;                               // output rows per wave
 constexpr int kC2TY = 4 * kC2Rows;                       // tile rows per block
-constexpr int kC2ZRun = 32;                              // output slices per block task
+constexpr int kC2ZRun = 32;                              // output slices per block task, at most
 constexpr int kC2HX = 18, kC2HY = kC2TY + 2;             // staged window of one input slice
 constexpr int kC2Win = kC2HX * kC2HY;                    // 324 voxels (one dword each)
 constexpr int kC2Ld = (kC2Win + 255) / 256;              // window dwords per thread
 __global__ __launch_bounds__(256) void k_conv3d_c2(const float *__restrict__ xin, const float *__restrict__ gin,
                                                    float g_scale, const __bf16 *__restrict__ wts,
-                                                   const float *__restrict__ bias, __bf16 *__restrict__ out, CnnShape S)
+                                                   const float *__restrict__ bias, __bf16 *__restrict__ out, CnnShape S,
+                                                   int zrun)
 {
     constexpr int R = kC2Rows;
     // slice zi in slot (zi + 1) mod 4; window column c is voxel x0 + c - 1
@@ -496,12 +514,12 @@ __global__ __launch_bounds__(256) void k_conv3d_c2(const float *__restrict__ xin
     for (int e = 0; e < 8; ++e) bv[e] = bias[8 * kg + e];
 
     const int tiles_x = (S.nx + 15) / 16, tiles_y = (S.ny + kC2TY - 1) / kC2TY;
-    const int zruns = (S.nz + kC2ZRun - 1) / kC2ZRun;
+    const int zruns = (S.nz + zrun - 1) / zrun;
     const int ntasks = tiles_x * tiles_y * zruns;
     const size_t plane = (size_t)S.ny * S.nx;   // voxels per slice
     for (int task = blockIdx.x; task < ntasks; task += gridDim.x) {
         const int x0 = (task % tiles_x) * 16, y0 = ((task / tiles_x) % tiles_y) * kC2TY;
-        const int z0 = (task / (tiles_x * tiles_y)) * kC2ZRun, z1 = min(S.nz, z0 + kC2ZRun);
+        const int z0 = (task / (tiles_x * tiles_y)) * zrun, z1 = min(S.nz, z0 + zrun);
         const int x = x0 + col;
         // window of input slice zi (voxels x0 - 1 .. x0 + 16, rows y0 - 1 ..
         // y0 + 16): voxel i of the window goes to thread i mod 256; outside
@@ -610,7 +628,7 @@ __global__ __launch_bounds__(256) void k_conv3d_c2(const float *__restrict__ xin
 // stores P in LDS, and each output gathers its nine taps of that slice.  A
 // slice contributes to the outputs one below (taps dz = +1), level (dz = 0)
 // and one above (dz = -1): three rolling sums per output, the lowest one
-// complete once the slice is done.  The block walks kConvZRun output slices.
+// complete once the slice is done.  The block walks up to kConvZRun output slices.
 // A 16 x 16 tile (38 KB of LDS, four blocks per CU) against 32 x 16 (70 KB,
 // two blocks): 0.28 -> 0.27 ms at 256^3, despite the larger halo share.
 constexpr int kO1TX = 16, kO1TY = 16, kO1HX = kO1TX + 2, kO1HY = kO1TY + 2;
@@ -622,7 +640,7 @@ constexpr int kO1Stride = kO1Tiles * 32 + 4;            // LDS floats per tap (+
 
 __global__ __launch_bounds__(256) void k_conv3d_out1(const __bf16 *__restrict__ in, const __bf16 *__restrict__ wts,
                                                      const float *__restrict__ bias, float *__restrict__ out,
-                                                     CnnShape S)
+                                                     CnnShape S, int zrun)
 {
     __shared__ float pl[kTaps * kO1Stride];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -641,12 +659,12 @@ __global__ __launch_bounds__(256) void k_conv3d_out1(const __bf16 *__restrict__ 
     const float b0 = bias[0];
     const size_t plane = (size_t)S.ny * S.nx * 32;   // bf16 elements per slice
     const int tiles_x = (S.nx + kO1TX - 1) / kO1TX, tiles_y = (S.ny + kO1TY - 1) / kO1TY;
-    const int zruns = (S.nz + kConvZRun - 1) / kConvZRun;
+    const int zruns = (S.nz + zrun - 1) / zrun;
     const int ncols = tiles_x * tiles_y * zruns;
     const int ox = threadIdx.x % kO1TX, oy0 = threadIdx.x / kO1TX;   // outputs (ox, oy0 + kO1Step k)
     for (int tcol = blockIdx.x; tcol < ncols; tcol += gridDim.x) {
         const int x0 = (tcol % tiles_x) * kO1TX, y0 = ((tcol / tiles_x) % tiles_y) * kO1TY;
-        const int zs = (tcol / (tiles_x * tiles_y)) * kConvZRun, ze = min(S.nz, zs + kConvZRun);
+        const int zs = (tcol / (tiles_x * tiles_y)) * zrun, ze = min(S.nz, zs + zrun);
         float acc_lo[kO1K], acc_mid[kO1K], acc_hi[kO1K];
 #pragma unroll
         for (int k = 0; k < kO1K; ++k) acc_lo[k] = acc_mid[k] = acc_hi[k] = 0.0f;
@@ -1079,11 +1097,22 @@ __global__ __launch_bounds__(256) void k_learned_candidate(const float *__restri
     xn[i] = fminf(fmaxf(x[i] + step[i] + out_scale * d[i], lo), hi);
 }
 
-int conv_grid(const CnnShape &S, int cin)
+// Output slices per block task: `most`, halved until every CU has two blocks.
+// A task of z slices reads z + 2, so short runs cost up to three times the
+// loads and pay where they put idle CUs to work.  At 64^3, 512 blocks against
+// `most` slices a task (16 to 64 blocks): 32 -> 32 channels 50 -> 21 us, 2 -> 32
+// 50 -> 11 us, 32 -> 1 28 -> 11 us, 1 -> 32 backwards 57 -> 17 us; 256 blocks
+// took 23, 11, 11 and 22 us, 1024 blocks 24, 11, 12 and 17 us.
+constexpr long kConvBlocks = 512;
+struct ZTasks {
+    int zrun;
+    long tasks;
+};
+ZTasks conv_tasks(long tiles, int nz, int most)
 {
-    const int ty = 4 * conv_rows(cin);
-    const long cols = (long)((S.nx + 31) / 32) * ((S.ny + ty - 1) / ty) * ((S.nz + kConvZRun - 1) / kConvZRun);
-    return (int)(cols < 2048 ? cols : 2048);
+    int z = most;
+    while (z > 1 && tiles * ((nz + z - 1) / z) < kConvBlocks) z /= 2;
+    return {z, tiles * ((nz + z - 1) / z)};
 }
 
 }  // namespace
@@ -1096,9 +1125,11 @@ hipError_t launch_conv3d(int cin_pad, int epi, const __bf16 *in, const __bf16 *w
                          void *out, const CnnShape &S, hipStream_t st)
 {
     if (!slice_fits(S)) return hipErrorInvalidValue;
-    const int grid = conv_grid(S, cin_pad);
+    const int ty = 4 * conv_rows(16);
+    const ZTasks T = conv_tasks((long)((S.nx + 31) / 32) * ((S.ny + ty - 1) / ty), S.nz, kConvZRun);
+    const dim3 grid((unsigned)std::min(T.tasks, 2048L));
 #define CTR_CONV(CIN, EPI)                                                                                          \
-    hipLaunchKernelGGL((k_conv3d<CIN, EPI>), dim3(grid), dim3(256), 0, st, in, w, bias, mask, out, S)
+    hipLaunchKernelGGL((k_conv3d<CIN, EPI>), grid, dim3(256), 0, st, in, w, bias, mask, out, S, T.zrun)
     if (cin_pad == 16) {
         if (epi == kEpiBiasRelu) CTR_CONV(16, kEpiBiasRelu);
         else if (epi == kEpiLinearF32) CTR_CONV(16, kEpiLinearF32);
@@ -1106,21 +1137,21 @@ hipError_t launch_conv3d(int cin_pad, int epi, const __bf16 *in, const __bf16 *w
         else return hipErrorInvalidValue;
     } else if (cin_pad == 32) {
         const long tiles = (long)((S.nx + 15) / 16) * ((S.ny + 4 * kC32zRows - 1) / (4 * kC32zRows));
-        int zrun = 64;
-        while (zrun > 16 && tiles * ((S.nz + zrun - 1) / zrun) < kC32MinTasks) zrun /= 2;
-        const long cols = tiles * ((S.nz + zrun - 1) / zrun);
-        const dim3 g32((unsigned)std::min(cols, 8192L));
+        int most = 64;
+        while (most > 16 && tiles * ((S.nz + most - 1) / most) < kC32MinTasks) most /= 2;
+        const ZTasks T = conv_tasks(tiles, S.nz, most);
+        const dim3 g32((unsigned)std::min(T.tasks, 8192L));
         if (epi == kEpiBiasRelu)
-            hipLaunchKernelGGL((k_conv3d_c32<kEpiBiasRelu>), g32, dim3(256), 0, st, in, w, bias, mask, out, S, zrun);
+            hipLaunchKernelGGL((k_conv3d_c32<kEpiBiasRelu>), g32, dim3(256), 0, st, in, w, bias, mask, out, S, T.zrun);
         else if (epi == kEpiLinearF32) {
             // one real output channel: the taps-as-rows kernel
-            const long cols = (long)((S.nx + kO1TX - 1) / kO1TX) * ((S.ny + kO1TY - 1) / kO1TY) *
-                              ((S.nz + kConvZRun - 1) / kConvZRun);
-            hipLaunchKernelGGL(k_conv3d_out1, dim3((unsigned)std::min(cols, 8192L)), dim3(256), 0, st, in, w, bias,
-                               (float *)out, S);
+            const ZTasks O = conv_tasks((long)((S.nx + kO1TX - 1) / kO1TX) * ((S.ny + kO1TY - 1) / kO1TY), S.nz,
+                                        kConvZRun);
+            hipLaunchKernelGGL(k_conv3d_out1, dim3((unsigned)std::min(O.tasks, 8192L)), dim3(256), 0, st, in, w, bias,
+                               (float *)out, S, O.zrun);
         }
         else if (epi == kEpiMask)
-            hipLaunchKernelGGL((k_conv3d_c32<kEpiMask>), g32, dim3(256), 0, st, in, w, bias, mask, out, S, zrun);
+            hipLaunchKernelGGL((k_conv3d_c32<kEpiMask>), g32, dim3(256), 0, st, in, w, bias, mask, out, S, T.zrun);
         else return hipErrorInvalidValue;
     } else {
         return hipErrorInvalidValue;
@@ -1190,9 +1221,9 @@ hipError_t launch_conv3d_first(const float *x, const float *g, float g_scale, co
                                __bf16 *out, const CnnShape &S, hipStream_t st)
 {
     if (!slice_fits(S)) return hipErrorInvalidValue;
-    const long tasks = (long)((S.nx + 15) / 16) * ((S.ny + kC2TY - 1) / kC2TY) * ((S.nz + kC2ZRun - 1) / kC2ZRun);
-    const dim3 grid((unsigned)std::min(tasks, 8192L));
-    hipLaunchKernelGGL(k_conv3d_c2, grid, dim3(256), 0, st, x, g, g_scale, w, bias, out, S);
+    const ZTasks T = conv_tasks((long)((S.nx + 15) / 16) * ((S.ny + kC2TY - 1) / kC2TY), S.nz, kC2ZRun);
+    const dim3 grid((unsigned)std::min(T.tasks, 8192L));
+    hipLaunchKernelGGL(k_conv3d_c2, grid, dim3(256), 0, st, x, g, g_scale, w, bias, out, S, T.zrun);
     return hipGetLastError();
 }
 
