@@ -28,7 +28,7 @@ thread_local std::string g_last_error;
 thread_local unsigned long long g_error_seq = 0;
 
 enum Slot { kWsIn = 0, kWsOut, kWsTmp, kWsR, kWsVinv, kWsPart, kWsSums, kWsG, kWsS, kWsD, kWsX2, kWsR2, kWsT, kWsYn,
-            kWsMask, kWsXs, kWsCells, kWsCount };
+            kWsMask, kWsXs, kWsCells, kWsBpParts, kWsCount };
 
 struct DevBuf {
     void *ptr = nullptr;
@@ -1472,6 +1472,16 @@ ctr_status ctr_cone_fp(ctr_ctx *ctx, const ctr_cone_geom *g, const float *vol, f
     return finish_out(ctx, dev, dp, proj, nray3(g));
 }
 
+static ctr_status bp_tiled(ctr_ctx *ctx, int kind, const BpParams &P, const float *src, float *vol, const char *what)
+{
+    const BpPlan &L = ctx->foot_bp.plan;
+    const int splits = bp_splits(kind, P, L);
+    if (splits > 1) TRY(buf_reserve(ctx, ctx->ws[kWsBpParts], sizeof(float) * splits * P.nt * P.ns * P.nz));
+    return check_launch(ctx, launch_bp_tiled(kind, P, L, (const int4 *)ctx->foot_bp.buf.ptr, src, vol,
+                                             splits > 1 ? (float *)ctx->ws[kWsBpParts].ptr : nullptr, ctx->stream),
+                        what);
+}
+
 ctr_status ctr_cone_bp_ref(ctr_ctx *ctx, const ctr_cone_geom *g, const float *proj, float *vol, unsigned flags)
 {
     TRY(check_cone(g, 1));
@@ -1485,8 +1495,7 @@ ctr_status ctr_cone_bp_ref(ctr_ctx *ctx, const ctr_cone_geom *g, const float *pr
     TRY(stage_out(ctx, dev, (flags & CTR_ACCUMULATE) != 0, kWsOut, vol, nvox3(g), &dv));
     BpParams P = cone_bp_params(ctx, g, flags);
     TRY(ensure_footprints(ctx, P, ctx->foot_bp, false));
-    TRY(check_launch(ctx, launch_bp_tiled(kBpRef, P, ctx->foot_bp.plan, (const int4 *)ctx->foot_bp.buf.ptr, dp, dv, ctx->stream),
-                     "cone reference backprojection"));
+    TRY(bp_tiled(ctx, kBpRef, P, dp, dv, "cone reference backprojection"));
     return finish_out(ctx, dev, dv, vol, nvox3(g));
 }
 
@@ -1583,8 +1592,7 @@ ctr_status ctr_fdk_bp(ctr_ctx *ctx, const ctr_cone_geom *g, const float *filtere
     TRY(stage_out(ctx, dev, (flags & CTR_ACCUMULATE) != 0, kWsOut, vol, nvox3(g), &dv));
     BpParams P = cone_bp_params(ctx, g, flags);
     TRY(ensure_footprints(ctx, P, ctx->foot_bp, false));
-    TRY(check_launch(ctx, launch_bp_tiled(kBpFdk, P, ctx->foot_bp.plan, (const int4 *)ctx->foot_bp.buf.ptr, dp, dv, ctx->stream),
-                     "FDK backprojection"));
+    TRY(bp_tiled(ctx, kBpFdk, P, dp, dv, "FDK backprojection"));
     return finish_out(ctx, dev, dv, vol, nvox3(g));
 }
 
@@ -1606,8 +1614,7 @@ ctr_status ctr_fdk(ctr_ctx *ctx, const ctr_cone_geom *g, int filter, const float
     TRY(cone_filter_impl(ctx, g, filter, dp, filt));
     BpParams P = cone_bp_params(ctx, g, flags);
     TRY(ensure_footprints(ctx, P, ctx->foot_bp, false));
-    TRY(check_launch(ctx, launch_bp_tiled(kBpFdk, P, ctx->foot_bp.plan, (const int4 *)ctx->foot_bp.buf.ptr, filt, dv, ctx->stream),
-                     "FDK backprojection"));
+    TRY(bp_tiled(ctx, kBpFdk, P, filt, dv, "FDK backprojection"));
     if (dev) HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));   // the filtered workspace is reused by the next call
     return finish_out(ctx, dev, dv, vol, nvox3(g));
 }
@@ -3296,7 +3303,7 @@ ctr_status ctr_autotune_cone(ctr_ctx *ctx, const ctr_cone_geom *g, ctr_tune_resu
         TRY(ensure_footprints(ctx, P, ctx->foot_bp, false));
         TRY(timed([&]() {
             return check_launch(ctx, launch_bp_tiled(kBpFdk, P, ctx->foot_bp.plan, (const int4 *)ctx->foot_bp.buf.ptr,
-                                                     proj, dst, st), "FDK backprojection");
+                                                     proj, dst, nullptr, st), "FDK backprojection");
         }, &res.bp_ms[i]));
         if (res.bp_ms[i] < bestv) {
             bestv = res.bp_ms[i];

@@ -250,8 +250,12 @@ struct BpPlan {
 BpPlan bp_plan(const BpParams &P, int pitch);        // pitch: 64, 72 or 80 floats per staged row
 BpPlan adjoint_plan(const BpParams &P, int cm);      // cm: 3, 4 or 6 candidate columns per chunk
 hipError_t launch_bp_footprints(const BpParams &P, const BpPlan &L, int4 *foot, hipStream_t st);
+// Small volumes: the views are split over bp_splits() sets of blocks, each
+// with a partial volume of its own in `parts` (splits x voxels; null: no split).
+int bp_share(long tiles, int nb);   // views per set of blocks
+int bp_splits(int kind, const BpParams &P, const BpPlan &L);
 hipError_t launch_bp_tiled(int kind, const BpParams &P, const BpPlan &L, const int4 *foot, const float *proj,
-                           float *vol, hipStream_t st);
+                           float *vol, float *parts, hipStream_t st);
 // proj is the adjoint's input already multiplied by the ray norm (P.adj_norm):
 // the SIRT residual kernels write it so, other callers scale with
 // launch_scale_by_norm first.  ones_input computes A'1 from P.adj_norm.
@@ -406,6 +410,8 @@ hipError_t launch_phantom(const PhantomEll *ell, int n_ell, int nt, int ns, int 
 hipError_t launch_diff_sums(const float *x, const float *ref, size_t n, double *partials, int *nblocks, hipStream_t st);
 
 // Utilities.
+// out = (accumulate ? out : 0) + parts[0] + parts[1] + ... (n floats each, added in order)
+hipError_t launch_sum_parts(const float *parts, int nparts, size_t n, float *out, int accumulate, hipStream_t st);
 hipError_t launch_fill(float *dst, float value, size_t n, hipStream_t st);
 // out [z][t][s] from in [z][s][t]; copy: null, or where in itself goes as well
 hipError_t launch_transpose_st(const float *in, float *out, float *copy, int nt, int ns, int nz, hipStream_t st);

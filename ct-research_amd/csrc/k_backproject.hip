@@ -166,12 +166,13 @@ __device__ __forceinline__ void dma_span(__amdgpu_buffer_rsrc_t rs, float *dst, 
 // fills the other with view b+1, so one barrier per view publishes the next
 // footprint and retires the previous one.  The view table is read through
 // the scalar cache (its own restrict argument), so no vector-memory wait in
-// the compute phase drains the prefetch.
+// the compute phase drains the prefetch.  Blocks of grid row s > 0 take the
+// s-th share of `share` views and the s-th of the partial volumes (bp_splits).
 template <int KIND, int TZ, int WP, int HMAX>
 __global__ __launch_bounds__(kThreads, 5) void k_bp_tiled(const float *__restrict__ proj, float *__restrict__ vol,
                                                        BpParams P, const int4 *__restrict__ foot,
                                                        const BpView *__restrict__ views,
-                                                       const float2 *__restrict__ zq)
+                                                       const float2 *__restrict__ zq, int share)
 {
     __shared__ float lds[2][HMAX * WP];
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -190,21 +191,22 @@ __global__ __launch_bounds__(kThreads, 5) void k_bp_tiled(const float *__restric
     // largest float below vmax: 0 <= v < vmax  <=>  med3(v, 0, vlast) == v
     const float vlast = __builtin_bit_cast(float, __builtin_bit_cast(int, P.vmax) - 1);
     const int4 *ft = foot + (size_t)tile * P.nb;
+    const int b0 = blockIdx.y * share, b1 = min(b0 + share, P.nb);
 
     float acc[TZ];
 #pragma unroll
     for (int k = 0; k < TZ; ++k) acc[k] = 0.0f;
 
-    int4 fn = ft[0];
-    issue_view<WP>(proj, P, 0, fn, lds[0]);
-    for (int b = 0; b < P.nb; ++b) {
+    int4 fn = ft[b0];
+    issue_view<WP>(proj, P, b0, fn, lds[b0 & 1]);
+    for (int b = b0; b < b1; ++b) {
         const int4 f = fn;
         const float *buf = lds[b & 1];
         // this wave's copies of view b are complete; after the barrier every
         // wave's are, and no wave still reads the other buffer (view b-1)
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        if (b + 1 < P.nb) {
+        if (b + 1 < b1) {
             fn = ft[b + 1];
             issue_view<WP>(proj, P, b + 1, fn, lds[(b + 1) & 1]);
         }
@@ -329,6 +331,7 @@ __global__ __launch_bounds__(kThreads, 5) void k_bp_tiled(const float *__restric
     }
 
     if (!col_in) return;
+    vol += blockIdx.y * ((size_t)P.nt * P.ns * P.nz);
 #pragma unroll
     for (int k = 0; k < TZ; ++k) {
         if (k < nzt) {
@@ -813,28 +816,53 @@ hipError_t launch_bp_footprints(const BpParams &Pin, const BpPlan &L, int4 *foot
 
 template <int KIND>
 static hipError_t launch_bp_kind(const BpParams &P, const BpPlan &L, const int4 *foot, const float *proj, float *vol,
-                                 hipStream_t st)
+                                 int share, hipStream_t st)
 {
-    const int nwg = L.tiles_t * L.tiles_s * L.tiles_z;
+    const dim3 grid(L.tiles_t * L.tiles_s * L.tiles_z, (P.nb + share - 1) / share);
     if (L.wp == 64)
-        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 64, 64>), dim3(nwg), dim3(kThreads), 0, st, proj, vol, P, foot,
-                           P.views, P.zq);
+        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 64, 64>), grid, dim3(kThreads), 0, st, proj, vol, P, foot,
+                           P.views, P.zq, share);
     else if (L.wp == 72)
-        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 72, 56>), dim3(nwg), dim3(kThreads), 0, st, proj, vol, P, foot,
-                           P.views, P.zq);
+        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 72, 56>), grid, dim3(kThreads), 0, st, proj, vol, P, foot,
+                           P.views, P.zq, share);
     else
-        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 80, 50>), dim3(nwg), dim3(kThreads), 0, st, proj, vol, P, foot,
-                           P.views, P.zq);
+        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 80, 50>), grid, dim3(kThreads), 0, st, proj, vol, P, foot,
+                           P.views, P.zq, share);
     return hipGetLastError();
 }
 
+// Views per set of blocks.  A tile is one block of four wavefronts, so a
+// volume below about 200^3 leaves CUs short of wavefronts: its views are then
+// split over several sets of blocks, up to kBpBlocks blocks (twice what the
+// chip holds, for the last blocks to even out) and not below kBpMinShare
+// views, and k_sum_parts adds the partial volumes (at most kBpBlocks tiles,
+// 42 MB).  Backprojection alone, one set of blocks against split: 32^3, 120
+// views 165 -> 14 us; 64^3, 360 views 516 -> 63 us; 128^3, 180 views 263 ->
+// 174 us; 150^3 322 -> 310 us; no difference from 1280 tiles on, where one set
+// is kept.  Half as many blocks: 59 us at 64^3, 187 us at 128^3.
+constexpr long kBpBlocks = 2560;
+constexpr int kBpMinShare = 4;
+int bp_share(long tiles, int nb)
+{
+    const long splits = std::min(kBpBlocks / tiles, (long)(nb / kBpMinShare));
+    return splits > 1 ? (int)((nb + splits - 1) / splits) : nb;
+}
+
+int bp_splits(int kind, const BpParams &P, const BpPlan &L)
+{
+    if (kind == kBpFdk && P.quirks) return 1;
+    const int share = bp_share((long)L.tiles_t * L.tiles_s * L.tiles_z, P.nb);
+    return (P.nb + share - 1) / share;
+}
+
 hipError_t launch_bp_tiled(int kind, const BpParams &Pin, const BpPlan &L, const int4 *foot, const float *proj,
-                           float *vol, hipStream_t st)
+                           float *vol, float *parts, hipStream_t st)
 {
     BpParams P = Pin;
+    const size_t nvox = (size_t)P.nt * P.ns * P.nz;
     if (kind == kBpFdk && P.quirks) {
         if (!P.accumulate) {
-            hipError_t e = hipMemsetAsync(vol, 0, sizeof(float) * (size_t)P.nt * P.ns * P.nz, st);
+            hipError_t e = hipMemsetAsync(vol, 0, sizeof(float) * nvox, st);
             if (e != hipSuccess) return e;
         }
         hipLaunchKernelGGL(k_fdk_quirk, dim3((P.nt + 15) / 16, (P.ns + 15) / 16), dim3(256), 0, st, proj, vol, P);
@@ -843,8 +871,14 @@ hipError_t launch_bp_tiled(int kind, const BpParams &Pin, const BpPlan &L, const
     P.tiles_t = L.tiles_t;
     P.tiles_s = L.tiles_s;
     P.tiles_z = L.tiles_z;
-    return kind == kBpFdk ? launch_bp_kind<kBpFdk>(P, L, foot, proj, vol, st)
-                          : launch_bp_kind<kBpRef>(P, L, foot, proj, vol, st);
+    const int splits = parts ? bp_splits(kind, P, L) : 1;
+    const int share = splits > 1 ? bp_share((long)L.tiles_t * L.tiles_s * L.tiles_z, P.nb) : P.nb;
+    float *dst = splits > 1 ? parts : vol;
+    if (splits > 1) P.accumulate = 0;
+    const hipError_t e = kind == kBpFdk ? launch_bp_kind<kBpFdk>(P, L, foot, proj, dst, share, st)
+                                        : launch_bp_kind<kBpRef>(P, L, foot, proj, dst, share, st);
+    if (e != hipSuccess || splits == 1) return e;
+    return launch_sum_parts(parts, splits, nvox, vol, Pin.accumulate, st);
 }
 
 template <int CM, bool FITALL>
