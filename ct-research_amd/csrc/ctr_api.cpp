@@ -1803,6 +1803,14 @@ ctr_status ctr_curved_filter(ctr_ctx *ctx, const ctr_curved_geom *g, const float
     return finish_out(ctx, dev, df, filtered, nrayc(g));
 }
 
+static ctr_status curved_bp(ctr_ctx *ctx, const CurvedBpParams &P, const float *src, float *vol)
+{
+    const int splits = curved_splits(P);
+    if (splits > 1) TRY(buf_reserve(ctx, ctx->ws[kWsBpParts], sizeof(float) * splits * P.nt * P.ns * P.nz));
+    float *parts = splits > 1 ? (float *)ctx->ws[kWsBpParts].ptr : nullptr;
+    return check_launch(ctx, launch_curved_bp(P, src, vol, parts, ctx->stream), "curved-detector backprojection");
+}
+
 ctr_status ctr_curved_bp(ctr_ctx *ctx, const ctr_curved_geom *g, const float *filtered, float *vol, unsigned flags)
 {
     TRY(check_curved(g));
@@ -1815,7 +1823,7 @@ ctr_status ctr_curved_bp(ctr_ctx *ctx, const ctr_curved_geom *g, const float *fi
     TRY(stage_out(ctx, dev, (flags & CTR_ACCUMULATE) != 0, kWsOut, vol, nvoxc(g), &dv));
     CurvedBpParams P = curved_bp_params(ctx, g, flags);
     TRY(curved_footprints(ctx, P));
-    TRY(check_launch(ctx, launch_curved_bp(P, df, dv, ctx->stream), "curved-detector backprojection"));
+    TRY(curved_bp(ctx, P, df, dv));
     return finish_out(ctx, dev, dv, vol, nvoxc(g));
 }
 
@@ -1834,7 +1842,7 @@ ctr_status ctr_curved_fdk(ctr_ctx *ctx, const ctr_curved_geom *g, const float *p
     TRY(curved_filter_impl(ctx, g, dp, filt));
     CurvedBpParams P = curved_bp_params(ctx, g, flags);
     TRY(curved_footprints(ctx, P));
-    TRY(check_launch(ctx, launch_curved_bp(P, filt, dv, ctx->stream), "curved-detector backprojection"));
+    TRY(curved_bp(ctx, P, filt, dv));
     if (dev) HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));   // the filtered workspace is reused by the next call
     return finish_out(ctx, dev, dv, vol, nvoxc(g));
 }

@@ -164,6 +164,22 @@ __device__ __forceinline__ float parker_weight(double b, double st, double g, do
     return 0.0f;
 }
 
+// atan(q) for |q| < kFanAtanMax: q + q^3 P(q^2), P the minimax polynomial of
+// (atan(sqrt(t)) / sqrt(t) - 1) / t on [0, 1/4]; relative error 3e-10 before
+// rounding.
+constexpr float kFanAtanMax = 0.5f;
+__device__ __forceinline__ float fan_atan(float q)
+{
+    const float t = q * q;
+    float c = 0.038723186f;
+    c = fmaf(c, t, -0.079840578f);
+    c = fmaf(c, t, 0.10940981f);
+    c = fmaf(c, t, -0.14272072f);
+    c = fmaf(c, t, 0.19999489f);
+    c = fmaf(c, t, -0.33333328f);
+    return fmaf(q * t, c, q);
+}
+
 // Curved (cylindrical, equiangular) cone-beam FDK backprojection.
 struct CurvedBpParams {
     int nt, ns, nz, ng, nx, nb;
@@ -184,7 +200,9 @@ struct CurvedBpParams {
 // the number of footprint entries (tiles x views).
 size_t curved_plan(CurvedBpParams &P);
 hipError_t launch_curved_footprints(const CurvedBpParams &P, int4 *foot, hipStream_t st);
-hipError_t launch_curved_bp(const CurvedBpParams &P, const float *filt, float *vol, hipStream_t st);
+// Sets of blocks that share the views of a small volume (see bp_splits).
+int curved_splits(const CurvedBpParams &P);
+hipError_t launch_curved_bp(const CurvedBpParams &P, const float *filt, float *vol, float *parts, hipStream_t st);
 
 // Fan-beam pixel-driven kernels.
 struct FanParams {

@@ -832,20 +832,21 @@ static hipError_t launch_bp_kind(const BpParams &P, const BpPlan &L, const int4 
 }
 
 // Views per set of blocks.  A tile is one block of four wavefronts, so a
-// volume below about 200^3 leaves CUs short of wavefronts: its views are then
+// volume below about 150^3 leaves CUs short of wavefronts: its views are then
 // split over several sets of blocks, up to kBpBlocks blocks (twice what the
-// chip holds, for the last blocks to even out) and not below kBpMinShare
-// views, and k_sum_parts adds the partial volumes (at most kBpBlocks tiles,
-// 42 MB).  Backprojection alone, one set of blocks against split: 32^3, 120
-// views 165 -> 14 us; 64^3, 360 views 516 -> 63 us; 128^3, 180 views 263 ->
-// 174 us; 150^3 322 -> 310 us; no difference from 1280 tiles on, where one set
-// is kept.  Half as many blocks: 59 us at 64^3, 187 us at 128^3.
+// chip holds, for the last blocks to even out), not below kBpMinShare views
+// and from three sets on, and k_sum_parts adds the partial volumes (at most
+// kBpBlocks tiles, 42 MB of 16 slices).  Backprojection alone, one set of
+// blocks against split: 32^3, 120 views 165 -> 14 us; 64^3, 360 views 516 ->
+// 63 us; 128^3, 180 views 263 -> 174 us.  Two sets are left out: 1000 tiles
+// gained 4% with 180 views, 1080 tiles lost 2% with 60.  Half as many blocks:
+// 59 us at 64^3, 187 us at 128^3.
 constexpr long kBpBlocks = 2560;
 constexpr int kBpMinShare = 4;
 int bp_share(long tiles, int nb)
 {
     const long splits = std::min(kBpBlocks / tiles, (long)(nb / kBpMinShare));
-    return splits > 1 ? (int)((nb + splits - 1) / splits) : nb;
+    return splits > 2 ? (int)((nb + splits - 1) / splits) : nb;
 }
 
 int bp_splits(int kind, const BpParams &P, const BpPlan &L)

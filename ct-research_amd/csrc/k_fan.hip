@@ -331,9 +331,7 @@ __device__ __forceinline__ float reciprocal(float v)
 //   equiangular (FanProjection.m:299-324): sum_b lerp(q)(gamma) / L^2 * dbeta,
 //   gamma = atan2(u, D - s), L^2 = u^2 + (D - s)^2
 // 8 x 8 pixels a block.  Where every lane's |u| < (D - s)/2, as inside any
-// usual fan, gamma is q + q^3 P(q^2) with q = u / (D - s) and P the minimax
-// polynomial of (atan(sqrt(t)) / sqrt(t) - 1) / t on [0, 1/4] (relative error
-// of gamma 3e-10); atan2f else.  360 views, 256^2, equiangular: 160 us for a
+// usual fan, gamma is fan_atan(u / (D - s)); atan2f else.  360 views, 256^2, equiangular: 160 us for a
 // thread per pixel, 43 us by eight wavefronts, 30 us with the shorter
 // angle and reciprocals.
 template <bool EQUIANGULAR>
@@ -359,16 +357,9 @@ __global__ __launch_bounds__(64 * kBpWaves, 8) void k_fan_fbp_bp(const float *__
             hit = pos >= 0.0f && pos < P.umax;
         } else {
             float g;
-            if (__all(!in || fabsf(u) < 0.5f * fabsf(w))) {
-                const float v = fabsf(w), r = __builtin_amdgcn_rcpf(v), q0 = u * r,
-                            q = fmaf(fmaf(-q0, v, u), r, q0), t = q * q;
-                float c = 0.038723186f;
-                c = fmaf(c, t, -0.079840578f);
-                c = fmaf(c, t, 0.10940981f);
-                c = fmaf(c, t, -0.14272072f);
-                c = fmaf(c, t, 0.19999489f);
-                c = fmaf(c, t, -0.33333328f);
-                g = fmaf(q * t, c, q);
+            if (__all(!in || fabsf(u) < kFanAtanMax * fabsf(w))) {
+                const float v = fabsf(w), r = __builtin_amdgcn_rcpf(v), q0 = u * r;
+                g = fan_atan(fmaf(fmaf(-q0, v, u), r, q0));
             } else {
                 g = atan2f(u, fabsf(w));
             }
