@@ -1615,7 +1615,6 @@ ctr_status ctr_fdk(ctr_ctx *ctx, const ctr_cone_geom *g, int filter, const float
     BpParams P = cone_bp_params(ctx, g, flags);
     TRY(ensure_footprints(ctx, P, ctx->foot_bp, false));
     TRY(bp_tiled(ctx, kBpFdk, P, filt, dv, "FDK backprojection"));
-    if (dev) HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));   // the filtered workspace is reused by the next call
     return finish_out(ctx, dev, dv, vol, nvox3(g));
 }
 
@@ -1712,7 +1711,6 @@ ctr_status ctr_fan_fbp(ctr_ctx *ctx, const ctr_fan_geom *g, int detector, int fi
     FanParams P = fan_params(ctx, g, flags);
     P.equiangular = detector == CTR_FAN_EQUIANGULAR;
     TRY(check_launch(ctx, launch_fan_fbp_bp(P, filt, di, ctx->stream), "fan FBP backprojection"));
-    if (dev) HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     return finish_out(ctx, dev, di, img, nvox2(g));
 }
 
@@ -1782,7 +1780,6 @@ ctr_status ctr_par_fbp(ctr_ctx *ctx, const ctr_par_geom *g, int filter, const fl
     TRY(par_filter_impl(ctx, g, filter, dp, filt));
     ParBpParams P = par_bp_params(ctx, g, true, flags);
     TRY(check_launch(ctx, launch_par_fbp_bp(P, filt, di, ctx->stream), "parallel FBP backprojection"));
-    if (dev) HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));   // the filtered workspace is reused by the next call
     return finish_out(ctx, dev, di, img, npix(g));
 }
 
@@ -1843,7 +1840,6 @@ ctr_status ctr_curved_fdk(ctr_ctx *ctx, const ctr_curved_geom *g, const float *p
     CurvedBpParams P = curved_bp_params(ctx, g, flags);
     TRY(curved_footprints(ctx, P));
     TRY(curved_bp(ctx, P, filt, dv));
-    if (dev) HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));   // the filtered workspace is reused by the next call
     return finish_out(ctx, dev, dv, vol, nvoxc(g));
 }
 

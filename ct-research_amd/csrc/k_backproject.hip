@@ -863,7 +863,7 @@ hipError_t launch_bp_tiled(int kind, const BpParams &Pin, const BpPlan &L, const
     const size_t nvox = (size_t)P.nt * P.ns * P.nz;
     if (kind == kBpFdk && P.quirks) {
         if (!P.accumulate) {
-            hipError_t e = hipMemsetAsync(vol, 0, sizeof(float) * nvox, st);
+            const hipError_t e = launch_fill(vol, 0.0f, nvox, st);
             if (e != hipSuccess) return e;
         }
         hipLaunchKernelGGL(k_fdk_quirk, dim3((P.nt + 15) / 16, (P.ns + 15) / 16), dim3(256), 0, st, proj, vol, P);

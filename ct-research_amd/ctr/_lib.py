@@ -391,7 +391,9 @@ class Context:
             import torch
             self._bind_torch_stream()
             if out is None:
-                out = torch.zeros(out_shape, dtype=torch.float32, device=inp.device)
+                # the operators write every element: no fill unless they add to it
+                make = torch.zeros if accumulate else torch.empty
+                out = make(out_shape, dtype=torch.float32, device=inp.device)
             assert out.dtype == torch.float32 and out.is_contiguous() and inp.is_contiguous()
             assert inp.dtype == torch.float32
             return inp.data_ptr(), out, out.data_ptr(), DEVICE_PTRS
@@ -403,7 +405,7 @@ class Context:
         return a, out, out.ctypes.data, 0
 
     def _run(self, fn, geom, inp, out_shape, out=None, flags=0, extra=()):
-        a, out, optr, f = self._io(inp, out_shape, out)
+        a, out, optr, f = self._io(inp, out_shape, out, bool(flags & ACCUMULATE))
         iptr = a if isinstance(a, int) else a.ctypes.data
         self._check(fn(self.h, ctypes.byref(geom.c), *extra, iptr, optr, f | flags))
         return out
