@@ -1516,10 +1516,16 @@ ctr_status ctr_cone_bp_adjoint(ctr_ctx *ctx, const ctr_cone_geom *g, const float
     TRY(buf_reserve(ctx, ctx->ws[kWsYn], nray3(g) * sizeof(float)));
     float *yn = (float *)ctx->ws[kWsYn].ptr;
     TRY(check_launch(ctx, launch_scale_by_norm(P, dp, yn, ctx->stream), "adjoint input scaling"));
-    TRY(check_launch(ctx,
-                     launch_adjoint(P, ctx->foot_adj.plan, (const int4 *)ctx->foot_adj.buf.ptr, yn, dv, nullptr, 0,
-                                    ctx->stream),
-                     "cone adjoint"));
+    const BpPlan &L = ctx->foot_adj.plan;
+    const int4 *foot = (const int4 *)ctx->foot_adj.buf.ptr;
+    const int splits = adjoint_splits(L, P.nb);
+    if (splits > 1) {
+        TRY(buf_reserve(ctx, ctx->ws[kWsBpParts], sizeof(float) * splits * nvox3(g)));
+        TRY(check_launch(ctx, launch_adjoint_split(P, L, foot, yn, dv, (float *)ctx->ws[kWsBpParts].ptr, ctx->stream),
+                         "cone adjoint"));
+    } else {
+        TRY(check_launch(ctx, launch_adjoint(P, L, foot, yn, dv, nullptr, 0, ctx->stream), "cone adjoint"));
+    }
     return finish_out(ctx, dev, dv, vol, nvox3(g));
 }
 

@@ -279,6 +279,12 @@ hipError_t launch_bp_tiled(int kind, const BpParams &P, const BpPlan &L, const i
 // launch_scale_by_norm first.  ones_input computes A'1 from P.adj_norm.
 hipError_t launch_adjoint(const BpParams &P, const BpPlan &L, const int4 *foot, const float *proj, float *vol,
                           const SirtUpdate *upd, int ones_input, hipStream_t st);
+// The adjoint with the views of a small volume split over adjoint_splits() sets
+// of blocks, each with a partial volume of its own in `parts`.  Not for SIRT,
+// whose residual history would show the order of the sums.
+int adjoint_splits(const BpPlan &L, int nb);
+hipError_t launch_adjoint_split(const BpParams &P, const BpPlan &L, const int4 *foot, const float *proj, float *vol,
+                                float *parts, hipStream_t st);
 // Fills P.adj_inva, adj_invb, adj_invxi and adj_norm (the pointers name the
 // destinations; P's views, pd and xd must be on the device).
 hipError_t launch_adjoint_tables(const BpParams &P, hipStream_t st);

@@ -490,7 +490,8 @@ struct AdjLds {
 template <int TZ, int WP, int CAPF, int CM, bool FITALL>
 __device__ __forceinline__ void adjoint_tile(const float *__restrict__ proj, float *__restrict__ vol, const BpParams &P,
                                              const int4 *__restrict__ foot, const BpView *__restrict__ views,
-                                             const SirtUpdate &U, int sirt, int ones, int tile, float *lds)
+                                             const SirtUpdate &U, int sirt, int ones, int tile, int b0, int b1,
+                                             float *lds)
 {
     constexpr int HMAX = AdjLds<TZ, WP, CAPF>::kHmax;
     float *yd = lds;                                // [HMAX][WP] (+ kCMax zero slack)
@@ -514,7 +515,7 @@ __device__ __forceinline__ void adjoint_tile(const float *__restrict__ proj, flo
 #pragma unroll
     for (int k = 0; k < TZ; ++k) acc[k] = 0.0f;
 
-    for (int b = 0; b < P.nb; ++b) {
+    for (int b = b0; b < b1; ++b) {
         const int4 f = ft[b];
         if (f.w & kFootEmpty) continue;
         // FITALL: the host found every footprint of the plan small enough
@@ -653,15 +654,18 @@ __device__ __forceinline__ void adjoint_tile(const float *__restrict__ proj, flo
 // (spills) 17.3 ms; eight at four 19.3 ms; five at six 17.3 ms; four at six
 // 16.9 ms, at seven (spills) 17.6 ms, at eight 18.9 ms; three at seven or
 // eight 19.4 ms; two at eight 22.6 ms.  The variant with the global path
-// keeps four waves.
+// keeps four waves.  Blocks of grid row s > 0 take the s-th share of `share`
+// views and the s-th of the partial volumes (adjoint_splits).
 template <int TZ, int WP, int CAPF, int CM, bool FITALL>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FITALL ? 6 : 4, FITALL ? 6 : 4))) void k_adjoint(const float *__restrict__ proj, float *__restrict__ vol, BpParams P,
                                                       const int4 *__restrict__ foot, const BpView *__restrict__ views,
-                                                      SirtUpdate U, int sirt, int ones)
+                                                      SirtUpdate U, int sirt, int ones, int share)
 {
     __shared__ __align__(16) float lds[AdjLds<TZ, WP, CAPF>::kFloats];
+    const int b0 = blockIdx.y * share;
+    vol += blockIdx.y * ((size_t)P.nt * P.ns * P.nz);
     adjoint_tile<TZ, WP, CAPF, CM, FITALL>(proj, vol, P, foot, views, U, sirt, ones, xcd_tile(blockIdx.x, gridDim.x),
-                                           lds);
+                                           b0, min(b0 + share, P.nb), lds);
 }
 
 // Many independent problems in one launch: block b belongs to the job whose
@@ -677,7 +681,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FITALL
     const BpParams P = jobs[p].P;
     const SirtUpdate U = jobs[p].U;
     adjoint_tile<TZ, WP, CAPF, CM, FITALL>(jobs[p].proj, jobs[p].vol, P, jobs[p].foot, P.views, U, sirt, ones,
-                                           xcd_tile(local, jobs[p].nblocks), lds);
+                                           xcd_tile(local, jobs[p].nblocks), 0, P.nb, lds);
 }
 
 // Number of (tile, view) footprints of a plan that are not empty and do not
@@ -884,45 +888,84 @@ hipError_t launch_bp_tiled(int kind, const BpParams &Pin, const BpPlan &L, const
 
 template <int CM, bool FITALL>
 static hipError_t launch_adjoint_cm(const BpParams &P, const BpPlan &L, const int4 *foot, const float *proj,
-                                    float *vol, const SirtUpdate &U, int sirt, int ones_input, hipStream_t st)
+                                    float *vol, const SirtUpdate &U, int sirt, int ones_input, int share,
+                                    hipStream_t st)
 {
-    const int nwg = L.tiles_t * L.tiles_s * L.tiles_z;
+    const dim3 grid(L.tiles_t * L.tiles_s * L.tiles_z, (P.nb + share - 1) / share);
     if (L.wp == 40)
-        hipLaunchKernelGGL((k_adjoint<kAdjTZ, 40, adj_cap(40), CM, FITALL>), dim3(nwg), dim3(kThreads), 0, st, proj, vol,
-                           P, foot, P.views, U, sirt, ones_input);
+        hipLaunchKernelGGL((k_adjoint<kAdjTZ, 40, adj_cap(40), CM, FITALL>), grid, dim3(kThreads), 0, st, proj, vol,
+                           P, foot, P.views, U, sirt, ones_input, share);
     else if (L.wp == 72)
-        hipLaunchKernelGGL((k_adjoint<kAdjTZ, 72, adj_cap(72), CM, FITALL>), dim3(nwg), dim3(kThreads), 0, st, proj, vol,
-                           P, foot, P.views, U, sirt, ones_input);
+        hipLaunchKernelGGL((k_adjoint<kAdjTZ, 72, adj_cap(72), CM, FITALL>), grid, dim3(kThreads), 0, st, proj, vol,
+                           P, foot, P.views, U, sirt, ones_input, share);
     else
-        hipLaunchKernelGGL((k_adjoint<kAdjTZ, 136, adj_cap(136), CM, FITALL>), dim3(nwg), dim3(kThreads), 0, st, proj,
-                           vol, P, foot, P.views, U, sirt, ones_input);
+        hipLaunchKernelGGL((k_adjoint<kAdjTZ, 136, adj_cap(136), CM, FITALL>), grid, dim3(kThreads), 0, st, proj,
+                           vol, P, foot, P.views, U, sirt, ones_input, share);
     return hipGetLastError();
 }
 
 template <int CM>
 static hipError_t launch_adjoint_fit(const BpParams &P, const BpPlan &L, const int4 *foot, const float *proj,
-                                     float *vol, const SirtUpdate &U, int sirt, int ones_input, hipStream_t st)
+                                     float *vol, const SirtUpdate &U, int sirt, int ones_input, int share,
+                                     hipStream_t st)
 {
-    return L.fit_all ? launch_adjoint_cm<CM, true>(P, L, foot, proj, vol, U, sirt, ones_input, st)
-                     : launch_adjoint_cm<CM, false>(P, L, foot, proj, vol, U, sirt, ones_input, st);
+    return L.fit_all ? launch_adjoint_cm<CM, true>(P, L, foot, proj, vol, U, sirt, ones_input, share, st)
+                     : launch_adjoint_cm<CM, false>(P, L, foot, proj, vol, U, sirt, ones_input, share, st);
 }
 
-hipError_t launch_adjoint(const BpParams &Pin, const BpPlan &L, const int4 *foot, const float *proj, float *vol,
-                          const SirtUpdate *upd, int ones_input, hipStream_t st)
+static hipError_t launch_adjoint_share(const BpParams &Pin, const BpPlan &L, const int4 *foot, const float *proj,
+                                       float *vol, const SirtUpdate &U, int sirt, int ones_input, int share,
+                                       hipStream_t st)
 {
     BpParams P = Pin;
     P.tiles_t = L.tiles_t;
     P.tiles_s = L.tiles_s;
     P.tiles_z = L.tiles_z;
-    SirtUpdate U = {};
-    int sirt = 0;
-    if (upd) {
-        U = *upd;
-        sirt = 1;
-    }
-    if (L.cm == 3) return launch_adjoint_fit<3>(P, L, foot, proj, vol, U, sirt, ones_input, st);
-    if (L.cm == 4) return launch_adjoint_fit<4>(P, L, foot, proj, vol, U, sirt, ones_input, st);
-    return launch_adjoint_fit<6>(P, L, foot, proj, vol, U, sirt, ones_input, st);
+    if (L.cm == 3) return launch_adjoint_fit<3>(P, L, foot, proj, vol, U, sirt, ones_input, share, st);
+    if (L.cm == 4) return launch_adjoint_fit<4>(P, L, foot, proj, vol, U, sirt, ones_input, share, st);
+    return launch_adjoint_fit<6>(P, L, foot, proj, vol, U, sirt, ones_input, share, st);
+}
+
+hipError_t launch_adjoint(const BpParams &P, const BpPlan &L, const int4 *foot, const float *proj, float *vol,
+                          const SirtUpdate *upd, int ones_input, hipStream_t st)
+{
+    return launch_adjoint_share(P, L, foot, proj, vol, upd ? *upd : SirtUpdate{}, upd ? 1 : 0, ones_input, P.nb, st);
+}
+
+// Views per set of blocks of the adjoint.  The chip holds 1536 blocks (tiles of
+// 16 x 16 x 4), so a volume of few of them leaves CUs idle, and one of a few
+// thousand most of them in its last round: up to 16384 blocks in up to ten
+// sets, or as many sets as make 2560 blocks, of at least 4 views, and of 16
+// (32) where one set has 1024 (4096) tiles and more to write.  One set
+// against split: 32^3, 60 views 114 -> 18 us; 64^3, 120 views 236 -> 88 us;
+// 128^3, 120 views 581 -> 519 us; 150 x 130 x 101, 120 views 671 -> 562 us (3
+// sets 581); 176^3, 120 views 1268 -> 1223 us; 192^3, 40 views 579 -> 589 us in
+// two sets, and 162 x 139 x 109, 24 views 161 -> 168 us in five, so one there.
+// 64^3 in 32 sets 92 us, 96^3 in 18 sets 245 us against
+// 234 in nine.
+constexpr long kAdjBlocks = 16384, kAdjSets = 10;
+static int adjoint_share(const BpPlan &L, int nb)
+{
+    const long tiles = (long)L.tiles_t * L.tiles_s * L.tiles_z;
+    const long sets = std::min(kAdjBlocks / tiles, std::max(kAdjSets, kBpBlocks / tiles));
+    const long splits = std::min(sets, (long)(nb / (tiles >= 4096 ? 32 : (tiles >= 1024 ? 16 : kBpMinShare))));
+    return splits > 1 ? (int)((nb + splits - 1) / splits) : nb;
+}
+
+int adjoint_splits(const BpPlan &L, int nb)
+{
+    const int share = adjoint_share(L, nb);
+    return (nb + share - 1) / share;
+}
+
+hipError_t launch_adjoint_split(const BpParams &Pin, const BpPlan &L, const int4 *foot, const float *proj, float *vol,
+                                float *parts, hipStream_t st)
+{
+    BpParams P = Pin;
+    P.accumulate = 0;
+    const hipError_t e = launch_adjoint_share(P, L, foot, proj, parts, SirtUpdate{}, 0, 0, adjoint_share(L, P.nb), st);
+    if (e != hipSuccess) return e;
+    return launch_sum_parts(parts, adjoint_splits(L, P.nb), (size_t)P.nt * P.ns * P.nz, vol, Pin.accumulate, st);
 }
 
 template <int CM, bool FITALL>

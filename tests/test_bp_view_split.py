@@ -1,7 +1,8 @@
-"""Backprojection of small volumes with the views split over sets of blocks:
-too few views for a split, shares with a remainder, one tile and several
-ragged ones.  Bounds: the ones of the suite's single-pass FDK and reference
-backprojections (the split changes the order of the sums only)."""
+"""Backprojection and exact adjoint of small volumes with the views split over
+sets of blocks: too few views for a split, shares with a remainder, one tile
+and several ragged ones.  Bounds: the ones of the suite's single-pass FDK,
+reference backprojection and adjoint (the split changes the order of the sums
+only)."""
 import numpy as np
 import pytest
 
@@ -28,3 +29,21 @@ def test_split_views(ctx, oracle, shape, views):
     report(f"split_bp[{shape},{views}]", rel_l2=e, max_rel=m, ref_rel_l2=e2, ref_max_rel=m2)
     assert e < 3e-5 and m < 1e-4 and e2 < 3e-5 and m2 < 1e-4
     np.testing.assert_array_equal(ctx.fdk_bp(g, y, out=img.copy(), flags=ctr.ACCUMULATE), img + img)
+
+
+@pytest.mark.parametrize("views", [2, 7, 8, 9, 41])
+@pytest.mark.parametrize("shape", [(16, 16, 4), (21, 17, 19)])
+def test_split_adjoint(ctx, oracle, shape, views):
+    import ctr
+    nt, ns, nz = shape
+    beta = (2 * np.pi / views * np.arange(views) + 0.1).astype(np.float32)
+    p, xi = (np.linspace(-1, 1, n).astype(np.float32) * np.float32(16.0) for n in (37, 33))
+    a = (nt, ns, nz, (nt * 1.0, ns * 1.1, nz * 0.9), 60.0, beta, p, xi)
+    g, og = ctr.ConeGeom(*a), oracle.Cone(*a)
+    y = np.random.default_rng(views).random(g.nray).astype(np.float32)
+    print(f"[case] split adjoint {shape}, {views} views", flush=True)
+    vol = ctx.cone_bp_adjoint(g, y)
+    e, m = errs(vol, oracle.cone_adjoint(og, y))
+    report(f"split_adjoint[{shape},{views}]", rel_l2=e, max_rel=m)
+    assert e < 1e-4 and m < 1e-3
+    np.testing.assert_array_equal(ctx.cone_bp_adjoint(g, y, out=vol.copy(), flags=ctr.ACCUMULATE), vol + vol)
