@@ -268,9 +268,9 @@ struct BpPlan {
 BpPlan bp_plan(const BpParams &P, int pitch);        // pitch: 64, 72 or 80 floats per staged row
 BpPlan adjoint_plan(const BpParams &P, int cm);      // cm: 3, 4 or 6 candidate columns per chunk
 hipError_t launch_bp_footprints(const BpParams &P, const BpPlan &L, int4 *foot, hipStream_t st);
-// Small volumes: the views are split over bp_splits() sets of blocks, each
+// The views of a volume of few tiles are split over bp_splits() sets of blocks, each
 // with a partial volume of its own in `parts` (splits x voxels; null: no split).
-int bp_share(long tiles, int nb);   // views per set of blocks
+int bp_share(long tiles, int nb, size_t nvox);   // views per set of blocks
 int bp_splits(int kind, const BpParams &P, const BpPlan &L);
 hipError_t launch_bp_tiled(int kind, const BpParams &P, const BpPlan &L, const int4 *foot, const float *proj,
                            float *vol, float *parts, hipStream_t st);

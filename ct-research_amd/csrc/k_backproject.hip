@@ -835,28 +835,34 @@ static hipError_t launch_bp_kind(const BpParams &P, const BpPlan &L, const int4 
     return hipGetLastError();
 }
 
-// Views per set of blocks.  A tile is one block of four wavefronts, so a
-// volume below about 150^3 leaves CUs short of wavefronts: its views are then
-// split over several sets of blocks, up to kBpBlocks blocks (twice what the
-// chip holds, for the last blocks to even out), not below kBpMinShare views
-// and from three sets on, and k_sum_parts adds the partial volumes (at most
-// kBpBlocks tiles, 42 MB of 16 slices).  Backprojection alone, one set of
-// blocks against split: 32^3, 120 views 165 -> 14 us; 64^3, 360 views 516 ->
-// 63 us; 128^3, 180 views 263 -> 174 us.  Two sets are left out: 1000 tiles
-// gained 4% with 180 views, 1080 tiles lost 2% with 60.  Half as many blocks:
-// 59 us at 64^3, 187 us at 128^3.
-constexpr long kBpBlocks = 2560;
+// Views per set of blocks.  A tile is one block of four wavefronts and the chip
+// holds 1280: a volume of fewer tiles leaves CUs short of wavefronts, and one
+// of a few thousand loses about 0.58 / rounds of its time in the last round
+// (rounds = tiles x sets / 1280).  The partial volumes cost a write and a read
+// a set, which the views pay for: the sum of both is least at
+// sqrt(160 views / tiles) sets.  That many are taken, from 2.3 on, in shares of
+// at least four views, up to four sets (or 2560 blocks) and kBpPartsBytes.
+// Backprojection alone, one set against split: 32^3, 120 views 165 -> 14 us;
+// 64^3, 360 views 516 -> 61 us; 128^3, 180 views 263 -> 174 us; 176^3, 180
+// views 497 -> 378 us (2 sets 414); 176^3, 60 views 169 -> 148 us; 256^3, 360
+// views 2616 -> 2498 us; 256^3, 90 views 581 -> 606 us in two sets, so one.
+constexpr double kBpSetsScale = 160.0;
+constexpr size_t kBpPartsBytes = (size_t)384 << 20;
 constexpr int kBpMinShare = 4;
-int bp_share(long tiles, int nb)
+constexpr long kBpBlocks = 2560;
+int bp_share(long tiles, int nb, size_t nvox)
 {
-    const long splits = std::min(kBpBlocks / tiles, (long)(nb / kBpMinShare));
-    return splits > 2 ? (int)((nb + splits - 1) / splits) : nb;
+    const double best = std::sqrt(kBpSetsScale * nb / tiles);
+    if (best < 2.3) return nb;
+    const long splits = std::min(std::min(std::lround(best), std::max(4L, kBpBlocks / tiles)),
+                                 std::min((long)(nb / kBpMinShare), (long)(kBpPartsBytes / (sizeof(float) * nvox))));
+    return splits > 1 ? (int)((nb + splits - 1) / splits) : nb;
 }
 
 int bp_splits(int kind, const BpParams &P, const BpPlan &L)
 {
     if (kind == kBpFdk && P.quirks) return 1;
-    const int share = bp_share((long)L.tiles_t * L.tiles_s * L.tiles_z, P.nb);
+    const int share = bp_share((long)L.tiles_t * L.tiles_s * L.tiles_z, P.nb, (size_t)P.nt * P.ns * P.nz);
     return (P.nb + share - 1) / share;
 }
 
@@ -877,7 +883,7 @@ hipError_t launch_bp_tiled(int kind, const BpParams &Pin, const BpPlan &L, const
     P.tiles_s = L.tiles_s;
     P.tiles_z = L.tiles_z;
     const int splits = parts ? bp_splits(kind, P, L) : 1;
-    const int share = splits > 1 ? bp_share((long)L.tiles_t * L.tiles_s * L.tiles_z, P.nb) : P.nb;
+    const int share = splits > 1 ? bp_share((long)L.tiles_t * L.tiles_s * L.tiles_z, P.nb, (size_t)P.nt * P.ns * P.nz) : P.nb;
     float *dst = splits > 1 ? parts : vol;
     if (splits > 1) P.accumulate = 0;
     const hipError_t e = kind == kBpFdk ? launch_bp_kind<kBpFdk>(P, L, foot, proj, dst, share, st)

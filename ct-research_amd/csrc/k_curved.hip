@@ -345,7 +345,7 @@ hipError_t launch_curved_footprints(const CurvedBpParams &P, int4 *foot, hipStre
 
 int curved_splits(const CurvedBpParams &P)
 {
-    const int share = bp_share((long)P.tiles_t * P.tiles_s * P.tiles_z, P.nb);
+    const int share = bp_share((long)P.tiles_t * P.tiles_s * P.tiles_z, P.nb, (size_t)P.nt * P.ns * P.nz);
     return (P.nb + share - 1) / share;
 }
 
@@ -354,7 +354,7 @@ hipError_t launch_curved_bp(const CurvedBpParams &Pin, const float *filt, float 
     if (!Pin.foot) return hipErrorInvalidValue;
     CurvedBpParams P = Pin;
     const int splits = parts ? curved_splits(P) : 1;
-    const int share = splits > 1 ? bp_share((long)P.tiles_t * P.tiles_s * P.tiles_z, P.nb) : P.nb;
+    const int share = splits > 1 ? bp_share((long)P.tiles_t * P.tiles_s * P.tiles_z, P.nb, (size_t)P.nt * P.ns * P.nz) : P.nb;
     float *dst = splits > 1 ? parts : vol;
     if (splits > 1) P.accumulate = 0;
     hipError_t e = hipErrorInvalidValue;
