@@ -447,30 +447,56 @@ __device__ __forceinline__ void column_box(const BpParams &P, const BpView &vw, 
     cu1 = (int)floorf(fminf(umax + eu, (float)P.np));
 }
 
-// Candidate detector rows of the voxel slice [zb, zt] (relative to the
-// source plane) seen through a column with magnification in [mmin, mmax].
-__device__ __forceinline__ void slice_rows(const BpParams &P, float zb, float zt, float mmin, float mmax, int &rv0,
-                                           int &rv1)
+// floor(x) as an int (one instruction; saturates)
+__device__ __forceinline__ int floor_int(float x)
 {
-    // extreme products of {zb, zt} x {mmin, mmax}.  The magnifications are
-    // positive (the geometry check keeps the source orbit outside the
-    // volume, so every voxel corner lies in front of the source), zb < zt,
-    // and rounding is monotone: the smallest product is zb times mmin or
-    // mmax by the sign of zb, the largest zt times mmax or mmin by the sign
-    // of zt (uniform over the block), bit for bit the min and max of all four
-    const float zlo = zb * (zb >= 0.0f ? mmin : mmax);
-    const float zhi = zt * (zt >= 0.0f ? mmax : mmin);
-    float v0 = fmaf(zlo, P.v_scale, P.v_off);
-    float v1 = fmaf(zhi, P.v_scale, P.v_off);
-    if (P.v_scale < 0.0f) {
-        const float t = v0;
-        v0 = v1;
-        v1 = t;
-    }
-    const float ev = 1e-3f + 4e-6f * fmaxf(fabsf(v0), fabsf(v1));
-    rv0 = (int)ceilf(fmaxf(v0 - ev, -1.0f));
-    rv1 = (int)floorf(fminf(v1 + ev, (float)P.nx));
+    int r;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
 }
+
+__device__ __forceinline__ float uniform(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
+// Candidate detector rows of a tile's slices.  Slice [zb, zt] (relative to the
+// source plane) seen through a column with magnification in [mmin, mmax] spans
+// the extreme products of {zb, zt} x {mmin, mmax}.  The magnifications are
+// positive (the geometry check keeps the source orbit outside the volume, so
+// every voxel corner lies in front of the source) and zb < zt: the smallest
+// product is zb times mmin or mmax by the sign of zb, the largest zt times mmax
+// or mmin by the sign of zt, which is uniform over the block and decided once.
+// A margin of 1e-3 rows and 4e-6 of the detector's rows covers the rounding; a
+// row that is a candidate without need adds 0.
+template <int TZ>
+struct SliceRows {
+    float low[TZ], high[TZ];             // face that the lowest / highest row comes from
+    bool low_far[TZ], high_far[TZ];      // its product with mmax (else mmin)
+    float off_low, off_high;
+
+    __device__ __forceinline__ SliceRows(const BpParams &P, float zbase)
+    {
+        const bool up = P.v_scale >= 0.0f;
+#pragma unroll
+        for (int k = 0; k < TZ; ++k) {
+            const float zb = uniform(fmaf((float)k, P.rz, zbase)), zt = uniform(zb + P.rz);
+            low[k] = up ? zb : zt;
+            high[k] = up ? zt : zb;
+            low_far[k] = up ? zb < 0.0f : zt >= 0.0f;
+            high_far[k] = up ? zt >= 0.0f : zb < 0.0f;
+        }
+        const float margin = 1e-3f + 4e-6f * (float)P.nx;
+        off_low = P.v_off - margin + 1.0f;   // the first row above: floor(v - margin) + 1
+        off_high = P.v_off + margin;
+    }
+    // smin, smax: mmin, mmax times v_scale
+    __device__ __forceinline__ void rows(int k, float smin, float smax, int first, int last, int &rv0, int &rv1) const
+    {
+        rv0 = max(floor_int(fmaf(low[k], low_far[k] ? smax : smin, off_low)), first);
+        rv1 = min(floor_int(fmaf(high[k], high_far[k] ? smax : smin, off_high)), last);
+    }
+};
 
 // Rows of the staged footprint and floats of LDS per adjoint block: the
 // footprint rows, the column tables, and the z-slab interval table of
@@ -511,6 +537,7 @@ __device__ __forceinline__ void adjoint_tile(const float *__restrict__ proj, flo
     // then only ever see finite values (their segment length is 0)
     for (int e = threadIdx.x; e < CAPF; e += kThreads) lds[e] = 0.0f;
 
+    const SliceRows<TZ> slices(P, zbase);
     float acc[TZ];
 #pragma unroll
     for (int k = 0; k < TZ; ++k) acc[k] = 0.0f;
@@ -565,6 +592,7 @@ __device__ __forceinline__ void adjoint_tile(const float *__restrict__ proj, flo
         const int rlo_lim = fits ? f.y : 0, rhi_lim = fits ? f.y + H - 1 : P.nx - 1;
         cu0 = max(cu0, clo_lim);
         cu1 = min(cu1, chi_lim);
+        const float smin = mmin * P.v_scale, smax = mmax * P.v_scale;
         // voxel low faces relative to the source, in FP64: for a ray nearly
         // parallel to a slab (small a or b) the slab's parameter interval is
         // this offset divided by that component, so its rounding is
@@ -588,38 +616,35 @@ __device__ __forceinline__ void adjoint_tile(const float *__restrict__ proj, flo
                 float l0, h0, l1, h1;
                 slab_interval(tlo, P.rt, ia, l0, h0);
                 slab_interval(slo, P.rs, ib, l1, h1);
-                // the ray's interval in the voxel column; invalid or empty
-                // candidates become [0, 0], which overlaps nothing
-                const float lo_ = fmaxf(l0, l1), hi_ = fminf(h0, h1);
-                const bool live = cb + q <= cu1 && lo_ < hi_;
-                clo[q] = live ? lo_ : 0.0f;
-                chi[q] = live ? hi_ : 0.0f;
+                // the ray's interval in the voxel column; an invalid or empty
+                // candidate ends where it begins and overlaps nothing
+                const float lo_ = fmaxf(l0, l1), hi_ = fmaxf(fminf(h0, h1), lo_);
+                clo[q] = lo_;
+                chi[q] = cb + q <= cu1 ? hi_ : lo_;
             }
 #pragma unroll
             for (int k = 0; k < TZ; ++k) {
-                const float zb = fmaf((float)k, P.rz, zbase), zt = zb + P.rz;
                 int rv0, rv1;
-                slice_rows(P, zb, zt, mmin, mmax, rv0, rv1);
-                rv0 = max(rv0, rlo_lim);
-                rv1 = min(rv1, rhi_lim);
+                slices.rows(k, smin, smax, rlo_lim, rhi_lim, rv0, rv1);
                 float a_k = 0.0f;
-                for (int r = rv0; r <= rv1; ++r) {
-                    float zl, zh;
-                    if (fits) {
-                        const float2 zz = ztab[(r - f.y) * TZ + k];
-                        zl = zz.x;
-                        zh = zz.y;
-                    } else {
-                        slab_interval(zb, P.rz, P.adj_invxi[r], zl, zh);
-                    }
-                    if (fits) {
-                        const float *sy = yd + (r - f.y) * WP + (cb - f.x);
+                if (fits) {
+                    // two rows an iteration, the second at immediate offsets
+                    const float2 *zt = ztab + (rv0 - f.y) * TZ + k, *zend = ztab + (rv1 - f.y) * TZ + k;
+                    const float *sy = yd + (rv0 - f.y) * WP + (cb - f.x);
+                    auto row = [&](const float2 *z, const float *y) {
+                        const float2 zz = *z;
 #pragma unroll
-                        for (int q = 0; q < CM; ++q) {
-                            const float len = overlap(zl, zh, clo[q], chi[q]);
-                            a_k = fmaf(len, sy[q], a_k);
-                        }
-                    } else {
+                        for (int q = 0; q < CM; ++q) a_k = fmaf(overlap(zz.x, zz.y, clo[q], chi[q]), y[q], a_k);
+                    };
+                    for (; zt <= zend; zt += 2 * TZ, sy += 2 * WP) {
+                        row(zt, sy);
+                        if (zt < zend) row(zt + TZ, sy + WP);
+                    }
+                } else {
+                    const float zb = fmaf((float)k, P.rz, zbase);
+                    for (int r = rv0; r <= rv1; ++r) {
+                        float zl, zh;
+                        slab_interval(zb, P.rz, P.adj_invxi[r], zl, zh);
 #pragma unroll
                         for (int q = 0; q < CM; ++q) {
                             const float len = overlap(zl, zh, clo[q], chi[q]);
