@@ -599,14 +599,14 @@ ctr_status ensure_footprints(ctr_ctx *ctx, const BpParams &P, FootCache &fc, boo
 }
 
 // The [z][t][s] copy of a volume for the forward projector (its views along t
-// read it), unless the geometry's tuning turned that layout off.
+// read it), unless the geometry's tuning turned that layout off; with `columns`
+// the z-fastest copy of the projector by detector columns where that is faster.
 ctr_status fp_transposed(ctr_ctx *ctx, RayParams &R, const float *vol, DevBuf &buf, hipStream_t st,
-                         bool enable = true, bool residual = false)
+                         bool enable = true, bool columns = false)
 {
     R.volT = nullptr;
     ColumnPlan L;
-    if (column_plan(R, residual, L)) {
-        // the projector by detector columns: a z-fastest copy and the lists of its cells
+    if (columns && column_plan(R, L)) {
         TRY(buf_reserve(ctx, buf, L.vol_bytes));
         TRY(buf_reserve(ctx, ctx->ws[kWsCells], L.list_bytes));
         TRY(check_launch(ctx, launch_z_fastest(vol, (float *)buf.ptr, R.nt, R.ns, R.nz, st), "volume transpose"));
@@ -1467,7 +1467,7 @@ ctr_status ctr_cone_fp(ctr_ctx *ctx, const ctr_cone_geom *g, const float *vol, f
     TRY(stage_in(ctx, dev, kWsIn, vol, nvox3(g), &dv));
     TRY(stage_out(ctx, dev, false, kWsOut, proj, nray3(g), &dp));
     RayParams R = cone_ray_params(ctx, g);
-    TRY(fp_transposed(ctx, R, dv, ctx->ws[kWsT], ctx->stream, tuning_for(ctx, ctx->cone.key).fp_transpose));
+    TRY(fp_transposed(ctx, R, dv, ctx->ws[kWsT], ctx->stream, tuning_for(ctx, ctx->cone.key).fp_transpose, true));
     TRY(check_launch(ctx, launch_ray_fp(R, dv, dp, ctx->stream), "cone forward projection"));
     return finish_out(ctx, dev, dp, proj, nray3(g));
 }
@@ -2151,7 +2151,7 @@ ctr_status ctr_sirt3d(ctr_ctx *ctx, const ctr_cone_geom *g, const float *b, floa
     const bool use_t = tuning_for(ctx, ctx->cone.key).fp_transpose;
     auto fp = [&](const float *xx, const float *bb, float *rr, double *part, int *nblk) {
         RayParams Rx = R;
-        TRY(fp_transposed(ctx, Rx, xx, ctx->ws[kWsT], ctx->stream, use_t, true));
+        TRY(fp_transposed(ctx, Rx, xx, ctx->ws[kWsT], ctx->stream, use_t));
         return check_launch(ctx, launch_ray_fp_residual(Rx, xx, bb, rr, part, nblk, ctx->stream), "SIRT residual");
     };
     auto ones = [&](float *vinv) {
@@ -2599,7 +2599,7 @@ ctr_status ctr_sirt3d_step(ctr_ctx *ctx, const ctr_cone_geom *g, const float *b_
     }));
     int nblk = 0;
     RayParams Rx = R;
-    TRY(fp_transposed(ctx, Rx, x, ctx->ws[kWsT], st, tuning_for(ctx, ctx->cone.key).fp_transpose, true));
+    TRY(fp_transposed(ctx, Rx, x, ctx->ws[kWsT], st, tuning_for(ctx, ctx->cone.key).fp_transpose));
     TRY(check_launch(ctx, launch_ray_fp_residual(Rx, x, b, r, part, &nblk, st), "SIRT residual"));
     TRY(check_launch(ctx, launch_adjoint(P, AL, AF, r, gb, nullptr, 0, st), "SIRT gradient"));
     TRY(check_launch(ctx, launch_sirt_step(vinv, gb, lambda, nvox, s, st), "SIRT step"));
@@ -2671,7 +2671,7 @@ ctr_status ctr_learned_sirt3d(ctr_ctx *ctx, const ctr_cone_geom *g, const float 
     auto residual_into = [&](const float *xx, float *rr, double *res) -> ctr_status {
         int nblk = 0;
         RayParams Rx = R;
-        TRY(fp_transposed(ctx, Rx, xx, ctx->ws[kWsT], st, tuning_for(ctx, ctx->cone.key).fp_transpose, true));
+        TRY(fp_transposed(ctx, Rx, xx, ctx->ws[kWsT], st, tuning_for(ctx, ctx->cone.key).fp_transpose));
         TRY(check_launch(ctx, launch_ray_fp_residual(Rx, xx, b, rr, part, &nblk, st), "SIRT residual"));
         TRY(check_launch(ctx, launch_reduce_partials(part, nblk, sums, st), "reduce"));
         double hh[2];
@@ -2841,7 +2841,7 @@ ctr_status ctr_sirt3d_emulated(ctr_ctx *ctx, const ctr_cone_geom *g, const float
     auto residual = [&](const float *xx, const float *bb, double *res) -> ctr_status {
         int nblk = 0;
         RayParams Rx = R;
-        TRY(fp_transposed(ctx, Rx, xx, ctx->ws[kWsT], st, fpT, true));
+        TRY(fp_transposed(ctx, Rx, xx, ctx->ws[kWsT], st, fpT));
         TRY(check_launch(ctx, launch_ray_fp_residual(Rx, xx, bb, r, part, &nblk, st), "SIRT residual"));
         if (!res) return CTR_OK;
         TRY(check_launch(ctx, launch_reduce_partials(part, nblk, sums, st), "reduce"));
@@ -2941,7 +2941,6 @@ struct BatchProblem {
     const float *bp = nullptr;
     float *xp = nullptr;
     int fp_blocks = 0, gx = 0, gy = 0;
-    ColumnPlan C{};          // C.views > 0: the projector by detector columns
 };
 
 void free_batch_problem(BatchProblem &q)
@@ -2956,7 +2955,6 @@ struct BatchRun {
     ctr_ctx *ctx;
     std::vector<BatchProblem> probs;
     DevBuf fp_jobs, red_jobs, adj_jobs, adj_ones_jobs, sums, norms, iter;
-    std::vector<DevBuf> cells;     // cell lists of the projector by detector columns, one per stream
     hipStream_t cs = nullptr;
     hipEvent_t ev = nullptr;
     std::vector<hipStream_t> ws;   // streams of the per-problem launches (joined into cs)
@@ -2980,7 +2978,6 @@ struct BatchRun {
         (void)hipStreamSynchronize(ctx->stream);
         for (auto &q : probs) free_batch_problem(q);
         for (DevBuf *b : {&fp_jobs, &red_jobs, &adj_jobs, &adj_ones_jobs, &sums, &norms, &iter}) buf_free(*b);
-        for (DevBuf &b : cells) buf_free(b);
     }
 };
 
@@ -3009,29 +3006,6 @@ ctr_status ctr_sirt3d_batched(ctr_ctx *ctx, const ctr_sirt_problem *pr, int n, c
     std::vector<int> group_blocks(3, 0), group_max(3, 0), group_cm(3, 4), group_fit(3, 1);
     const int pitches[3] = {40, 72, 136};
     int fp_total = 0, fp_max = 0;
-    // CTR_BATCH_STREAMS = K > 0 (default 4): each problem runs its own
-    // single-problem kernels (its tuned adjoint variant) on stream p mod K,
-    // forked from and joined into the iteration's stream, so that problems
-    // overlap; 0: the job-table kernels, one launch per phase for all problems.
-    int nstreams = 4;
-    if (const char *e = std::getenv("CTR_BATCH_STREAMS")) nstreams = std::max(0, std::atoi(e));
-    nstreams = std::min(nstreams, n);
-    // problems of one stream follow each other: they share its cell lists
-    B.cells.resize(std::max(nstreams, 1));
-    for (int p = 0; p < n; ++p) {
-        const ctr_cone_geom *g = &pr[p].geom;
-        RayParams R{};
-        R.nt = g->nt;
-        R.ns = g->ns;
-        R.nz = g->nz;
-        R.np = g->n_p;
-        R.nx = g->n_xi;
-        R.nb = g->n_beta;
-        ColumnPlan C;
-        if (!column_plan(R, true, C)) continue;
-        B.probs[p].C = C;
-        TRY(buf_reserve(ctx, B.cells[nstreams ? p % nstreams : 0], C.list_bytes));
-    }
     for (int p = 0; p < n; ++p) {
         BatchProblem &q = B.probs[p];
         const ctr_cone_geom *g = &pr[p].geom;
@@ -3054,18 +3028,15 @@ ctr_status ctr_sirt3d_batched(ctr_ctx *ctx, const ctr_sirt_problem *pr, int n, c
         }
         TRY(buf_reserve(ctx, q.r, q.nray * sizeof(float)));
         TRY(buf_reserve(ctx, q.vinv, q.nvox * sizeof(float)));
-        if (q.C.views > 0) {
-            TRY(buf_reserve(ctx, q.vt, q.C.vol_bytes));
-            column_bind(q.R, q.C, (float *)q.vt.ptr, B.cells[nstreams ? p % nstreams : 0].ptr);
-        } else if (tuning_for(ctx, q.T.key).fp_transpose) {
+        if (tuning_for(ctx, q.T.key).fp_transpose) {
             TRY(buf_reserve(ctx, q.vt, q.nvox * sizeof(float)));
             q.R.volT = (const float *)q.vt.ptr;   // refreshed from x before every residual pass
         }
         q.fp_blocks = fp_job_blocks(q.R, &q.gx, &q.gy);
         TRY(buf_reserve(ctx, q.part, sizeof(double) * 2 * ((size_t)std::max(q.fp_blocks, 4096) + kReduceSlack)));
         fj[p] = FpJob{q.R, q.xp, q.bp, (float *)q.r.ptr, (double *)q.part.ptr, fp_total, q.gx, q.gy};
-        fp_total += q.gx * q.gy * q.R.nb;
-        fp_max = std::max(fp_max, q.gx * q.gy * q.R.nb);
+        fp_total += q.fp_blocks;
+        fp_max = std::max(fp_max, q.fp_blocks);
         rj[p] = ReduceJob{(const double *)q.part.ptr, q.fp_blocks};
         const BpPlan &L = q.F.plan;
         BpParams P = q.P;
@@ -3131,6 +3102,13 @@ ctr_status ctr_sirt3d_batched(ctr_ctx *ctx, const ctr_sirt_problem *pr, int n, c
     HIP_TRY(ctx, hipEventCreateWithFlags(&B.ev, hipEventDisableTiming));
     HIP_TRY(ctx, hipEventRecord(B.ev, st));
     HIP_TRY(ctx, hipStreamWaitEvent(B.cs, B.ev, 0));
+    // CTR_BATCH_STREAMS = K > 0 (default 4): each problem runs its own
+    // single-problem kernels (its tuned adjoint variant) on stream p mod K,
+    // forked from and joined into the iteration's stream, so that problems
+    // overlap; 0: the job-table kernels, one launch per phase for all problems.
+    int nstreams = 4;
+    if (const char *e = std::getenv("CTR_BATCH_STREAMS")) nstreams = std::max(0, std::atoi(e));
+    nstreams = std::min(nstreams, n);
     for (int j = 0; j < nstreams; ++j) {
         B.ws.push_back(nullptr);
         HIP_TRY(ctx, hipStreamCreateWithFlags(&B.ws.back(), hipStreamNonBlocking));
@@ -3142,16 +3120,6 @@ ctr_status ctr_sirt3d_batched(ctr_ctx *ctx, const ctr_sirt_problem *pr, int n, c
     // residual sums: slot k of problem p at 2 (p nslots + k) with streams,
     // at 2 (k n + p) with the job-table reduction
     auto sum_index = [&](int p, size_t k) { return nstreams ? 2 * ((size_t)p * nslots + k) : 2 * (k * n + p); };
-    // the copy of a problem's iterate that its projector reads
-    auto volume_copy = [&](const BatchProblem &q, hipStream_t s) -> ctr_status {
-        if (q.R.volZ)
-            return check_launch(ctx, launch_z_fastest(q.xp, (float *)q.vt.ptr, q.R.nt, q.R.ns, q.R.nz, s),
-                                "volume transpose");
-        if (q.R.volT)
-            return check_launch(ctx, launch_transpose_st(q.xp, (float *)q.vt.ptr, nullptr, q.R.nt, q.R.ns, q.R.nz, s),
-                                "volume transpose");
-        return CTR_OK;
-    };
     auto iteration = [&](hipStream_t s, bool update) -> ctr_status {
         if (nstreams) {
             HIP_TRY(ctx, hipEventRecord(B.wev[nstreams], s));
@@ -3159,7 +3127,9 @@ ctr_status ctr_sirt3d_batched(ctr_ctx *ctx, const ctr_sirt_problem *pr, int n, c
             for (int p = 0; p < n; ++p) {
                 const BatchProblem &q = B.probs[p];
                 hipStream_t t = B.ws[p % nstreams];
-                TRY(volume_copy(q, t));
+                if (q.R.volT)
+                    TRY(check_launch(ctx, launch_transpose_st(q.xp, (float *)q.vt.ptr, nullptr, q.R.nt, q.R.ns, q.R.nz, t),
+                                     "volume transpose"));
                 int nblk = 0;
                 TRY(check_launch(ctx, launch_ray_fp_residual(q.R, q.xp, q.bp, (float *)q.r.ptr, (double *)q.part.ptr,
                                                              &nblk, t), "residual"));
@@ -3177,14 +3147,11 @@ ctr_status ctr_sirt3d_batched(ctr_ctx *ctx, const ctr_sirt_problem *pr, int n, c
         } else {
             for (int p = 0; p < n; ++p) {
                 const BatchProblem &q = B.probs[p];
-                TRY(volume_copy(q, s));
-                int nblk = 0;
-                if (q.R.volZ)
-                    TRY(check_launch(ctx, launch_ray_fp_residual(q.R, q.xp, q.bp, (float *)q.r.ptr,
-                                                                 (double *)q.part.ptr, &nblk, s), "residual"));
+                if (q.R.volT)
+                    TRY(check_launch(ctx, launch_transpose_st(q.xp, (float *)q.vt.ptr, nullptr, q.R.nt, q.R.ns, q.R.nz, s),
+                                     "volume transpose"));
             }
-            if (fp_max > 0)
-                TRY(check_launch(ctx, launch_ray_fp_residual_batched(dfp, n, fp_max, s), "batched residual"));
+            TRY(check_launch(ctx, launch_ray_fp_residual_batched(dfp, n, fp_max, s), "batched residual"));
             TRY(check_launch(ctx, launch_reduce_jobs(drj, n, diter, dsums, s), "batched reduce"));
             if (update)
                 for (int gi = 0; gi < 3; ++gi)

@@ -242,14 +242,13 @@ hipError_t scan_counts(const long long *counts, long long *out, int n, void *tmp
 hipError_t launch_ray_fp_residual(const RayParams &g, const float *vol, const float *b, float *r,
                                   double *partials, int *nblocks, hipStream_t st);
 int ray_fp_blocks(const RayParams &g);
-// Whether the cone projection (residual: the SIRT residual pass) runs by
-// detector columns, and the sizes of its volume copy and list workspace;
-// column_bind points g at them.
+// Whether the cone projection runs by detector columns, and the sizes of its
+// volume copy and list workspace; column_bind points g at them.
 struct ColumnPlan {
     int stride, views;
     size_t vol_bytes, list_bytes;
 };
-bool column_plan(const RayParams &g, bool residual, ColumnPlan &L);
+bool column_plan(const RayParams &g, ColumnPlan &L);
 void column_bind(RayParams &g, const ColumnPlan &L, float *volz, void *lists);
 
 // Tiling of the voxel-driven backprojection and its per-(tile, view) detector

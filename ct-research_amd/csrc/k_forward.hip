@@ -911,13 +911,12 @@ __device__ __forceinline__ float column_sum(__amdgpu_buffer_rsrc_t rs, const Col
 }
 
 // Line integrals of the 64 rows of a wavefront through the cells of detector
-// column `col`; chord is the row's length in the volume box.
+// column `col`.
 __device__ __forceinline__ float trace_column(const RayParams &g, const ColumnHead *__restrict__ heads,
                                               const ColumnBlock *__restrict__ blocks, size_t stride, size_t col, int ip,
-                                              int ix, bool valid, float &chord)
+                                              int ix, bool valid)
 {
     const ColumnHead h = heads[col];
-    chord = 0.0f;
     if (h.n == 0) return 0.0f;
     const double slope = g.xi[valid ? ix : g.nx - 1] * h.inv_rho;   // z per in-plane length
     // first slice, next plane and the step between planes
@@ -930,9 +929,8 @@ __device__ __forceinline__ float trace_column(const RayParams &g, const ColumnHe
         dz = g.rz * fabs(inv_s);
         out = (slope > 0.0 ? g.bz - g.sz : -g.sz) * inv_s - h.lo;
     }
-    const double norm = sqrt(fma(slope, slope, 1.0)), length = fmin(h.len, out);
-    const bool hit = length > 0.0;
-    chord = hit ? (float)(length * norm) : 0.0f;
+    const double norm = sqrt(fma(slope, slope, 1.0));
+    const bool hit = fmin(h.len, out) > 0.0;
     const float Z0 = (float)z0, dZ = (float)dz;
     const int top = 4 * (g.nz + 1);   // slices 0 and nz + 1 of the copy are zeros
     const int zb = (int)fmin(fmax(4.0 * (k0 + 1.0), 0.0), (double)top), sgn = slope > 0.0 ? 4 : -4;
@@ -1012,62 +1010,27 @@ __device__ __forceinline__ ColumnTile column_tile(const RayParams &g, int views)
                       rest / tv * 64};
 }
 
-// kResidual: the SIRT residual pass (fp_residual_block) instead of the projection.
-template <bool kResidual>
-__global__ __launch_bounds__(64 * kColWaves, 8) void k_ray_columns(const float *__restrict__ b, float *__restrict__ out,
-                                                                double *__restrict__ partials,
+__global__ __launch_bounds__(64 * kColWaves, 8) void k_ray_columns(float *__restrict__ out,
                                                                 const ColumnHead *__restrict__ heads,
                                                                 const ColumnBlock *__restrict__ blocks, RayParams g,
                                                                 int stride, int view0, int views)
 {
-    __shared__ float sums[kColWaves][65], chords[kColWaves][65];
-    __shared__ double red[2][kColWaves];
+    __shared__ float sums[kColWaves][65];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const ColumnTile B = column_tile(g, views);
     const int ip = B.p0 + wave;
-    float chord = 0.0f, acc = 0.0f;
+    float acc = 0.0f;
     const bool there = B.p0 < g.np && B.v < views && B.row0 < g.nx;
     if (there && ip < g.np) {
         const int ix = B.row0 + lane;
-        acc = trace_column(g, heads, blocks, stride, (size_t)B.v * g.np + ip, ip, ix, ix < g.nx, chord);
+        acc = trace_column(g, heads, blocks, stride, (size_t)B.v * g.np + ip, ip, ix, ix < g.nx);
     }
     // the block's 64 x 4 results, four neighbouring columns of a row per four threads
     sums[wave][lane] = acc;
-    if (kResidual) chords[wave][lane] = chord;
     __syncthreads();
     const int c = threadIdx.x % kColWaves, r = threadIdx.x / kColWaves;
     const int oc = B.p0 + c, orow = B.row0 + r;
-    double e2 = 0.0, e1 = 0.0;
-    if (there && oc < g.np && orow < g.nx) {
-        const size_t ray = ((size_t)(view0 + B.v) * g.nx + orow) * g.np + oc;
-        if (kResidual) {
-            const float e = b[ray] - sums[c][r];
-            const float rr = e / (chords[c][r] + 1e-9f);
-            out[ray] = g.residual_norm ? rr * ray_norm((float)g.p[oc], (float)g.xi[orow], (float)g.D) : rr;
-            e2 = (double)e * (double)e;
-            e1 = fabs((double)e);
-        } else {
-            out[ray] = sums[c][r];
-        }
-    }
-    if (kResidual) {
-        e2 = wave_sum(e2);
-        e1 = wave_sum(e1);
-        if (lane == 0) {
-            red[0][wave] = e2;
-            red[1][wave] = e1;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double s2 = 0.0, s1 = 0.0;
-            for (int w = 0; w < kColWaves; ++w) {
-                s2 += red[0][w];
-                s1 += red[1][w];
-            }
-            partials[2 * (size_t)blockIdx.x] = s2;
-            partials[2 * (size_t)blockIdx.x + 1] = s1;
-        }
-    }
+    if (there && oc < g.np && orow < g.nx) out[((size_t)(view0 + B.v) * g.nx + orow) * g.np + oc] = sums[c][r];
 }
 
 int column_blocks(const RayParams &g, int views)
@@ -1077,22 +1040,17 @@ int column_blocks(const RayParams &g, int views)
 }
 
 // Lists of C.views views at a time, then their rays.
-template <bool kResidual>
-hipError_t launch_columns(const RayParams &g, const float *b, float *out, double *partials, int *nblocks, hipStream_t st)
+hipError_t launch_columns(const RayParams &g, float *out, hipStream_t st)
 {
     const ColumnLists &C = g.cols;
-    int blocks = 0;
     for (int v0 = 0; v0 < g.nb; v0 += C.views) {
         const int views = g.nb - v0 < C.views ? g.nb - v0 : C.views, n = column_blocks(g, views);
         hipLaunchKernelGGL(k_ray_cells, dim3(g.np, views), dim3(64), (2 * C.stride + 1) * sizeof(float), st, g, C, v0);
-        hipLaunchKernelGGL(k_ray_columns<kResidual>, dim3((unsigned)n), dim3(64 * kColWaves), 0, st, b, out,
-                           partials ? partials + 2 * (size_t)blocks : nullptr, C.head, C.blocks, g, C.stride / kColBlock, v0,
-                           views);
+        hipLaunchKernelGGL(k_ray_columns, dim3((unsigned)n), dim3(64 * kColWaves), 0, st, out, C.head, C.blocks, g,
+                           C.stride / kColBlock, v0, views);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        blocks += n;
     }
-    if (nblocks) *nblocks = blocks;
     return hipSuccess;
 }
 
@@ -1117,23 +1075,21 @@ constexpr size_t kColListBytes = (size_t)256 << 20;
 //   128^3, 180 x 192 x 192     608 /  400      50 slices, 180 x 192 x 72    226 /  267
 //    70 slices, 120 x 300 x 100 509 / 397      28 slices, 180 x 192 x 40    125 /  170
 //    64^3, 90 x 96 x 96 (17k wavefronts) 81 / 76,   60 x 52 x 44, 45 x 96 x 80 (9k) 42 / 53
-// The residual pass of SIRT has a second line: its history of residual norms
-// averages the rounding of all rays, which for fewer than 2^22 of them differs
-// between the two kernels by more than 1e-9 of the norm (4e-10 at 3e5 rays a
-// view, 2e-9 at 20000).
-static bool column_use(const RayParams &g, bool residual)
+// The residual pass of SIRT keeps the slab walk: the history of its norms, in 64
+// bits, shows the rounding of the walk's chain of sums (1e-9 to 1e-8 of a norm,
+// also for 2e7 rays), and a problem's history is not to depend on the kernel.
+static bool column_use(const RayParams &g)
 {
     if (const char *e = std::getenv("CTR_FP_COLUMNS")) return std::atoi(e) != 0;
     const size_t chunks = (g.nx + 63) / 64, waves = (size_t)g.nb * g.np * chunks;
-    if (residual && (size_t)g.nb * g.np * g.nx < ((size_t)1 << 22)) return false;
     return 10 * (size_t)g.nx >= 7 * 64 * chunks && waves >= 12000;
 }
 
-bool column_plan(const RayParams &g, bool residual, ColumnPlan &L)
+bool column_plan(const RayParams &g, ColumnPlan &L)
 {
     // 32-bit offsets into the z-fastest copy, one workgroup row per view in the list kernel
     if (g.parallel || (size_t)g.nt * g.ns * (g.nz + 2) > ((size_t)1 << 30)) return false;
-    if (!column_use(g, residual)) return false;
+    if (!column_use(g)) return false;
     L.stride = (g.nt + g.ns + 1 + 2 * kColBlock - 1) / (2 * kColBlock) * (2 * kColBlock) + kColBlock;
     if (L.stride > 4096) return false;   // the list kernel's LDS
     const size_t per_view = (size_t)g.np * (L.stride / kColBlock * sizeof(ColumnBlock) + sizeof(ColumnHead));
@@ -1156,9 +1112,8 @@ void column_bind(RayParams &g, const ColumnPlan &L, float *volz, void *lists)
 int ray_fp_blocks(const RayParams &g)
 {
     if (g.flat) return (int)flat_blocks(g);
-    // of either kernel: a caller sizes the partial sums before the plan is bound
     const dim3 grid = fp_grid(g);
-    return std::max((int)(grid.x * grid.y * grid.z), kColTileV * column_blocks(g, g.nb));
+    return (int)(grid.x * grid.y * grid.z);
 }
 
 hipError_t launch_sysmat_count(const RayParams &g, long long *counts, hipStream_t st)
@@ -1177,7 +1132,7 @@ hipError_t launch_sysmat_fill(const RayParams &g, const long long *row_ptr, int 
 
 hipError_t launch_ray_fp(const RayParams &g, const float *vol, float *proj, hipStream_t st)
 {
-    if (g.volZ) return launch_columns<false>(g, nullptr, proj, nullptr, nullptr, st);
+    if (g.volZ) return launch_columns(g, proj, st);
     if (g.flat) {
         hipLaunchKernelGGL(k_ray_fp_flat, dim3(flat_blocks(g)), dim3(64, kFlatWaves), 0, st, proj, g);
         return hipGetLastError();
@@ -1189,7 +1144,6 @@ hipError_t launch_ray_fp(const RayParams &g, const float *vol, float *proj, hipS
 hipError_t launch_ray_fp_residual(const RayParams &g, const float *vol, const float *b, float *r, double *partials,
                                   int *nblocks, hipStream_t st)
 {
-    if (g.volZ) return launch_columns<true>(g, b, r, partials, nblocks, st);
     if (g.flat) {
         *nblocks = (int)flat_blocks(g);
         hipLaunchKernelGGL(k_ray_fp_residual_flat, dim3(flat_blocks(g)), dim3(64, kFlatWaves), 0, st, b, r, partials, g);
@@ -1203,12 +1157,6 @@ hipError_t launch_ray_fp_residual(const RayParams &g, const float *vol, const fl
 
 int fp_job_blocks(const RayParams &g, int *gx, int *gy)
 {
-    if (g.volZ) {   // not in the job table: its own launches' partial sums
-        *gx = *gy = 0;
-        int blocks = 0;
-        for (int v0 = 0; v0 < g.nb; v0 += g.cols.views) blocks += column_blocks(g, std::min(g.nb - v0, g.cols.views));
-        return blocks;
-    }
     const dim3 grid = fp_grid(g);
     *gx = (int)grid.x;
     *gy = (int)grid.y;

@@ -63,23 +63,15 @@ def test_column_projector_of_ones(ctx, oracle, columns):
     assert e < 2e-7 and m < 1e-6
 
 
-@pytest.mark.parametrize("streams", ["0", "2"])
-def test_column_residual(ctx, monkeypatch, streams):
-    """SIRT on the columns' residual pass: the slab walk's iterates to the
-    rounding of the ray sums, and the batched forms' bits."""
+def test_columns_leave_sirt_alone(ctx, monkeypatch):
+    """The residual pass of SIRT keeps the slab walk, whose rounding its residual
+    history shows: iterates and history do not depend on the projector's kernel."""
     import ctr
     g = _geom("rows130", ctr.ConeGeom)
     vol = np.random.default_rng(4).random(g.nvox).astype(np.float32)
     monkeypatch.setenv("CTR_FP_COLUMNS", "0")
     b = ctx.cone_fp(g, vol)
-    x0, r0, s0 = ctx.sirt3d(g, b, 4)
+    x0, r0, s0 = ctx.sirt3d(g, b, 2)
     monkeypatch.setenv("CTR_FP_COLUMNS", "1")
-    monkeypatch.setenv("CTR_BATCH_STREAMS", streams)
-    x1, r1, s1 = ctx.sirt3d(g, b, 4)
-    e, m = errs(x1, x0)
-    report("column residual", rel_l2=e, max_rel=m, dres=float(np.abs(r1 - r0).max()))
-    # two float sums of about 100 segments per ray, four iterations
-    assert e < 5e-6 and m < 5e-5 and np.abs(r1 - r0).max() < 1e-6
-    xs, rs = ctx.sirt3d_batched([(g, b), (g, b)], 4)
-    for x, r in zip(xs, rs):
-        assert np.array_equal(x, x1) and np.abs(r - r1).max() < 1e-12
+    x1, r1, s1 = ctx.sirt3d(g, b, 2)
+    assert np.array_equal(x1, x0) and np.array_equal(r1, r0) and np.array_equal(s1, s0)
