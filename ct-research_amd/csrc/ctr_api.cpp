@@ -489,10 +489,9 @@ RayParams cone_ray_params_from(const ConeTables &T, const ctr_cone_geom *g)
     r.p = (const double *)T.d_p.ptr;
     r.xi = (const double *)T.d_xi.ptr;
     r.residual_norm = 1;
-    // masked second/third voxel reads once the volume exceeds the 256 MiB
-    // Infinity Cache (measured: 512^3 301 -> 270 ms, 256^3 19.3 -> 20.4 ms);
-    // CTR_FP_SKIP=0/1 overrides
-    r.skip_empty = (size_t)g->nt * g->ns * g->nz * sizeof(float) > ((size_t)256 << 20);
+    // masked second/third voxel reads and slabs in blocks from 2^19 voxels on
+    // (trace_ray); CTR_FP_SKIP=0/1 overrides
+    r.skip_empty = (size_t)g->nt * g->ns * g->nz >= ((size_t)1 << 19);
     if (const char *e = std::getenv("CTR_FP_SKIP")) r.skip_empty = std::atoi(e) != 0;
     return r;
 }
@@ -599,14 +598,15 @@ ctr_status ensure_footprints(ctr_ctx *ctx, const BpParams &P, FootCache &fc, boo
 }
 
 // The [z][t][s] copy of a volume for the forward projector (its views along t
-// read it), unless the geometry's tuning turned that layout off; with `columns`
-// the z-fastest copy of the projector by detector columns where that is faster.
+// read it), unless the geometry's tuning turned that layout off; with a row
+// pitch (mm at the isocentre) the z-fastest copy of the projector by detector
+// columns where that is faster.
 ctr_status fp_transposed(ctr_ctx *ctx, RayParams &R, const float *vol, DevBuf &buf, hipStream_t st,
-                         bool enable = true, bool columns = false)
+                         bool enable = true, double row_pitch = 0.0)
 {
     R.volT = nullptr;
     ColumnPlan L;
-    if (columns && column_plan(R, L)) {
+    if (row_pitch > 0.0 && column_plan(R, row_pitch, L)) {
         TRY(buf_reserve(ctx, buf, L.vol_bytes));
         TRY(buf_reserve(ctx, ctx->ws[kWsCells], L.list_bytes));
         TRY(check_launch(ctx, launch_z_fastest(vol, (float *)buf.ptr, R.nt, R.ns, R.nz, st), "volume transpose"));
@@ -1467,7 +1467,8 @@ ctr_status ctr_cone_fp(ctr_ctx *ctx, const ctr_cone_geom *g, const float *vol, f
     TRY(stage_in(ctx, dev, kWsIn, vol, nvox3(g), &dv));
     TRY(stage_out(ctx, dev, false, kWsOut, proj, nray3(g), &dp));
     RayParams R = cone_ray_params(ctx, g);
-    TRY(fp_transposed(ctx, R, dv, ctx->ws[kWsT], ctx->stream, tuning_for(ctx, ctx->cone.key).fp_transpose, true));
+    const double row_pitch = std::fabs((double)g->xi[g->n_xi - 1] - (double)g->xi[0]) / std::max(g->n_xi - 1, 1);
+    TRY(fp_transposed(ctx, R, dv, ctx->ws[kWsT], ctx->stream, tuning_for(ctx, ctx->cone.key).fp_transpose, row_pitch));
     TRY(check_launch(ctx, launch_ray_fp(R, dv, dp, ctx->stream), "cone forward projection"));
     return finish_out(ctx, dev, dp, proj, nray3(g));
 }

@@ -58,8 +58,7 @@ struct RayParams {
     int residual_norm;      // the SIRT residual pass stores r times the ray norm (the cone
                             // adjoint's input form); the fan adjoint reads r itself
     int skip_empty;         // a slab's second and third voxels are read only by lanes whose
-                            // segment in them is not empty (pays once the volume outgrows the
-                            // Infinity Cache; costs instructions below that)
+                            // segment in them is not empty, and slabs are taken in blocks
 };
 
 // Per-view constants of the voxel-driven backprojectors, float:
@@ -248,7 +247,7 @@ struct ColumnPlan {
     int stride, views;
     size_t vol_bytes, list_bytes;
 };
-bool column_plan(const RayParams &g, ColumnPlan &L);
+bool column_plan(const RayParams &g, double row_pitch, ColumnPlan &L);
 void column_bind(RayParams &g, const ColumnPlan &L, float *volz, void *lists);
 
 // Tiling of the voxel-driven backprojection and its per-(tile, view) detector
