@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <complex>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -1022,6 +1023,28 @@ ctr_status curved_footprints(ctr_ctx *ctx, CurvedBpParams &P)
     return CTR_OK;
 }
 
+// Forward transform of a power-of-two length (radix 2, decimation in time).
+void fft_in_place(std::vector<std::complex<long double>> &c)
+{
+    const size_t L = c.size();
+    for (size_t i = 1, j = 0; i < L; ++i) {
+        size_t bit = L >> 1;
+        for (; j & bit; bit >>= 1) j ^= bit;
+        j |= bit;
+        if (i < j) std::swap(c[i], c[j]);
+    }
+    for (size_t len = 2; len <= L; len *= 2) {
+        std::vector<std::complex<long double>> w(len / 2);
+        for (size_t k = 0; k < len / 2; ++k) w[k] = std::polar(1.0L, -2.0L * 3.14159265358979323846264L * k / len);
+        for (size_t i = 0; i < L; i += len)
+            for (size_t k = 0; k < len / 2; ++k) {
+                const std::complex<long double> a = c[i + k], b = c[i + k + len / 2] * w[k];
+                c[i + k] = a + b;
+                c[i + k + len / 2] = a - b;
+            }
+    }
+}
+
 // Half-scaled ramp taps times the pitch, two-sided: h2[k] = d * h[|k-(n-1)|].
 ctr_status tap_table(ctr_ctx *ctx, int filter, int equiangular, double d, int n)
 {
@@ -1059,16 +1082,24 @@ ctr_status tap_table(ctr_ctx *ctx, int filter, int equiangular, double d, int n)
     if (s != CTR_OK) return s;
     // spectrum of the circular kernel c[m] = c[L-m] = h[m] (m < n) for the FFT
     // path: H[k] = h[0] + 2 sum_m h[m] cos(2 pi k m / L), real because c is even
-    T.fft_len = fft_filter_length(n);
+    T.fft_len = fft_flat_length(n);
     if (T.fft_len) {
         const int L = T.fft_len;
         std::vector<double> cosL(L);
         for (int i = 0; i < L; ++i) cosL[i] = std::cos(2.0 * pi * i / L);
         T.spec.assign(L, 0.0);
-        for (int k = 0; k < L; ++k) {
-            long double acc = h[0];
-            for (int m = 1; m < n; ++m) acc += 2.0L * h[m] * cosL[((long)k * m) % L];
-            T.spec[k] = (double)(acc / L);
+        if (L <= 2048) {
+            for (int k = 0; k < L; ++k) {
+                long double acc = h[0];
+                for (int m = 1; m < n; ++m) acc += 2.0L * h[m] * cosL[((long)k * m) % L];
+                T.spec[k] = (double)(acc / L);
+            }
+        } else {
+            // the sums of 4096 x 2048 terms would take 30 ms
+            std::vector<std::complex<long double>> c(L);
+            for (int m = 0; m < n; ++m) c[m] = c[(L - m) % L] = h[m];
+            fft_in_place(c);
+            for (int k = 0; k < L; ++k) T.spec[k] = (double)(c[k].real() / L);
         }
         s = upload(ctx, T.d_spec, T.spec.data(), sizeof(double) * L);
         if (s != CTR_OK) return s;

@@ -335,6 +335,7 @@ hipError_t launch_row_filter(const FilterParams &P, const float *in, float *out,
 hipError_t launch_cone_weights(double D, const float *pd, const float *xd, int np, int nx, double *pw, hipStream_t st);
 // transform length of the FFT filter path for np columns (0: direct convolution)
 int fft_filter_length(int np);
+int fft_flat_length(int np);
 // Restricted Chebyshev emulation of SIRT: mask = v > thr; out = a * m; the
 // masked plain step w0 = mask lambda V g with acc = c0 w0; one recurrence
 // term w_{j+1} = mask (2 (2M - I) w_j - w_{j-1}) (first: mask (2M - I) w_0)
