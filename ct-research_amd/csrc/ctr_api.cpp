@@ -28,6 +28,8 @@ thread_local std::string g_last_error;
 // before the context is looked at) happened on the thread.
 thread_local unsigned long long g_error_seq = 0;
 
+constexpr size_t kFlatAlone = 1 << 14;   // pixels that the 2-D projector reads without their transpose
+
 enum Slot { kWsIn = 0, kWsOut, kWsTmp, kWsR, kWsVinv, kWsPart, kWsSums, kWsG, kWsS, kWsD, kWsX2, kWsR2, kWsT, kWsYn,
             kWsMask, kWsXs, kWsCells, kWsBpParts, kWsCount };
 
@@ -626,10 +628,16 @@ ctr_status fp_transposed(ctr_ctx *ctx, RayParams &R, const float *vol, DevBuf &b
 // The 2-D projector's image: a copy of it followed by its transpose, so that
 // every ray of a wavefront reads along its own axis from one buffer.  Images
 // above 2^28 pixels (whose pair would pass the 32-bit offsets) keep the 3-D
-// kernel and its transposed copy.
-ctr_status fp_flat(ctr_ctx *ctx, RayParams &R, const float *img, DevBuf &buf, hipStream_t st)
+// kernel and its transposed copy.  A projection of few rays reads an image that
+// fits a CU's caches as it is, without the launch of the copy.
+ctr_status fp_flat(ctr_ctx *ctx, RayParams &R, const float *img, DevBuf &buf, hipStream_t st, bool projection = false)
 {
     const size_t n = (size_t)R.nt * R.ns;
+    if (projection && n <= kFlatAlone && flat_split(R)) {
+        R.flat = img;
+        R.flat_alone = 1;
+        return CTR_OK;
+    }
     if (n > ((size_t)1 << 28)) return fp_transposed(ctx, R, img, buf, st);
     TRY(buf_reserve(ctx, buf, 2 * n * sizeof(float)));
     float *pair = (float *)buf.ptr;
@@ -1669,7 +1677,7 @@ ctr_status ctr_fan_fp(ctr_ctx *ctx, const ctr_fan_geom *g, const float *img, flo
     TRY(stage_in(ctx, dev, kWsIn, img, nvox2(g), &di));
     TRY(stage_out(ctx, dev, false, kWsOut, proj, nray2(g), &dp));
     RayParams R = fan_ray_params(ctx, g);
-    TRY(fp_flat(ctx, R, di, ctx->ws[kWsT], ctx->stream));
+    TRY(fp_flat(ctx, R, di, ctx->ws[kWsT], ctx->stream, true));
     TRY(check_launch(ctx, launch_ray_fp(R, di, dp, ctx->stream), "fan forward projection"));
     return finish_out(ctx, dev, dp, proj, nray2(g));
 }
@@ -1765,7 +1773,7 @@ ctr_status ctr_par_fp(ctr_ctx *ctx, const ctr_par_geom *g, const float *img, flo
     TRY(stage_in(ctx, dev, kWsIn, img, npix(g), &di));
     TRY(stage_out(ctx, dev, false, kWsOut, proj, nrayp(g), &dp));
     RayParams R = par_ray_params(ctx, g);
-    TRY(fp_flat(ctx, R, di, ctx->ws[kWsT], ctx->stream));
+    TRY(fp_flat(ctx, R, di, ctx->ws[kWsT], ctx->stream, true));
     TRY(check_launch(ctx, launch_ray_fp(R, di, dp, ctx->stream), "parallel forward projection"));
     return finish_out(ctx, dev, dp, proj, nrayp(g));
 }

@@ -55,6 +55,7 @@ struct RayParams {
     ColumnLists cols;
     const float *flat;      // 2-D image (one slice, one detector row at its height: fan, parallel beam):
                             // the image [nt*ns] followed by its transpose, at most 2^29 floats together
+    int flat_alone;         // without the transpose
     int residual_norm;      // the SIRT residual pass stores r times the ray norm (the cone
                             // adjoint's input form); the fan adjoint reads r itself
     int skip_empty;         // a slab's second and third voxels are read only by lanes whose
@@ -241,6 +242,7 @@ hipError_t scan_counts(const long long *counts, long long *out, int n, void *tmp
 hipError_t launch_ray_fp_residual(const RayParams &g, const float *vol, const float *b, float *r,
                                   double *partials, int *nblocks, hipStream_t st);
 int ray_fp_blocks(const RayParams &g);
+bool flat_split(const RayParams &g);   // few 2-D rays: each walked by several wavefronts
 // Whether the cone projection runs by detector columns, and the sizes of its
 // volume copy and list workspace; column_bind points g at them.
 struct ColumnPlan {

@@ -573,20 +573,24 @@ __global__ __launch_bounds__(kBX *kBY) void k_ray_fp_residual_batched(const FpJo
 // ---------------------------------------------------------------------------
 constexpr int kFlatUnroll = 8, kFlatWaves = 4;
 
-__device__ __forceinline__ float trace_ray_flat(const RayParams &g, int ib, int ip, bool valid, float &chord)
+// Part `part` of `parts` of the ray's slabs (the whole ray: 0 of 1).
+__device__ __forceinline__ float trace_ray_flat(const RayParams &g, int ib, int ip, bool valid, float &chord, int part = 0,
+                                                int parts = 1)
 {
     RayWalk w;
     const bool go = valid && ray_walk(g, ib, ip, 0, false, w);
     chord = go ? (float)w.lam_end : 0.0f;
     if (__ballot(go) == 0) return 0.0f;
     const int npix = g.nt * g.ns;
-    __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)g.flat, 0, (int)((unsigned)npix * 8u), kBufDword3);
+    __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)g.flat, 0, (int)((unsigned)npix * (g.flat_alone ? 4u : 8u)), kBufDword3);
     const bool lane_t = w.at.stride != 0 && (w.as.stride == 0 || w.at.step <= w.as.step);
     const AxisSetup aD = lane_t ? w.at : w.as;
     const AxisSetup aA = lane_t ? w.as : w.at;
     const int sgnD = aD.stride > 0 ? 1 : -1, sgnA = aA.stride > 0 ? 1 : (aA.stride < 0 ? -1 : 0);
-    const unsigned sA = (unsigned)sgnA * 4u, sD = (unsigned)(sgnD * (lane_t ? g.ns : g.nt)) * 4u;
-    const unsigned idx0 = lane_t ? (unsigned)(npix + w.at.i0 * g.ns + w.as.i0) : (unsigned)w.idx0;
+    const bool swap = lane_t && !g.flat_alone;   // reads the transpose
+    const unsigned sA = (unsigned)(sgnA * (lane_t && g.flat_alone ? g.nt : 1)) * 4u;
+    const unsigned sD = (unsigned)(sgnD * (swap ? g.ns : (lane_t ? 1 : g.nt))) * 4u;
+    const unsigned idx0 = swap ? (unsigned)(npix + w.at.i0 * g.ns + w.as.i0) : (unsigned)w.idx0;
 
     // trace_ray's 16 neighbouring rays that do not all have the view's axis as
     // their shorter one walk crossing by crossing, with one segment behind the
@@ -625,7 +629,25 @@ __device__ __forceinline__ float trace_ray_flat(const RayParams &g, int ib, int 
     const float ninf = opaque_ninf();
     float w1[kFlatUnroll], w2[kFlatUnroll], v1[kFlatUnroll], v2[kFlatUnroll];
     unsigned o1[kFlatUnroll];
-    for (int u = 0; u <= uend; u += kFlatUnroll) {
+    int ubegin = 0, ulast = uend;
+    if (parts > 1) {
+        // this part's blocks of slabs, and the ray's state where they begin
+        const int blocks = uend / kFlatUnroll + 1;
+        ubegin = blocks * part / parts * kFlatUnroll;
+        ulast = min(uend, blocks * (part + 1) / parts * kFlatUnroll - 1);
+        const int k = ubegin - o;
+        if (go && k > 0 && k <= nD) {
+            s = min_nc(fmaf((float)(k - 1), dD, D0), lend, ninf);
+            if (pA < s) {   // crossings before s: a guess, and its neighbours by the walk's own comparison
+                cA = fminf(fmaxf(ceilf((s - A0) / dA), 0.0f), (float)aA.n);
+                if (cA > 0.0f && fmaf(cA - 1.0f, dA, A0) >= s) cA -= 1.0f;
+                if (cA < (float)aA.n && fmaf(cA, dA, A0) < s) cA += 1.0f;
+            }
+            pA = fmaf(cA, dA, A0);
+            off += (unsigned)(int)cA * sA + (unsigned)k * sD;
+        }
+    }
+    for (int u = ubegin; u <= ulast; u += kFlatUnroll) {
         const int k0 = u - o;
         const float kf = (float)k0;
         // all slabs of the block lie on every ray and end before its last
@@ -713,6 +735,31 @@ __global__ __launch_bounds__(64 * kFlatWaves) void k_ray_fp_flat(float *__restri
     float chord;
     const float acc = trace_ray_flat(g, ib, ip, ip < g.np, chord);
     if (ip < g.np) proj[(size_t)ib * g.np + ip] = acc;
+}
+
+// The same for few rays: the block's wavefronts walk a share of the slabs of the
+// same 64 rays each, and the shares are added in order.  A ray's walk is a chain
+// of gathers' latencies that nothing hides below a few wavefronts per SIMD.
+// Whole calls, a ray to one lane / split by 2 / 4 / 8 (pixels, views x bins):
+//    64^2,  90 x   96   17.8 / 11.0 / 10.2 / 10.4 us
+//   128^2, 180 x  192   29.1 / 20.8 / 17.6 / 16.3 us
+//   256^2, 360 x  512   50.2 / 50.2 / 47.1 / 57.4 us
+//   512^2, 360 x  730  125.6 / 105.8 / 99.7 / 113.3 us (4320 wavefronts of rays)
+//   512^2, 720 x 1024    156 / 191 / 231 / 285 us (11520)
+// 3 us of the first line are the image's transpose, left out up to 128^2 pixels.
+__global__ __launch_bounds__(64 * kFlatWaves) void k_ray_fp_flat_split(float *__restrict__ proj, RayParams g)
+{
+    __shared__ float part[kFlatWaves][64];
+    const int chunks = (g.np + 63) / 64, ib = blockIdx.x / chunks, ip = (blockIdx.x - ib * chunks) * 64 + (int)threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    float chord;
+    part[wave][threadIdx.x] = trace_ray_flat(g, ib, ip, ip < g.np, chord, wave, kFlatWaves);
+    __syncthreads();
+    if (wave != 0 || ip >= g.np) return;
+    float sum = part[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < kFlatWaves; ++w) sum += part[w][threadIdx.x];
+    proj[(size_t)ib * g.np + ip] = sum;
 }
 
 // The residual pass (fp_residual_block) of a 2-D problem.
@@ -1203,9 +1250,16 @@ hipError_t launch_sysmat_fill(const RayParams &g, const long long *row_ptr, int 
     return hipGetLastError();
 }
 
+// Where splitting the rays of a 2-D projection is faster (k_ray_fp_flat_split).
+bool flat_split(const RayParams &g) { return (long)((g.np + 63) / 64) * g.nb < 6144; }
+
 hipError_t launch_ray_fp(const RayParams &g, const float *vol, float *proj, hipStream_t st)
 {
     if (g.volZ) return launch_columns(g, proj, st);
+    if (g.flat && flat_split(g)) {
+        hipLaunchKernelGGL(k_ray_fp_flat_split, dim3((g.np + 63) / 64 * g.nb), dim3(64, kFlatWaves), 0, st, proj, g);
+        return hipGetLastError();
+    }
     if (g.flat) {
         hipLaunchKernelGGL(k_ray_fp_flat, dim3(flat_blocks(g)), dim3(64, kFlatWaves), 0, st, proj, g);
         return hipGetLastError();

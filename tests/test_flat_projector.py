@@ -14,7 +14,9 @@ from conftest import errs, report
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nt,ns,bins,views", [(1, 1, 1, 4), (1, 37, 63, 9), (41, 1, 64, 9), (40, 33, 65, 16),
+# up to 6143 wavefronts of 64 rays a ray is split over four of them, and up to
+# 128^2 pixels the image is read without its transpose
+@pytest.mark.parametrize("nt,ns,bins,views", [(1, 1, 1, 4), (129, 130, 70, 7), (40, 33, 256, 1600), (1, 37, 63, 9), (41, 1, 64, 9), (40, 33, 65, 16),
                                               (64, 64, 130, 24), (257, 129, 200, 8)])
 @pytest.mark.parametrize("beam", ["fan", "parallel"])
 def test_flat_projector(ctx, oracle, nt, ns, bins, views, beam):
