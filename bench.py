@@ -61,7 +61,7 @@ def _profile_value(path, section, key):
 
 
 def traffic_from_profiles():
-    """HBM bytes per launch of the FDK kernel measured with rocprofv3 --pmc
+    """HBM bytes per call of the FDK kernels measured with rocprofv3 --pmc
     (FETCH_SIZE + WRITE_SIZE, calibrated with a copy kernel).  None when not measured."""
     try:
         with open(TRAFFIC_PROFILE) as f:
@@ -203,7 +203,7 @@ def main():
                    "views_per_pass": K, "filter_ms": round(filter_ms, 4), "kernel_ms": round(kernel_ms, 4)},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic_from_profiles(),
-                     "traffic_source": "FETCH_SIZE x 2 + WRITE_SIZE of k_bp_tiled, "
+                     "traffic_source": "FETCH_SIZE x 2 + WRITE_SIZE of k_bp_tiled and k_sum_parts, "
                                        "profiles/fdk_bp_256_360_traffic.txt",
                      # HBM is the contract's memory roofline but not what bounds this kernel
                      "binds": False, "binding_roofline": "valu_roofline"},
