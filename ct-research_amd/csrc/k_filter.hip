@@ -557,8 +557,22 @@ __device__ __forceinline__ void transform(double2 *v, double *words, int j, doub
 }
 }  // namespace f16
 
+// Sample q of a row times its pre-weight, rounded to float (MODE as k_fft16_filter).
+template <int MODE>
+__device__ __forceinline__ float weighted_sample(const FilterParams &P, const float *src, const double *pw, float xi, int q)
+{
+    if constexpr (MODE == 0) return cone_preweight(src[q], cone_weight64(P.Dd, P.pd[q], xi));
+    else if constexpr (MODE == 4) return cone_preweight(src[q], pw[q]);
+    else return src[q] * (MODE == 1 ? P.colw[q] : 1.0f);
+}
+
+__device__ __forceinline__ bool not_finite(float x) { return (__float_as_uint(x) & 0x7f800000u) == 0x7f800000u; }
+
 // MODE as k_fft_filter (0, 1, 2, 4; rows are paired as 2p, 2p + 1); each
 // group of G lanes filters one row pair per step.
+// Rows of L = 4096 keep their infinities and NaN to themselves, as the direct
+// convolution does: a row that holds one enters the transform as zeros, and
+// its output is formed by the direct sums.
 // Four waves per SIMD (128 registers); the FP64 weights formed per sample
 // (MODE 0) need more, so three.
 template <int L, int MODE>
@@ -593,6 +607,7 @@ void k_fft16_filter(const float *__restrict__ in, float *__restrict__ out, Filte
         const double *pw0 = MODE == 4 ? P.pw + (size_t)(rd0 % P.nx) * np : nullptr;
         const double *pw1 = MODE == 4 ? P.pw + (size_t)(rd1 % P.nx) * np : nullptr;
         double2 v[16];
+        bool bad0 = false, bad1 = false;
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const int q = jr + F::G * t, qc = q < np ? q : np - 1;
@@ -610,8 +625,22 @@ void k_fft16_filter(const float *__restrict__ in, float *__restrict__ out, Filte
                 a = (double)(src0[qc] * w);
                 b = (double)(src1[qc] * w);
             }
+            // (columns past the end repeat the last one, an absent second row the first)
+            if constexpr (L == 4096) {
+                bad0 |= not_finite((float)a);
+                bad1 |= not_finite((float)b);
+            }
             v[t] = make_double2(q < np && has0 ? a : 0.0, q < np && has1 ? b : 0.0);
             v[t + 8] = make_double2(0.0, 0.0);
+        }
+        if constexpr (L == 4096) {
+            static_assert(F::kPerBlock == 1, "the flags are the workgroup's");
+            if (__syncthreads_or(bad0 || bad1)) {
+                bad0 = __syncthreads_or(bad0);
+                bad1 = __syncthreads_or(bad1);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) v[t] = make_double2(bad0 ? 0.0 : v[t].x, bad1 ? 0.0 : v[t].y);
+            }
         }
         f16::transform<L, true>(v, mine, j, t256, tL);
         // H[k] / L (real) at k = j + G t, from a uniform base and a 32-bit offset
@@ -622,6 +651,25 @@ void k_fft16_filter(const float *__restrict__ in, float *__restrict__ out, Filte
             v[t] = make_double2(v[t].x * h, -v[t].y * h);
         }
         f16::transform<L, false>(v, mine, j, t256, tL);
+        if constexpr (L == 4096) {
+            if (bad0 || bad1) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t) v[t] = make_double2(bad0 ? 0.0 : v[t].x, bad1 ? 0.0 : v[t].y);
+#pragma unroll 1
+                for (int k = 0; k < np; ++k) {
+                    const double a = bad0 ? (double)weighted_sample<MODE>(P, src0, pw0, xi0, k) : 0.0;
+                    const double b = bad1 ? (double)weighted_sample<MODE>(P, src1, pw1, xi1, k) : 0.0;
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) {
+                        const int q = jr + F::G * t;
+                        const double h = P.taps[(q < np ? q : np - 1) - k + np - 1];
+                        v[t].x = fma(a, h, v[t].x);
+                        v[t].y = fma(-b, h, v[t].y);
+                    }
+                }
+                __syncthreads();   // a row filtered in place is read to its end before it is overwritten
+            }
+        }
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const int q = jr + F::G * t;
