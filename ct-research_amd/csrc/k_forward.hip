@@ -1054,12 +1054,17 @@ __device__ __forceinline__ float trace_column(const RayParams &g, const ColumnHe
     float acc = 0.0f;
     const int nb = h.n / kColBlock;
     if (__ballot(dZ != 0.0f && dZ < h.pair) == 0) {
-        // widest run of slices (bytes): the rows fan out from the source until
-        // the line leaves the box or the outermost row its top or bottom, where
-        // its slice stays
+        // widest run of slices (bytes) between the first and the last row, the
+        // outermost ones: a row's height grows with the way from the source until
+        // the line leaves the box, or the row its top or bottom, where its slice
+        // stays.  Rows on one side of the source plane fan out until the outer one
+        // leaves; on both sides each goes on until it leaves by itself.
         const float s0 = lane_float((float)slope, 0), s1 = lane_float((float)slope, 63);
-        const float reach = (float)(h.lo + h.len), outer = fmaxf(fabsf(s0), fabsf(s1)) * reach, half = 0.5f * (float)g.bz;
-        const float wide = 4.0f * (fabsf(s1 - s0) * reach * (outer > half ? half / outer : 1.0f) * (float)inv_rz) + 36.0f;
+        const float reach = (float)(h.lo + h.len), half = 0.5f * (float)g.bz;
+        const float r0 = fabsf(s0) * reach, r1 = fabsf(s1) * reach, outer = fmaxf(r0, r1);
+        const float fan = s0 * s1 < 0.0f ? fminf(r0, half) + fminf(r1, half)
+                                         : fabsf(s1 - s0) * reach * (outer > half ? half / outer : 1.0f);
+        const float wide = 4.0f * (fan * (float)inv_rz) + 36.0f;
         const bool narrow = wide <= 4.0f * 63.0f, gentle = __ballot(dZ != 0.0f && dZ < h.block) == 0;
         const ColumnLane lane{Z0, dZ, zb, sgn};
         if (gentle)

@@ -75,3 +75,51 @@ def test_columns_leave_sirt_alone(ctx, monkeypatch):
     monkeypatch.setenv("CTR_FP_COLUMNS", "1")
     x1, r1, s1 = ctx.sirt3d(g, b, 2)
     assert np.array_equal(x1, x0) and np.array_equal(r1, r0) and np.array_equal(s1, s0)
+
+
+OFF_CENTRE = {
+    # name: nt, ns, nz, size, D, rows, row pitch, rows the detector is shifted by.
+    # All but the last two have a wavefront whose first and last row lie on both
+    # sides of the source plane, one farther out than the other, more slices apart
+    # than the shared window holds, or close to it, where the line leaves the
+    # volume; "fits" has the same within the window.
+    "one_chunk_up": (256, 256, 80, (256.0, 256.0, 80.0), 600.0, 64, 1.65, 18.5),
+    "one_chunk_down": (256, 256, 80, (256.0, 256.0, 80.0), 600.0, 64, 1.65, -18.5),
+    "near_the_source": (128, 128, 80, (128.0, 128.0, 80.0), 205.0, 128, 1.0, -16.0),
+    "three_chunks": (256, 256, 80, (256.0, 256.0, 80.0), 600.0, 191, 1.1, 15.0),
+    "centred": (256, 256, 100, (256.0, 256.0, 100.0), 600.0, 246, 2.5, 0.0),
+    "descending": (256, 256, 80, (256.0, 256.0, 80.0), 600.0, 191, -1.1, 15.0),
+    "fits": (256, 256, 80, (256.0, 256.0, 80.0), 600.0, 64, 0.55, 12.0),
+    "one_side": (256, 256, 80, (256.0, 256.0, 80.0), 600.0, 64, 1.1, 32.5),
+}
+
+
+def _off_centre(case, lib, views, columns):
+    nt, ns, nz, size, D, nx, px, shift = OFF_CENTRE[case]
+    beta = (np.pi / 4 + 2 * np.pi / views * np.arange(views)).astype(np.float32)
+    p = (150.0 / columns * (np.arange(columns) - (columns - 1) / 2) + 0.03).astype(np.float32)
+    xi = (px * (np.arange(nx) - (nx - 1) / 2 + shift)).astype(np.float32)
+    return lib(nt, ns, nz, size, D, beta, p, xi)
+
+
+@pytest.mark.parametrize("case", OFF_CENTRE)
+def test_rows_on_both_sides_of_the_source_plane(ctx, oracle, columns, case):
+    import ctr
+    g, og = _off_centre(case, ctr.ConeGeom, 3, 9), _off_centre(case, oracle.Cone, 3, 9)
+    vol = np.random.default_rng(len(case)).random(g.nvox).astype(np.float32)
+    print(f"[case] columns off centre {case} {g.vol_shape} {g.proj_shape}", flush=True)
+    e, m = errs(ctx.cone_fp(g, vol), oracle.cone_fp_exact(og, vol))
+    report(f"columns_off_centre[{case}]", rel_l2=e, max_rel=m)
+    assert e < 2e-6 and m < 2e-5
+
+
+@pytest.mark.parametrize("case", ["one_chunk_up", "one_chunk_down"])
+def test_off_centre_rows_by_the_librarys_own_rule(ctx, oracle, case):
+    """Enough wavefronts and slices for the library to take the columns by itself."""
+    import ctr
+    g, og = _off_centre(case, ctr.ConeGeom, 121, 101), _off_centre(case, oracle.Cone, 121, 101)
+    vol = np.random.default_rng(7).random(g.nvox).astype(np.float32)
+    print(f"[case] columns by rule {case} {g.vol_shape} {g.proj_shape}", flush=True)
+    e, m = errs(ctx.cone_fp(g, vol), oracle.cone_fp_exact(og, vol))
+    report(f"columns_by_rule[{case}]", rel_l2=e, max_rel=m)
+    assert e < 2e-6 and m < 2e-5
