@@ -490,11 +490,12 @@ struct SliceRows {
         off_low = P.v_off - margin + 1.0f;   // the first row above: floor(v - margin) + 1
         off_high = P.v_off + margin;
     }
-    // smin, smax: mmin, mmax times v_scale
+    // smin, smax: mmin, mmax times v_scale.  Both ends stay within one row of
+    // [first, last]: a thick slice may lie any number of rows off the detector.
     __device__ __forceinline__ void rows(int k, float smin, float smax, int first, int last, int &rv0, int &rv1) const
     {
-        rv0 = max(floor_int(fmaf(low[k], low_far[k] ? smax : smin, off_low)), first);
-        rv1 = min(floor_int(fmaf(high[k], high_far[k] ? smax : smin, off_high)), last);
+        rv0 = min(max(floor_int(fmaf(low[k], low_far[k] ? smax : smin, off_low)), first), last + 1);
+        rv1 = max(min(floor_int(fmaf(high[k], high_far[k] ? smax : smin, off_high)), last), first - 1);
     }
 };
 
@@ -629,16 +630,16 @@ __device__ __forceinline__ void adjoint_tile(const float *__restrict__ proj, flo
                 float a_k = 0.0f;
                 if (fits) {
                     // two rows an iteration, the second at immediate offsets
-                    const float2 *zt = ztab + (rv0 - f.y) * TZ + k, *zend = ztab + (rv1 - f.y) * TZ + k;
+                    const float2 *zt = ztab + (rv0 - f.y) * TZ + k;
                     const float *sy = yd + (rv0 - f.y) * WP + (cb - f.x);
                     auto row = [&](const float2 *z, const float *y) {
                         const float2 zz = *z;
 #pragma unroll
                         for (int q = 0; q < CM; ++q) a_k = fmaf(overlap(zz.x, zz.y, clo[q], chi[q]), y[q], a_k);
                     };
-                    for (; zt <= zend; zt += 2 * TZ, sy += 2 * WP) {
+                    for (int n = rv1 - rv0 + 1; n > 0; n -= 2, zt += 2 * TZ, sy += 2 * WP) {
                         row(zt, sy);
-                        if (zt < zend) row(zt + TZ, sy + WP);
+                        if (n > 1) row(zt + TZ, sy + WP);
                     }
                 } else {
                     const float zb = fmaf((float)k, P.rz, zbase);

@@ -47,3 +47,28 @@ def test_split_adjoint(ctx, oracle, shape, views):
     report(f"split_adjoint[{shape},{views}]", rel_l2=e, max_rel=m)
     assert e < 1e-4 and m < 1e-3
     np.testing.assert_array_equal(ctx.cone_bp_adjoint(g, y, out=vol.copy(), flags=ctr.ACCUMULATE), vol + vol)
+
+
+@pytest.mark.parametrize("pitch", [0.01, 1e-9])
+@pytest.mark.parametrize("nz", [4, 6])
+def test_adjoint_of_slices_far_off_the_rows(ctx, oracle, nz, pitch):
+    """Few fine rows and thick slices: the slices of a tile that the rows miss lie
+    hundreds of rows (and more than an int counts) away from the staged ones.
+    Rows of 1e-9 mm are finer than a float knows a face of a 6 mm slice (4e-7 mm),
+    so that only the slices which no ray comes near have a value to hold to."""
+    import ctr
+    beta = (2 * np.pi / 9 * np.arange(9) + 0.1).astype(np.float32)
+    p = (0.8 * (np.arange(37) - 18)).astype(np.float32)
+    xi = (pitch * (np.arange(20) - 9.3)).astype(np.float32)
+    a = (16, 17, nz, (16.0, 17.0, 6.0 * nz), 60.0, beta, p, xi)
+    g, og = ctr.ConeGeom(*a), oracle.Cone(*a)
+    y = np.random.default_rng(nz).random(g.nray).astype(np.float32)
+    print(f"[case] adjoint of {nz} slices of 6 mm, 20 rows of {pitch} mm", flush=True)
+    vol, ref = ctx.cone_bp_adjoint(g, y), oracle.cone_adjoint(og, y)
+    if pitch < 1e-6:
+        slices = np.asarray(vol).reshape(g.vol_shape).any(axis=(1, 2))
+        assert np.isfinite(vol).all() and list(np.flatnonzero(slices)) == [nz // 2 - 1, nz // 2]
+        return
+    e, m = errs(vol, ref)
+    report(f"thick_slices[{nz},{pitch}]", rel_l2=e, max_rel=m)
+    assert e < 1e-4 and m < 1e-3
