@@ -1043,6 +1043,7 @@ __device__ __forceinline__ float trace_column(const RayParams &g, const ColumnHe
     }
     const double norm = sqrt(fma(slope, slope, 1.0));
     const bool hit = fmin(h.len, out) > 0.0;
+    if (__ballot(hit) == 0) return 0.0f;
     const float Z0 = (float)z0, dZ = (float)dz;
     const int top = 4 * (g.nz + 1);   // slices 0 and nz + 1 of the copy are zeros
     const int zb = (int)fmin(fmax(4.0 * (k0 + 1.0), 0.0), (double)top), sgn = slope > 0.0 ? 4 : -4;
@@ -1074,7 +1075,11 @@ __device__ __forceinline__ float trace_column(const RayParams &g, const ColumnHe
             acc = narrow ? column_sum<true, kColBlock / 2>(rs, blk, nb, top, lane)
                          : column_sum<false, kColBlock / 2>(rs, blk, nb, top, lane);
     } else {
-        float pZ = Z0;
+        // a ray crosses no planes behind the volume's top or bottom: it may be
+        // steep enough for any number of them there (thin slices, rows far off
+        // the volume)
+        const int edge = slope > 0.0 ? top : 0;
+        float pZ = zb == edge ? __builtin_huge_valf() : Z0;
         int za = zb, cz = 0;
         auto load = [&](int z, unsigned cell) {
             return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, z, (int)cell, 0));
@@ -1091,8 +1096,8 @@ __device__ __forceinline__ float trace_column(const RayParams &g, const ColumnHe
                     l = pZ;
                 }
                 ++cz;
-                pZ = fmaf((float)cz, dZ, Z0);
                 za = clamp_i(__mul24(cz, sgn) + zb, top);
+                pZ = za == edge ? __builtin_huge_valf() : fmaf((float)cz, dZ, Z0);
             }
             if (l1 > l) acc = fmaf(l1 - l, load(za, cell), acc);
         }
@@ -1212,8 +1217,9 @@ static bool column_use(const RayParams &g, double row_pitch)
 
 bool column_plan(const RayParams &g, double row_pitch, ColumnPlan &L)
 {
-    // 32-bit offsets into the z-fastest copy, one workgroup row per view in the list kernel
-    if (g.parallel || (size_t)g.nt * g.ns * (g.nz + 2) > ((size_t)1 << 30)) return false;
+    // 32-bit offsets into the z-fastest copy, 24-bit offsets into its columns,
+    // one workgroup row per view in the list kernel
+    if (g.parallel || (size_t)g.nt * g.ns * (g.nz + 2) > ((size_t)1 << 30) || g.nz > (1 << 20)) return false;
     if (!column_use(g, row_pitch)) return false;
     L.stride = (g.nt + g.ns + 1 + 2 * kColBlock - 1) / (2 * kColBlock) * (2 * kColBlock) + kColBlock;
     if (L.stride > 4096) return false;   // the list kernel's LDS

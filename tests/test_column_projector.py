@@ -123,3 +123,27 @@ def test_off_centre_rows_by_the_librarys_own_rule(ctx, oracle, case):
     e, m = errs(ctx.cone_fp(g, vol), oracle.cone_fp_exact(og, vol))
     report(f"columns_by_rule[{case}]", rel_l2=e, max_rel=m)
     assert e < 2e-6 and m < 2e-5
+
+
+@pytest.mark.parametrize("depth", [6e-7, 1e-44])
+def test_rows_far_off_thin_slices(ctx, oracle, columns, depth):
+    """Six slices whose thickness is next to nothing: the rows that miss them pass
+    tens of millions of their planes, were these to go on, or planes so close that
+    a float has no distance for them.  Rays end at the top and the bottom slice."""
+    import ctr
+    beta = (2 * np.pi / 5 * np.arange(5) + 0.1).astype(np.float32)
+    p = (0.9 * (np.arange(30) - 14.5) + 0.03).astype(np.float32)
+    inside = np.array([-1.15, -0.9, -0.4, 0.0, 0.3, 0.8, 1.2]) * 0.5 * depth
+    xi = np.unique(np.concatenate([np.linspace(-15, -0.25, 30), inside, np.linspace(0.5, 15, 33)]).astype(np.float32))
+    a = (24, 20, 6, (24.0, 20.0, depth), 70.0, beta, p, xi)
+    g, og = ctr.ConeGeom(*a), oracle.Cone(*a)
+    vol = np.random.default_rng(5).random(g.nvox).astype(np.float32)
+    print(f"[case] columns, six slices in {depth} mm, {len(xi)} rows", flush=True)
+    got, ref = ctx.cone_fp(g, vol), oracle.cone_fp_exact(og, vol)
+    if depth < 1e-40:   # thinner than the oracle's own arithmetic: the rows off the volume only
+        off = np.abs(np.broadcast_to(xi[None, :, None], g.proj_shape)) > 0.1
+        assert not np.asarray(got).reshape(g.proj_shape)[off].any()
+        return
+    e, m = errs(got, ref)
+    report(f"columns_thin[{depth}]", rel_l2=e, max_rel=m)
+    assert e < 2e-6 and m < 2e-5
