@@ -1193,7 +1193,7 @@ constexpr size_t kColListBytes = (size_t)256 << 20;
 // overrides).  A wavefront always pays for 64 rows, so they need about 0.7 of
 // its lanes filled, and three launches and a list of the cells pay from 12000
 // wavefronts and 80 slices on; the rows of a wavefront are to span less than 70
-// slices at the far side (they share one run of 64) unless nearly all are
+// slices at the far side (they share one run of 64), or 110 where nearly all are
 // filled.  Slab walk / columns in us (nz, views x columns x rows, span):
 //   324, 183 x 674 x 467, 59   11910 / 8180    269, 25 x 567 x 521, 74   1458 / 1944
 //   254, 223 x 688 x 414, 57   12409 / 8869    258, 105 x 408 x 387, 87  3522 / 3783
@@ -1201,6 +1201,12 @@ constexpr size_t kColListBytes = (size_t)256 << 20;
 //   125, 25 x 358 x 156, 53      218 /  173     51, 232 x 164 x 101, 54   197 /  214
 //    89, 124 x 173 x 126, 61     198 /  137     43, 290 x 121 x 60, 59    116 /  121
 //   109, 350 x 288 x 132, 73    1770 / 1750     52, 139 x 186 x 69 (0.54 filled) 121 / 147
+// Wider spans, all lanes filled (rows leave the volume at its top and bottom,
+// and the slab walk ends there; beyond 250 slices the columns lose without limit,
+// 153 / 570 us at 4100):
+//    80, 60 x 300 x 128, 82    359 / 264        80, 60 x 300 x 128, 164   267 / 276
+//   120, 60 x 300 x 128, 123   396 / 453       200, 60 x 300 x 256, 115   677 / 767
+//   320, 90 x 300 x 384, 115  3929 / 3371      200, 60 x 300 x 256, 262   433 / 500
 // Over 66 geometries of 20 to 400 slices: 0.6% slower on the mean than the
 // faster of the two each time, 10% faster than the slab walk.
 // The residual pass of SIRT keeps the slab walk: the history of its norms, in 64
@@ -1212,7 +1218,7 @@ static bool column_use(const RayParams &g, double row_pitch)
     const size_t chunks = (g.nx + 63) / 64, waves = (size_t)g.nb * g.np * chunks;
     const double fill = (double)g.nx / (64.0 * chunks), far = g.D + 0.5 * std::hypot(g.bt, g.bs);
     const double span = 63.0 * row_pitch * far / (g.D * g.rz);
-    return g.nz >= 80 && waves >= 12000 && fill >= 0.7 && (span < 70.0 || fill > 0.95);
+    return g.nz >= 80 && waves >= 12000 && fill >= 0.7 && span < (fill > 0.95 ? 110.0 : 70.0);
 }
 
 bool column_plan(const RayParams &g, double row_pitch, ColumnPlan &L)

@@ -85,6 +85,8 @@ OFF_CENTRE = {
     # volume; "fits" has the same within the window.
     "one_chunk_up": (256, 256, 80, (256.0, 256.0, 80.0), 600.0, 64, 1.65, 18.5),
     "one_chunk_down": (256, 256, 80, (256.0, 256.0, 80.0), 600.0, 64, 1.65, -18.5),
+    "fine_up": (256, 256, 80, (256.0, 256.0, 80.0), 600.0, 64, 1.3, 16.0),
+    "fine_down": (256, 256, 80, (256.0, 256.0, 80.0), 600.0, 64, 1.3, -16.0),
     "near_the_source": (128, 128, 80, (128.0, 128.0, 80.0), 205.0, 128, 1.0, -16.0),
     "three_chunks": (256, 256, 80, (256.0, 256.0, 80.0), 600.0, 191, 1.1, 15.0),
     "centred": (256, 256, 100, (256.0, 256.0, 100.0), 600.0, 246, 2.5, 0.0),
@@ -113,7 +115,7 @@ def test_rows_on_both_sides_of_the_source_plane(ctx, oracle, columns, case):
     assert e < 2e-6 and m < 2e-5
 
 
-@pytest.mark.parametrize("case", ["one_chunk_up", "one_chunk_down"])
+@pytest.mark.parametrize("case", ["fine_up", "fine_down"])
 def test_off_centre_rows_by_the_librarys_own_rule(ctx, oracle, case):
     """Enough wavefronts and slices for the library to take the columns by itself."""
     import ctr
