@@ -1052,7 +1052,38 @@ __device__ __forceinline__ float trace_column(const RayParams &g, const ColumnHe
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         (void *)g.volZ, 0, (int)(vbytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (unsigned)vbytes), kBufDword3);
     const ColumnBlock *__restrict__ blk = blocks + col * stride;
+    // cell by cell: the voxels that the ray meets and no others
+    auto by_cells = [&]() {
+        // a ray crosses no planes behind the volume's top or bottom: it may be
+        // steep enough for any number of them there (thin slices, rows far off
+        // the volume)
+        const int edge = slope > 0.0 ? top : 0;
+        float sum = 0.0f, pZ = zb == edge ? __builtin_huge_valf() : Z0;
+        int za = zb, cz = 0;
+        auto load = [&](int z, unsigned cell) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, z, (int)cell, 0));
+        };
+        for (int i = 0; i < h.n; ++i) {
+            const ColumnBlock &c = blk[i / kColBlock];
+            const int j = i % kColBlock;
+            const float l1 = c.l[j + 1];
+            const unsigned cell = c.off[j];
+            float l = c.l[j];
+            while (pZ < l1) {
+                if (pZ > l) {
+                    sum = fmaf(pZ - l, load(za, cell), sum);
+                    l = pZ;
+                }
+                ++cz;
+                za = clamp_i(__mul24(cz, sgn) + zb, top);
+                pZ = za == edge ? __builtin_huge_valf() : fmaf((float)cz, dZ, Z0);
+            }
+            if (l1 > l) sum = fmaf(l1 - l, load(za, cell), sum);
+        }
+        return sum;
+    };
     float acc = 0.0f;
+    bool again = true;
     const int nb = h.n / kColBlock;
     if (__ballot(dZ != 0.0f && dZ < h.pair) == 0) {
         // widest run of slices (bytes) between the first and the last row, the
@@ -1074,33 +1105,13 @@ __device__ __forceinline__ float trace_column(const RayParams &g, const ColumnHe
         else
             acc = narrow ? column_sum<true, kColBlock / 2>(rs, blk, nb, top, lane)
                          : column_sum<false, kColBlock / 2>(rs, blk, nb, top, lane);
-    } else {
-        // a ray crosses no planes behind the volume's top or bottom: it may be
-        // steep enough for any number of them there (thin slices, rows far off
-        // the volume)
-        const int edge = slope > 0.0 ? top : 0;
-        float pZ = zb == edge ? __builtin_huge_valf() : Z0;
-        int za = zb, cz = 0;
-        auto load = [&](int z, unsigned cell) {
-            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, z, (int)cell, 0));
-        };
-        for (int i = 0; i < h.n; ++i) {
-            const ColumnBlock &c = blk[i / kColBlock];
-            const int j = i % kColBlock;
-            const float l1 = c.l[j + 1];
-            const unsigned cell = c.off[j];
-            float l = c.l[j];
-            while (pZ < l1) {
-                if (pZ > l) {
-                    acc = fmaf(pZ - l, load(za, cell), acc);
-                    l = pZ;
-                }
-                ++cz;
-                za = clamp_i(__mul24(cz, sgn) + zb, top);
-                pZ = za == edge ? __builtin_huge_valf() : fmaf((float)cz, dZ, Z0);
-            }
-            if (l1 > l) acc = fmaf(l1 - l, load(za, cell), acc);
-        }
+        // column_sum multiplies a block's other slice by 0, and an infinite or
+        // NaN voxel there makes a NaN of a ray that passes it by
+        again = !(fabsf(acc) < __builtin_huge_valf());
+    }
+    if (__ballot(again) != 0) {
+        const float sum = by_cells();
+        acc = again ? sum : acc;
     }
     return hit ? acc * (float)norm : 0.0f;
 }

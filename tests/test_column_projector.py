@@ -149,3 +149,30 @@ def test_rows_far_off_thin_slices(ctx, oracle, columns, depth):
     e, m = errs(got, ref)
     report(f"columns_thin[{depth}]", rel_l2=e, max_rel=m)
     assert e < 2e-6 and m < 2e-5
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("case", ["rows130", "rows65", "steep", "very_steep", "wide_rows"])
+def test_a_voxel_that_is_not_finite(ctx, columns, case, bad):
+    """It reaches the rays that cross it, and those alone: the others have the bits
+    of the projection with a 0 in its place."""
+    import ctr
+    g = _geom(case, ctr.ConeGeom)
+    nz, ns, nt = g.vol_shape
+    vol = np.random.default_rng(3).random(g.vol_shape).astype(np.float32)
+    crossed = 0
+    for at in ((nz // 2, ns // 2, nt // 3), (nz - 1, ns // 2, nt // 2), (0, 0, 0)):
+        print(f"[case] {case} {bad} at {at}", flush=True)
+        one = np.zeros(g.vol_shape, np.float32)
+        one[at] = 1.0
+        meets = ctx.cone_fp(g, one.ravel())
+        vol[at] = 0.0
+        clean = ctx.cone_fp(g, vol.ravel())
+        vol[at] = bad
+        got = ctx.cone_fp(g, vol.ravel())
+        vol[at] = 0.5
+        assert np.array_equal(got[meets == 0], clean[meets == 0])
+        hit = meets > 1e-4 * meets.max() if meets.any() else np.zeros(len(meets), bool)
+        assert np.array_equal(got[hit], np.full(hit.sum(), bad, np.float32), equal_nan=True)
+        crossed += hit.sum()
+    assert crossed
