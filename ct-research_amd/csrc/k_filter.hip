@@ -566,13 +566,23 @@ __device__ __forceinline__ float weighted_sample(const FilterParams &P, const fl
     else return src[q] * (MODE == 1 ? P.colw[q] : 1.0f);
 }
 
-__device__ __forceinline__ bool not_finite(float x) { return (__float_as_uint(x) & 0x7f800000u) == 0x7f800000u; }
+// Largest of a wavefront.
+__device__ __forceinline__ unsigned wave_max(unsigned v)
+{
+    for (int m = 32; m > 0; m >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, m, 64));
+    return v;
+}
+
+__device__ __forceinline__ double power_of_two(int e) { return __builtin_bit_cast(double, (unsigned long long)(1023 + e) << 52); }
 
 // MODE as k_fft_filter (0, 1, 2, 4; rows are paired as 2p, 2p + 1); each
 // group of G lanes filters one row pair per step.
-// Rows of L = 4096 keep their infinities and NaN to themselves, as the direct
-// convolution does: a row that holds one enters the transform as zeros, and
-// its output is formed by the direct sums.
+// Rows of L = 4096 are as accurate as the direct convolution makes them,
+// whatever shares their transform: each enters it scaled by a power of two that
+// brings its largest sample to [1, 2), so that the rounding of a row 1e9 times
+// larger stays in that row, and a row of zeros comes out as zeros.  A row that
+// holds an infinity or NaN enters as zeros, and its output is formed by the
+// direct sums.
 // Four waves per SIMD (128 registers); the FP64 weights formed per sample
 // (MODE 0) need more, so three.
 template <int L, int MODE>
@@ -607,7 +617,7 @@ void k_fft16_filter(const float *__restrict__ in, float *__restrict__ out, Filte
         const double *pw0 = MODE == 4 ? P.pw + (size_t)(rd0 % P.nx) * np : nullptr;
         const double *pw1 = MODE == 4 ? P.pw + (size_t)(rd1 % P.nx) * np : nullptr;
         double2 v[16];
-        bool bad0 = false, bad1 = false;
+        unsigned top0 = 0, top1 = 0;   // largest magnitudes, as bits
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const int q = jr + F::G * t, qc = q < np ? q : np - 1;
@@ -627,20 +637,34 @@ void k_fft16_filter(const float *__restrict__ in, float *__restrict__ out, Filte
             }
             // (columns past the end repeat the last one, an absent second row the first)
             if constexpr (L == 4096) {
-                bad0 |= not_finite((float)a);
-                bad1 |= not_finite((float)b);
+                top0 = max(top0, __float_as_uint((float)a) & 0x7fffffffu);
+                top1 = max(top1, __float_as_uint((float)b) & 0x7fffffffu);
             }
             v[t] = make_double2(q < np && has0 ? a : 0.0, q < np && has1 ? b : 0.0);
             v[t + 8] = make_double2(0.0, 0.0);
         }
         if constexpr (L == 4096) {
-            static_assert(F::kPerBlock == 1, "the flags are the workgroup's");
-            if (__syncthreads_or(bad0 || bad1)) {
-                bad0 = __syncthreads_or(bad0);
-                bad1 = __syncthreads_or(bad1);
-#pragma unroll
-                for (int t = 0; t < 8; ++t) v[t] = make_double2(bad0 ? 0.0 : v[t].x, bad1 ? 0.0 : v[t].y);
+            static_assert(F::kPerBlock == 1, "the maxima are the workgroup's");
+            constexpr int W = F::kThreads / 64;
+            __shared__ unsigned tops[2][W];
+            top0 = wave_max(top0);
+            top1 = wave_max(top1);
+            if ((threadIdx.x & 63) == 0) {
+                tops[0][threadIdx.x >> 6] = top0;
+                tops[1][threadIdx.x >> 6] = top1;
             }
+            __syncthreads();   // (the transforms' barriers lie before the next pair's maxima)
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                top0 = max(top0, tops[0][w]);
+                top1 = max(top1, tops[1][w]);
+            }
+            top0 = __builtin_amdgcn_readfirstlane(top0);
+            top1 = __builtin_amdgcn_readfirstlane(top1);
+            const bool bad0 = top0 >= 0x7f800000u, bad1 = top1 >= 0x7f800000u;
+            const double s0 = power_of_two(127 - max((int)(top0 >> 23), 1)), s1 = power_of_two(127 - max((int)(top1 >> 23), 1));
+#pragma unroll
+            for (int t = 0; t < 8; ++t) v[t] = make_double2(bad0 ? 0.0 : v[t].x * s0, bad1 ? 0.0 : v[t].y * s1);
         }
         f16::transform<L, true>(v, mine, j, t256, tL);
         // H[k] / L (real) at k = j + G t, from a uniform base and a 32-bit offset
@@ -652,9 +676,13 @@ void k_fft16_filter(const float *__restrict__ in, float *__restrict__ out, Filte
         }
         f16::transform<L, false>(v, mine, j, t256, tL);
         if constexpr (L == 4096) {
-            if (bad0 || bad1) {
+            const bool bad0 = top0 >= 0x7f800000u, bad1 = top1 >= 0x7f800000u;
+            const double u0 = bad0 || top0 == 0 ? 0.0 : power_of_two(max((int)(top0 >> 23), 1) - 127);
+            const double u1 = bad1 || top1 == 0 ? 0.0 : power_of_two(max((int)(top1 >> 23), 1) - 127);
+            // (a product of -0 is +0 after the addition)
 #pragma unroll
-                for (int t = 0; t < 8; ++t) v[t] = make_double2(bad0 ? 0.0 : v[t].x, bad1 ? 0.0 : v[t].y);
+            for (int t = 0; t < 8; ++t) v[t] = make_double2(fma(v[t].x, u0, 0.0), -fma(-v[t].y, u1, 0.0));
+            if (bad0 || bad1) {
 #pragma unroll 1
                 for (int k = 0; k < np; ++k) {
                     const double a = bad0 ? (double)weighted_sample<MODE>(P, src0, pw0, xi0, k) : 0.0;

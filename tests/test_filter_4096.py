@@ -71,3 +71,35 @@ def test_a_row_keeps_its_infinities_to_itself(ctx, oracle, bins):
             for i in (1, 2, 6):
                 assert np.array_equal(np.isnan(got[i]), np.isnan(want[i])), (name, i)
                 assert np.array_equal(got[i][~np.isnan(got[i])], want[i][~np.isnan(want[i])].astype(np.float32)), (name, i)
+
+
+@pytest.mark.parametrize("bins", [1025, 1500, 2048])
+@pytest.mark.parametrize("filt", [0, 1])
+def test_a_row_keeps_its_rounding_to_itself(ctx, oracle, bins, filt):
+    """Rows of every size from 1e-30 to 1e30 and rows of zeros side by side: each is
+    held to the suite's bound by its own size, and zeros come out as zeros."""
+    import ctr
+    rng = np.random.default_rng(bins)
+    t = (0.05 * (np.arange(bins) - 0.5 * (bins - 1))).astype(np.float32).astype(np.float64)
+    beta = np.deg2rad(np.arange(1, 10) * 40.0)
+    sizes = np.array([1.0, 1e30, 1e-30, 0.0, 0.0, 3e4, 1e12, 1.0, 1e-20], np.float32)
+    y = sizes[:, None] * rng.random((9, bins)).astype(np.float32)
+    y[7, bins // 3:] = 0.0
+    three = (8, 8, 4, (8.0, 8.0, 4.0), 1000.0, beta[:3].astype(np.float32), t.astype(np.float32),
+             np.array([-0.5, 0.0, 0.5], np.float32))
+    forms = {
+        "parallel": (ctr.ParGeom, oracle.Par, (8, 8, (8.0, 8.0), beta, t), ctx.par_filter, oracle.par_filter),
+        "fan": (ctr.FanGeom, oracle.Fan, (8, 8, (8.0, 8.0), 1000.0, beta, t), ctx.fan_filter, oracle.fan_filter),
+        "cone": (ctr.ConeGeom, oracle.Cone, three, ctx.cone_filter, oracle.cone_filter),
+    }
+    for name, (G, O, a, run, ref) in forms.items():
+        print(f"[case] {name} {bins} filter {filt}", flush=True)
+        got = np.asarray(run(G(*a), y.ravel(), filt=filt)).reshape(9, bins)
+        want = np.asarray(ref(O(*a), y.ravel(), filt=filt)).reshape(9, bins)
+        for i, size in enumerate(sizes):
+            if size == 0.0:
+                assert not got[i].any() and not np.signbit(got[i]).any()
+                continue
+            e, m = errs(got[i].astype(np.float64) / size, want[i].astype(np.float64) / size)
+            report(f"rows of {size}[{name},{bins},f={filt}]", rel_l2=e, max_rel=m)
+            assert e < 1e-6 and m < 1e-5
