@@ -62,6 +62,7 @@ struct FanTables {
     uint64_t adj_key = 0;
     std::vector<int> h_lut;
     double lut_lo = 0, lut_scale = 0;
+    bool has_rays = false;
     DevBuf d_lut, d_rays;
 };
 
@@ -140,7 +141,7 @@ struct ctr_ctx {
     // it for the operator with this key; reserve_vinv clears the key whenever
     // the buffer may be reallocated, and sirt_norm sets it once V is written
     uint64_t vinv_key = 0;
-    int fault = 0;   // CTR_FAULT test hook: 1 alloc, 2 launch, 3 copy
+    int fault = 0;   // CTR_FAULT test hook: 1 alloc, 2 launch, 3 copy, 4 spare (buf_spare)
     // device address of the library's fixed scratch array on this device
     // (the allocation-free filter's tables), looked up at creation
     void *scratch = nullptr;
@@ -190,13 +191,13 @@ int parse_fault()
     if (!strcmp(f, "alloc")) return 1;
     if (!strcmp(f, "launch")) return 2;
     if (!strcmp(f, "copy")) return 3;
+    if (!strcmp(f, "spare")) return 4;
     return 0;
 }
 
-ctr_status buf_reserve(ctr_ctx *ctx, DevBuf &b, size_t bytes)
+hipError_t buf_grow(ctr_ctx *ctx, DevBuf &b, size_t bytes)
 {
-    if (ctx->fault == 1) return fail(ctx, CTR_EFAULT_INJECTED, "CTR_FAULT=alloc: device allocation of %zu bytes", bytes);
-    if (bytes <= b.bytes && b.ptr) return CTR_OK;
+    if (bytes <= b.bytes && b.ptr) return hipSuccess;
     if (b.ptr) {
         // the old buffer may still be read by queued work
         (void)hipStreamSynchronize(ctx->stream);
@@ -208,11 +209,34 @@ ctr_status buf_reserve(ctr_ctx *ctx, DevBuf &b, size_t bytes)
     hipError_t e = hipMalloc(&p, bytes ? bytes : 16);
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        return fail(ctx, CTR_ENOMEM, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
+        return e;
     }
     b.ptr = p;
     b.bytes = bytes;
+    return hipSuccess;
+}
+
+ctr_status buf_reserve(ctr_ctx *ctx, DevBuf &b, size_t bytes)
+{
+    if (ctx->fault == 1) return fail(ctx, CTR_EFAULT_INJECTED, "CTR_FAULT=alloc: device allocation of %zu bytes", bytes);
+    const hipError_t e = buf_grow(ctx, b, bytes);
+    if (e != hipSuccess) return fail(ctx, CTR_ENOMEM, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
     return CTR_OK;
+}
+
+// Room for a path that is only the faster one: false, and no error, where the
+// device has none left, or while the stream is captured, when nothing can be
+// allocated.  The caller then takes the path without it.
+bool buf_spare(ctr_ctx *ctx, DevBuf &b, size_t bytes)
+{
+    if (ctx->fault == 1 || ctx->fault == 4) return false;
+    if (bytes <= b.bytes && b.ptr) return true;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return buf_grow(ctx, b, bytes) == hipSuccess;
 }
 
 // The workspace of SIRT's V: a reallocation (even one that fails, or that
@@ -609,9 +633,8 @@ ctr_status fp_transposed(ctr_ctx *ctx, RayParams &R, const float *vol, DevBuf &b
 {
     R.volT = nullptr;
     ColumnPlan L;
-    if (row_pitch > 0.0 && column_plan(R, row_pitch, L)) {
-        TRY(buf_reserve(ctx, buf, L.vol_bytes));
-        TRY(buf_reserve(ctx, ctx->ws[kWsCells], L.list_bytes));
+    if (row_pitch > 0.0 && column_plan(R, row_pitch, L) && buf_spare(ctx, buf, L.vol_bytes) &&
+        buf_spare(ctx, ctx->ws[kWsCells], L.list_bytes)) {
         TRY(check_launch(ctx, launch_z_fastest(vol, (float *)buf.ptr, R.nt, R.ns, R.nz, st), "volume transpose"));
         column_bind(R, L, (float *)buf.ptr, ctx->ws[kWsCells].ptr);
         return CTR_OK;
@@ -768,8 +791,8 @@ FanParams fan_params(ctr_ctx *ctx, const ctr_fan_geom *g, unsigned flags)
 
 // Tables of the exact fan adjoint, once per geometry: the bin index (first bin
 // at or above each of 4 n_p positions over the detector) and the ray records.
-// Records take 16 bytes per ray; beyond 2^26 rays (1 GiB) the kernel forms them
-// as it goes.
+// Records take 16 bytes per ray; beyond 2^26 rays (1 GiB), or without the memory
+// for them, the kernel forms them as it goes.
 ctr_status fan_adjoint_tables(ctr_ctx *ctx, const ctr_fan_geom *g, FanParams &P)
 {
     FanTables &T = ctx->fan;
@@ -795,8 +818,8 @@ ctr_status fan_adjoint_tables(ctr_ctx *ctx, const ctr_fan_geom *g, FanParams &P)
             T.h_lut[k] = c;
         }
         TRY(upload(ctx, T.d_lut, T.h_lut.data(), sizeof(int) * T.h_lut.size()));
-        if (table) {
-            TRY(buf_reserve(ctx, T.d_rays, nray * sizeof(double2)));
+        T.has_rays = table && buf_spare(ctx, T.d_rays, nray * sizeof(double2));
+        if (T.has_rays) {
             TRY(check_launch(ctx, launch_fan_ray_table(P, (double2 *)T.d_rays.ptr, ctx->stream), "fan ray records"));
         }
         T.adj_key = T.key;
@@ -805,7 +828,7 @@ ctr_status fan_adjoint_tables(ctr_ctx *ctx, const ctr_fan_geom *g, FanParams &P)
     P.lut_scale = (float)T.lut_scale;
     P.lut_eps = (float)(1e-3 + 1e-6 * (hi - lo));
     P.lut = (const int *)T.d_lut.ptr;
-    if (table) P.rays = (const double2 *)T.d_rays.ptr;
+    if (T.has_rays) P.rays = (const double2 *)T.d_rays.ptr;
     return CTR_OK;
 }
 
@@ -1512,13 +1535,19 @@ ctr_status ctr_cone_fp(ctr_ctx *ctx, const ctr_cone_geom *g, const float *vol, f
     return finish_out(ctx, dev, dp, proj, nray3(g));
 }
 
+// Partial volumes of the backprojections that split their views over sets of
+// blocks; null for one set, or where there is no room for them.
+static float *part_volumes(ctr_ctx *ctx, int splits, size_t nvox)
+{
+    DevBuf &b = ctx->ws[kWsBpParts];
+    return splits > 1 && buf_spare(ctx, b, sizeof(float) * splits * nvox) ? (float *)b.ptr : nullptr;
+}
+
 static ctr_status bp_tiled(ctr_ctx *ctx, int kind, const BpParams &P, const float *src, float *vol, const char *what)
 {
     const BpPlan &L = ctx->foot_bp.plan;
-    const int splits = bp_splits(kind, P, L);
-    if (splits > 1) TRY(buf_reserve(ctx, ctx->ws[kWsBpParts], sizeof(float) * splits * P.nt * P.ns * P.nz));
-    return check_launch(ctx, launch_bp_tiled(kind, P, L, (const int4 *)ctx->foot_bp.buf.ptr, src, vol,
-                                             splits > 1 ? (float *)ctx->ws[kWsBpParts].ptr : nullptr, ctx->stream),
+    float *parts = part_volumes(ctx, bp_splits(kind, P, L), (size_t)P.nt * P.ns * P.nz);
+    return check_launch(ctx, launch_bp_tiled(kind, P, L, (const int4 *)ctx->foot_bp.buf.ptr, src, vol, parts, ctx->stream),
                         what);
 }
 
@@ -1558,14 +1587,9 @@ ctr_status ctr_cone_bp_adjoint(ctr_ctx *ctx, const ctr_cone_geom *g, const float
     TRY(check_launch(ctx, launch_scale_by_norm(P, dp, yn, ctx->stream), "adjoint input scaling"));
     const BpPlan &L = ctx->foot_adj.plan;
     const int4 *foot = (const int4 *)ctx->foot_adj.buf.ptr;
-    const int splits = adjoint_splits(L, P.nb);
-    if (splits > 1) {
-        TRY(buf_reserve(ctx, ctx->ws[kWsBpParts], sizeof(float) * splits * nvox3(g)));
-        TRY(check_launch(ctx, launch_adjoint_split(P, L, foot, yn, dv, (float *)ctx->ws[kWsBpParts].ptr, ctx->stream),
-                         "cone adjoint"));
-    } else {
-        TRY(check_launch(ctx, launch_adjoint(P, L, foot, yn, dv, nullptr, 0, ctx->stream), "cone adjoint"));
-    }
+    float *parts = part_volumes(ctx, adjoint_splits(L, P.nb), nvox3(g));
+    TRY(check_launch(ctx, parts ? launch_adjoint_split(P, L, foot, yn, dv, parts, ctx->stream)
+                                : launch_adjoint(P, L, foot, yn, dv, nullptr, 0, ctx->stream), "cone adjoint"));
     return finish_out(ctx, dev, dv, vol, nvox3(g));
 }
 
@@ -1848,9 +1872,7 @@ ctr_status ctr_curved_filter(ctr_ctx *ctx, const ctr_curved_geom *g, const float
 
 static ctr_status curved_bp(ctr_ctx *ctx, const CurvedBpParams &P, const float *src, float *vol)
 {
-    const int splits = curved_splits(P);
-    if (splits > 1) TRY(buf_reserve(ctx, ctx->ws[kWsBpParts], sizeof(float) * splits * P.nt * P.ns * P.nz));
-    float *parts = splits > 1 ? (float *)ctx->ws[kWsBpParts].ptr : nullptr;
+    float *parts = part_volumes(ctx, curved_splits(P), (size_t)P.nt * P.ns * P.nz);
     return check_launch(ctx, launch_curved_bp(P, src, vol, parts, ctx->stream), "curved-detector backprojection");
 }
 
