@@ -58,12 +58,14 @@ struct FanTables {
     std::vector<double> h_view, h_p, h_zero;
     std::vector<float> h_pf, h_gam, h_colw, h_xf;
     DevBuf d_view, d_p, d_zero, d_pf, d_gam, d_colw, d_xf;
-    // exact adjoint, built on its first use: bin index over the detector, ray records
-    uint64_t adj_key = 0;
-    std::vector<int> h_lut;
+    // exact adjoint: bin index over the detector (lut_n + 1 ints after the positions
+    // in d_pf), ray records
+    int asc = 1, lut_n = 0;
     double lut_lo = 0, lut_scale = 0;
+    float lut_eps = 0;
+    uint64_t rays_key = 0;
     bool has_rays = false;
-    DevBuf d_lut, d_rays;
+    DevBuf d_rays;
 };
 
 struct ParTables {
@@ -224,19 +226,23 @@ ctr_status buf_reserve(ctr_ctx *ctx, DevBuf &b, size_t bytes)
     return CTR_OK;
 }
 
+// Whether the context's stream is captured: nothing can be allocated or waited for.
+bool capturing(const ctr_ctx *ctx)
+{
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 // Room for a path that is only the faster one: false, and no error, where the
-// device has none left, or while the stream is captured, when nothing can be
-// allocated.  The caller then takes the path without it.
+// device has none left, or while the stream is captured.  The caller then takes
+// the path without it.
 bool buf_spare(ctr_ctx *ctx, DevBuf &b, size_t bytes)
 {
     if (ctx->fault == 1 || ctx->fault == 4) return false;
     if (bytes <= b.bytes && b.ptr) return true;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return buf_grow(ctx, b, bytes) == hipSuccess;
+    return !capturing(ctx) && buf_grow(ctx, b, bytes) == hipSuccess;
 }
 
 // The workspace of SIRT's V: a reallocation (even one that fails, or that
@@ -710,11 +716,28 @@ ctr_status fan_tables(ctr_ctx *ctx, const ctr_fan_geom *g)
         T.h_colw[i] = (float)(D * std::cos(gam));
     }
     T.h_xf.assign(1, 0.0f);
+    // the adjoint's bin index: first bin, in ascending position, at or above each
+    // of 4 n_p positions over the detector
+    T.asc = g->p[np - 1] >= g->p[0];
+    const double lo = T.asc ? g->p[0] : g->p[np - 1], hi = T.asc ? g->p[np - 1] : g->p[0];
+    T.lut_n = (int)std::min(4 * (size_t)np, (size_t)1 << 16);
+    T.lut_lo = (double)(float)lo;
+    T.lut_scale = (double)(float)(1.0 / (hi > lo ? (hi - lo) / T.lut_n : 1.0));
+    T.lut_eps = (float)(1e-3 + 1e-6 * (hi - lo));
+    T.h_pf.resize((size_t)np + T.lut_n + 1);
+    const double *first = T.asc ? g->p : g->p + (np - 1), cell = 1.0 / T.lut_scale;
+    const std::ptrdiff_t step = T.asc ? 1 : -1;
+    for (int k = 0, c = 0; k <= T.lut_n; ++k) {
+        const double edge = T.lut_lo + k * cell;
+        if (k == T.lut_n) c = np;
+        else while (k > 0 && c < np && first[c * step] < edge) ++c;
+        std::memcpy(&T.h_pf[(size_t)np + k], &c, sizeof c);
+    }
     ctr_status s;
     if ((s = upload(ctx, T.d_view, T.h_view.data(), sizeof(double) * T.h_view.size())) != CTR_OK) return s;
     if ((s = upload(ctx, T.d_p, T.h_p.data(), sizeof(double) * np)) != CTR_OK) return s;
     if ((s = upload(ctx, T.d_zero, T.h_zero.data(), sizeof(double))) != CTR_OK) return s;
-    if ((s = upload(ctx, T.d_pf, T.h_pf.data(), sizeof(float) * np)) != CTR_OK) return s;
+    if ((s = upload(ctx, T.d_pf, T.h_pf.data(), sizeof(float) * T.h_pf.size())) != CTR_OK) return s;
     if ((s = upload(ctx, T.d_gam, T.h_gam.data(), sizeof(float) * np)) != CTR_OK) return s;
     if ((s = upload(ctx, T.d_colw, T.h_colw.data(), sizeof(float) * np)) != CTR_OK) return s;
     if ((s = upload(ctx, T.d_xf, T.h_xf.data(), sizeof(float))) != CTR_OK) return s;
@@ -789,46 +812,28 @@ FanParams fan_params(ctr_ctx *ctx, const ctr_fan_geom *g, unsigned flags)
     return P;
 }
 
-// Tables of the exact fan adjoint, once per geometry: the bin index (first bin
-// at or above each of 4 n_p positions over the detector) and the ray records.
-// Records take 16 bytes per ray; beyond 2^26 rays (1 GiB), or without the memory
-// for them, the kernel forms them as it goes.
+// The exact fan adjoint's tables: the bin index of the geometry (fan_tables) and
+// the ray records, formed on the first use.  Records take 16 bytes per ray;
+// beyond 2^26 rays (1 GiB), without the memory for them, or in a captured call
+// that nothing formed them for, the kernel forms them as it goes.
 ctr_status fan_adjoint_tables(ctr_ctx *ctx, const ctr_fan_geom *g, FanParams &P)
 {
     FanTables &T = ctx->fan;
-    const int np = g->n_p;
-    const bool asc = g->p[np - 1] >= g->p[0];
-    const size_t nray = (size_t)g->n_beta * np;
-    const bool table = nray <= ((size_t)1 << 26);
-    const double lo = asc ? g->p[0] : g->p[np - 1], hi = asc ? g->p[np - 1] : g->p[0];
-    const int cells = std::min(4 * (size_t)np, (size_t)1 << 16);
-    P.asc = asc;
-    P.lut_n = cells;
-    if (T.adj_key != T.key || !T.d_lut.ptr) {
-        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));   // queued work may still read the old tables
-        T.adj_key = 0;
-        const double h = hi > lo ? (hi - lo) / cells : 1.0;
-        T.lut_lo = (double)(float)lo;
-        T.lut_scale = (double)(float)(1.0 / h);
-        T.h_lut.resize((size_t)cells + 1);
-        int c = 0;
-        for (int k = 0; k <= cells; ++k) {
-            const double edge = k == cells ? std::numeric_limits<double>::infinity() : T.lut_lo + k / T.lut_scale;
-            while (k > 0 && c < np && (asc ? g->p[c] : g->p[np - 1 - c]) < edge) ++c;
-            T.h_lut[k] = c;
-        }
-        TRY(upload(ctx, T.d_lut, T.h_lut.data(), sizeof(int) * T.h_lut.size()));
-        T.has_rays = table && buf_spare(ctx, T.d_rays, nray * sizeof(double2));
-        if (T.has_rays) {
+    const size_t nray = (size_t)g->n_beta * g->n_p;
+    if (T.rays_key != T.key && nray <= ((size_t)1 << 26) && !capturing(ctx)) {
+        T.rays_key = 0;
+        T.has_rays = buf_spare(ctx, T.d_rays, nray * sizeof(double2));
+        if (T.has_rays)
             TRY(check_launch(ctx, launch_fan_ray_table(P, (double2 *)T.d_rays.ptr, ctx->stream), "fan ray records"));
-        }
-        T.adj_key = T.key;
+        T.rays_key = T.key;
     }
+    if (T.rays_key == T.key && T.has_rays) P.rays = (const double2 *)T.d_rays.ptr;
+    P.asc = T.asc;
+    P.lut_n = T.lut_n;
     P.lut_lo = (float)T.lut_lo;
     P.lut_scale = (float)T.lut_scale;
-    P.lut_eps = (float)(1e-3 + 1e-6 * (hi - lo));
-    P.lut = (const int *)T.d_lut.ptr;
-    if (T.has_rays) P.rays = (const double2 *)T.d_rays.ptr;
+    P.lut_eps = T.lut_eps;
+    P.lut = reinterpret_cast<const int *>((const float *)T.d_pf.ptr + g->n_p);
     return CTR_OK;
 }
 
@@ -1442,7 +1447,7 @@ void ctr_ctx_destroy(ctr_ctx *ctx)
     for (auto &b : ctx->ws) buf_free(b);
     for (DevBuf *b : {&ctx->cone.d_view, &ctx->cone.d_p, &ctx->cone.d_xi, &ctx->cone.d_bp, &ctx->cone.d_pf,
                       &ctx->cone.d_xf, &ctx->cone.d_zq, &ctx->fan.d_view, &ctx->fan.d_p, &ctx->fan.d_zero, &ctx->fan.d_pf,
-                      &ctx->fan.d_gam, &ctx->fan.d_colw, &ctx->fan.d_xf, &ctx->fan.d_lut,
+                      &ctx->fan.d_gam, &ctx->fan.d_colw, &ctx->fan.d_xf,
                       &ctx->fan.d_rays, &ctx->taps.d, &ctx->taps.d_spec, &ctx->foot_bp.buf, &ctx->foot_adj.buf})
         buf_free(*b);
     if (ctx->own) (void)hipStreamDestroy(ctx->own);

@@ -105,3 +105,29 @@ def test_fan_adjoint_ignores_samples_it_does_not_meet(ctx):
     b = ctx.fan_bp_adjoint(g, y)
     assert hit.any() and not hit.all()
     assert np.all(np.isinf(b[hit])) and np.array_equal(b[~hit], a[~hit])
+
+
+def test_fan_adjoint_captured_before_its_first_use(ctx):
+    """A geometry that only the projector has seen: the captured adjoint allocates
+    and waits for nothing, and replays give the eager call's bits, also after the
+    eager call has formed the ray records."""
+    import ctr
+    import torch
+    g = ctr.FanGeom(40, 36, (40.0, 36.0), 90.0, 2 * np.pi / 31 * np.arange(31), 0.7 * (np.arange(81) - 40.2))
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        y = ctx.fan_fp(g, torch.rand(g.nvox, device="cuda"))
+        out = torch.empty(g.nvox, device="cuda")
+        stream.synchronize()
+        print("[case] capture", flush=True)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            ctx.fan_bp_adjoint(g, y, out=out)
+        for _ in range(3):
+            y.copy_(torch.rand(g.nray, device="cuda"))
+            out.fill_(float("nan"))
+            graph.replay()
+            got = out.clone()
+            assert torch.equal(got, ctx.fan_bp_adjoint(g, y))
+    torch.cuda.synchronize()
+    ctx.fan_bp_adjoint(g, np.ones(g.nray, np.float32))
