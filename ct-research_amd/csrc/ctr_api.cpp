@@ -1556,6 +1556,16 @@ static ctr_status bp_tiled(ctr_ctx *ctx, int kind, const BpParams &P, const floa
                         what);
 }
 
+// src: the projections times the ray norms
+static ctr_status adjoint_tiled(ctr_ctx *ctx, const BpParams &P, const float *src, float *vol)
+{
+    const BpPlan &L = ctx->foot_adj.plan;
+    const int4 *foot = (const int4 *)ctx->foot_adj.buf.ptr;
+    float *parts = part_volumes(ctx, adjoint_splits(L, P.nb), (size_t)P.nt * P.ns * P.nz);
+    return check_launch(ctx, parts ? launch_adjoint_split(P, L, foot, src, vol, parts, ctx->stream)
+                                   : launch_adjoint(P, L, foot, src, vol, nullptr, 0, ctx->stream), "cone adjoint");
+}
+
 ctr_status ctr_cone_bp_ref(ctr_ctx *ctx, const ctr_cone_geom *g, const float *proj, float *vol, unsigned flags)
 {
     TRY(check_cone(g, 1));
@@ -1590,11 +1600,7 @@ ctr_status ctr_cone_bp_adjoint(ctr_ctx *ctx, const ctr_cone_geom *g, const float
     TRY(buf_reserve(ctx, ctx->ws[kWsYn], nray3(g) * sizeof(float)));
     float *yn = (float *)ctx->ws[kWsYn].ptr;
     TRY(check_launch(ctx, launch_scale_by_norm(P, dp, yn, ctx->stream), "adjoint input scaling"));
-    const BpPlan &L = ctx->foot_adj.plan;
-    const int4 *foot = (const int4 *)ctx->foot_adj.buf.ptr;
-    float *parts = part_volumes(ctx, adjoint_splits(L, P.nb), nvox3(g));
-    TRY(check_launch(ctx, parts ? launch_adjoint_split(P, L, foot, yn, dv, parts, ctx->stream)
-                                : launch_adjoint(P, L, foot, yn, dv, nullptr, 0, ctx->stream), "cone adjoint"));
+    TRY(adjoint_tiled(ctx, P, yn, dv));
     return finish_out(ctx, dev, dv, vol, nvox3(g));
 }
 
@@ -3345,10 +3351,7 @@ ctr_status ctr_autotune_cone(ctr_ctx *ctx, const ctr_cone_geom *g, ctr_tune_resu
         t.bp_pitch = pitches[i];
         ctx->tune[key] = t;
         TRY(ensure_footprints(ctx, P, ctx->foot_bp, false));
-        TRY(timed([&]() {
-            return check_launch(ctx, launch_bp_tiled(kBpFdk, P, ctx->foot_bp.plan, (const int4 *)ctx->foot_bp.buf.ptr,
-                                                     proj, dst, nullptr, st), "FDK backprojection");
-        }, &res.bp_ms[i]));
+        TRY(timed([&]() { return bp_tiled(ctx, kBpFdk, P, proj, dst, "FDK backprojection"); }, &res.bp_ms[i]));
         if (res.bp_ms[i] < bestv) {
             bestv = res.bp_ms[i];
             res.bp_pitch = pitches[i];
@@ -3361,16 +3364,15 @@ ctr_status ctr_autotune_cone(ctr_ctx *ctx, const ctr_cone_geom *g, ctr_tune_resu
         t.adj_cm = cms[i];
         ctx->tune[key] = t;
         TRY(ensure_footprints(ctx, P, ctx->foot_adj, true));
-        TRY(timed([&]() {
-            return check_launch(ctx, launch_adjoint(P, ctx->foot_adj.plan, (const int4 *)ctx->foot_adj.buf.ptr, proj,
-                                                    dst, nullptr, 0, st), "adjoint");
-        }, &res.adj_ms[i]));
+        TRY(timed([&]() { return adjoint_tiled(ctx, P, proj, dst); }, &res.adj_ms[i]));
         if (res.adj_ms[i] < bestv) {
             bestv = res.adj_ms[i];
             res.adj_cm = cms[i];
         }
     }
     best.adj_cm = res.adj_cm;
+    // the slab walk's layout: SIRT's residual pass is the slab walk where the
+    // projection goes by detector columns, too
     for (int i = 0; i < 2; ++i) {
         TRY(timed([&]() {
             RayParams R = cone_ray_params(ctx, g);

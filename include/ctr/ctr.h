@@ -357,9 +357,10 @@ typedef struct ctr_tune_result {
     int bp_pitch;           /* chosen row pitch (floats) of the FDK / BP_REF footprint buffers */
     int adj_cm;             /* chosen candidate-column chunk of the exact adjoint */
     int fp_transpose;       /* 1: views along t read a [z][t][s] copy of the volume */
-    double bp_ms[3];        /* FDK backprojection, pitch 64 / 72 / 80 */
-    double adj_ms[3];       /* exact adjoint, chunk 3 / 4 / 6 */
-    double fp_ms[2];        /* forward projection, without / with the transposed copy */
+    double bp_ms[3];        /* FDK backprojection as ctr_fdk_bp runs it, pitch 64 / 72 / 80 */
+    double adj_ms[3];       /* exact adjoint as ctr_cone_bp_adjoint runs it, chunk 3 / 4 / 6 */
+    double fp_ms[2];        /* slab walk without / with the transposed copy: SIRT's residual pass, and
+                               ctr_cone_fp where it does not go by detector columns */
 } ctr_tune_result;
 
 ctr_status ctr_autotune_cone(ctr_ctx *ctx, const ctr_cone_geom *g, ctr_tune_result *out);

@@ -96,3 +96,28 @@ def test_calls_do_without_the_memory_of_their_faster_paths(ctx, bare, monkeypatc
         assert np.linalg.norm(a - b) < 2e-6 * np.linalg.norm(a), name
         if name != "fan_bp_adjoint":   # formed as they go, the records have the same bits
             assert not np.array_equal(a, b), name   # the other path it is
+
+def test_autotuner_times_what_the_calls_run(ctx):
+    """A small volume with many views: the calls split the views over sets of blocks
+    (an eighth of the time of one set), and so do the autotuner's runs: its best is
+    below twice the time of the whole call."""
+    import torch
+    g = ctr.geometry.cone_circular(32, 1.0, 120, 64, 64, 1.0, 150.0, 300.0)
+    proj, vol = torch.rand(g.nray, device="cuda"), torch.empty(g.nvox, device="cuda")
+    tuned = ctr.Context(0)
+    try:
+        r = tuned.autotune_cone(g)
+        for name, call in (("bp_ms", tuned.fdk_bp), ("adj_ms", tuned.cone_bp_adjoint)):
+            ms = []
+            for _ in range(8):
+                a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                a.record()
+                call(g, proj, out=vol)
+                b.record()
+                torch.cuda.synchronize()
+                ms.append(a.elapsed_time(b))
+            t = float(np.median(ms))
+            print(f"[case] {name} {r[name]} call {t}", flush=True)
+            assert min(r[name]) < 2 * t
+    finally:
+        tuned.close()
