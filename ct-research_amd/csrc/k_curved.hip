@@ -298,17 +298,27 @@ int cv_rows(const CurvedBpParams &P, int tz)
     return most;
 }
 
+// Blocks that the chip holds at a time (five of 32 KiB of LDS per CU).
+constexpr long kCvBlocks = 1280;
+
 // z depth of a tile: the per-view column set-up (about 55 instructions) is
 // shared by the tile's slices (about 15 each; 45 where the footprints exceed
-// LDS); slices past nz are wasted work
+// LDS); slices past nz are wasted work.  More than 8 slices only where tiles and
+// sets of views still fill the chip: of few views a block's time is what counts
+// (258 x 121 x 56, 12 views: 31 us with 8 slices, 36 us with 20; 117 x 4 x 46, 7
+// views: 17 and 25 us).
 int choose_tz(const CurvedBpParams &P)
 {
     static const int cand[] = {4, 6, 8, 10, 12, 16, 20, 25, 32};
-    int best = 10;
+    const long columns = (long)((P.nt + kCvTX - 1) / kCvTX) * ((P.ns + kCvTS - 1) / kCvTS);
+    int best = 8;
     long best_cost = -1;
     for (int tz : cand) {
+        const long tiles_z = (P.nz + tz - 1) / tz, tiles = columns * tiles_z;
+        const int share = bp_share(tiles, P.nb, (size_t)P.nt * P.ns * P.nz);
+        if (tz > 8 && tiles * ((P.nb + share - 1) / share) < kCvBlocks) continue;
         const long each = cv_rows(P, tz) * kCvNarrow <= kCvCap ? 15 : 45;
-        const long cost = (long)((P.nz + tz - 1) / tz) * (55 + each * tz);
+        const long cost = tiles_z * (55 + each * tz);
         if (best_cost < 0 || cost < best_cost) {
             best = tz;
             best_cost = cost;
