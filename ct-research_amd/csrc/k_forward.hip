@@ -1032,7 +1032,8 @@ __device__ __forceinline__ float trace_column(const RayParams &g, const ColumnHe
     if (h.n == 0) return 0.0f;
     const double slope = g.xi[valid ? ix : g.nx - 1] * h.inv_rho;   // z per in-plane length
     // first slice, next plane and the step between planes
-    const double inv_rz = 1.0 / g.rz, zin = (g.sz + h.lo * slope) * inv_rz;
+    // (divided as in setup_axis: a level ray between two slices takes the same one)
+    const double zin = (g.sz + h.lo * slope) / g.rz;
     const double k0 = slope < 0.0 ? ceil(zin) - 1.0 : floor(zin);
     double z0 = __builtin_huge_val(), dz = 0.0, out = __builtin_huge_val();
     if (slope != 0.0) {
@@ -1096,7 +1097,7 @@ __device__ __forceinline__ float trace_column(const RayParams &g, const ColumnHe
         const float r0 = fabsf(s0) * reach, r1 = fabsf(s1) * reach, outer = fmaxf(r0, r1);
         const float fan = s0 * s1 < 0.0f ? fminf(r0, half) + fminf(r1, half)
                                          : fabsf(s1 - s0) * reach * (outer > half ? half / outer : 1.0f);
-        const float wide = 4.0f * (fan * (float)inv_rz) + 36.0f;
+        const float wide = 4.0f * (fan / (float)g.rz) + 36.0f;
         const bool narrow = wide <= 4.0f * 63.0f, gentle = __ballot(dZ != 0.0f && dZ < h.block) == 0;
         const ColumnLane lane{Z0, dZ, zb, sgn};
         if (gentle)

@@ -176,3 +176,21 @@ def test_a_voxel_that_is_not_finite(ctx, columns, case, bad):
         assert np.array_equal(got[hit], np.full(hit.sum(), bad, np.float32), equal_nan=True)
         crossed += hit.sum()
     assert crossed
+
+
+@pytest.mark.parametrize("depth", [18.400000000000002, 31.2, 36.800000000000004, 80.0])
+def test_level_rays_between_two_slices(ctx, oracle, columns, depth):
+    """The middle one of an odd number of rows runs along the plane between the two
+    middle slices: it takes the upper one, as in the slab walk and the matrix, also
+    where depth / 2 times the reciprocal of the slice height rounds below it."""
+    import ctr
+    beta = (2 * np.pi / 5 * np.arange(5) + 0.1).astype(np.float32)
+    p = (0.9 * (np.arange(30) - 14.5) + 0.03).astype(np.float32)
+    xi = (0.31 * (np.arange(65) - 32)).astype(np.float32)
+    a = (24, 20, 80, (24.0, 20.0, depth), 70.0, beta, p, xi)
+    g, og = ctr.ConeGeom(*a), oracle.Cone(*a)
+    vol = np.random.default_rng(6).random(g.nvox).astype(np.float32)
+    print(f"[case] columns, level rays, 80 slices in {depth} mm", flush=True)
+    e, m = errs(ctx.cone_fp(g, vol), oracle.cone_fp_exact(og, vol))
+    report(f"columns_level[{depth}]", rel_l2=e, max_rel=m)
+    assert e < 2e-6 and m < 2e-5
