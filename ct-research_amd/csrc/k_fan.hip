@@ -141,7 +141,7 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-constexpr int kFanWaves = 8;     // views of a round: one per wave of the block
+constexpr int kFanWaves = 8;     // views of a round, at most: one per wave of the block
 constexpr int kFanStage = 64;    // rays of a view staged per wave
 constexpr int kFanSlots = 6;     // lengths a pixel keeps per view (a pixel of two bins' width meets 5 at most)
 
@@ -165,15 +165,21 @@ constexpr int kFanSlots = 6;     // lengths a pixel keeps per view (a pixel of t
 // pixel, two binary searches per view and four FP64 divisions and a root per
 // ray; 200 us now, VALU issue (about 200 instructions per wave and view: 50 to
 // find the bins, 75 for the lengths, 35 to add).
-template <bool TABLE>
-__global__ __launch_bounds__(64 * kFanWaves, 8) void k_fan_adjoint(const float *__restrict__ proj, float *__restrict__ img,
-                                                                FanParams P, SirtUpdate U, int sirt, int ones)
+//
+// A block has W waves: as many as views, rounded up to a power of two, where that
+// is less than 8 (a single view or a few of an ordered subset: the others would
+// only hold room).  One view of 2048^2 pixels, 1024 bins: 51 us with one thread
+// per pixel, 109 us by blocks of 8 waves, 27 us by one; two views 89 / 127 / 49
+// us.
+template <bool TABLE, int W>
+__global__ __launch_bounds__(64 * W, 8) void k_fan_adjoint(const float *__restrict__ proj, float *__restrict__ img,
+                                                          FanParams P, SirtUpdate U, int sirt, int ones)
 {
-    __shared__ double2 rays[kFanWaves][kFanStage];
-    __shared__ float ys[2][kFanWaves][kFanStage];
-    __shared__ float slot[2][kFanWaves][kFanSlots][64];
-    __shared__ unsigned char first[2][kFanWaves][64];   // the pixel's first ray in ys
-    __shared__ int count[2][kFanWaves];   // slots in use, -1: a view for the adding wave
+    __shared__ double2 rays[W][kFanStage];
+    __shared__ float ys[2][W][kFanStage];
+    __shared__ float slot[2][W][kFanSlots][64];
+    __shared__ unsigned char first[2][W][64];   // the pixel's first ray in ys
+    __shared__ int count[2][W];   // slots in use, -1: a view for the adding wave
     __shared__ float sum[64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int i = blockIdx.x * 8 + (lane & 7), j = blockIdx.y * 8 + (lane >> 3);
@@ -227,7 +233,7 @@ __global__ __launch_bounds__(64 * kFanWaves, 8) void k_fan_adjoint(const float *
         const double2 ray = record(b, cl);
         const float yv = ones ? 1.0f : proj[(size_t)b * P.np + cl];
         const int rel = in ? c0 - cmin : 0, mine = in ? c1 - c0 : -1;
-        if (b + kFanWaves < P.nb) bins(b + kFanWaves, c0, c1);
+        if (b + W < P.nb) bins(b + W, c0, c1);
         if (!fits) return;
         rays[wave][lane] = ray;
         ys[h][wave][lane] = yv;
@@ -256,24 +262,24 @@ __global__ __launch_bounds__(64 * kFanWaves, 8) void k_fan_adjoint(const float *
     // a length of 0 adds nothing, whatever the sample holds
     auto add = [](float len, float yv, float acc) { return len != 0.0f ? fmaf(len, yv, acc) : acc; };
 
-    const int rounds = (P.nb + kFanWaves - 1) / kFanWaves;
+    const int rounds = (P.nb + W - 1) / W;
     if (wave < P.nb) {
         bins(wave, c0, c1);
         form(wave, 0);
     }
     for (int r = 0; r < rounds; ++r) {
-        const int h = r & 1, next = (r + 1) * kFanWaves + wave;
+        const int h = r & 1, next = (r + 1) * W + wave;
         __syncthreads();
-        if (r % kFanWaves == wave) {
+        if (r % W == wave) {
             float acc = sum[lane];
-            for (int w = 0; w < kFanWaves && r * kFanWaves + w < P.nb; ++w) {
+            for (int w = 0; w < W && r * W + w < P.nb; ++w) {
                 const int n = __builtin_amdgcn_readfirstlane(count[h][w]);
                 if (n >= 0) {
                     const int rel = first[h][w][lane];
                     for (int k = 0; k < n; ++k)
                         acc = add(slot[h][w][k][lane], ys[h][w][(rel + k) & (kFanStage - 1)], acc);
                 } else {
-                    const int b = r * kFanWaves + w;
+                    const int b = r * W + w;
                     int c0, c1;
                     bins(b, c0, c1);
                     const double st = P.view[4 * (size_t)b + 2], ss = P.view[4 * (size_t)b + 3];
@@ -467,6 +473,15 @@ hipError_t launch_fan_ray_table(const FanParams &P, double2 *rays, hipStream_t s
     return hipGetLastError();
 }
 
+template <int W>
+static void launch_fan_adjoint_waves(const FanParams &P, const float *proj, float *img, const SirtUpdate &U, int sirt,
+                                     int ones_input, hipStream_t st)
+{
+    const dim3 grid((P.nt + 7) / 8, (P.ns + 7) / 8), block(64 * W);
+    if (P.rays) hipLaunchKernelGGL((k_fan_adjoint<true, W>), grid, block, 0, st, proj, img, P, U, sirt, ones_input);
+    else hipLaunchKernelGGL((k_fan_adjoint<false, W>), grid, block, 0, st, proj, img, P, U, sirt, ones_input);
+}
+
 hipError_t launch_fan_adjoint(const FanParams &P, const float *proj, float *img, const SirtUpdate *upd, int ones_input,
                               hipStream_t st)
 {
@@ -476,9 +491,10 @@ hipError_t launch_fan_adjoint(const FanParams &P, const float *proj, float *img,
         U = *upd;
         sirt = 1;
     }
-    const dim3 grid((P.nt + 7) / 8, (P.ns + 7) / 8), block(64 * kFanWaves);
-    if (P.rays) hipLaunchKernelGGL((k_fan_adjoint<true>), grid, block, 0, st, proj, img, P, U, sirt, ones_input);
-    else hipLaunchKernelGGL((k_fan_adjoint<false>), grid, block, 0, st, proj, img, P, U, sirt, ones_input);
+    if (P.nb > 4) launch_fan_adjoint_waves<kFanWaves>(P, proj, img, U, sirt, ones_input, st);
+    else if (P.nb > 2) launch_fan_adjoint_waves<4>(P, proj, img, U, sirt, ones_input, st);
+    else if (P.nb > 1) launch_fan_adjoint_waves<2>(P, proj, img, U, sirt, ones_input, st);
+    else launch_fan_adjoint_waves<1>(P, proj, img, U, sirt, ones_input, st);
     return hipGetLastError();
 }
 

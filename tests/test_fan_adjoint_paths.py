@@ -131,3 +131,18 @@ def test_fan_adjoint_captured_before_its_first_use(ctx):
             assert torch.equal(got, ctx.fan_bp_adjoint(g, y))
     torch.cuda.synchronize()
     ctx.fan_bp_adjoint(g, np.ones(g.nray, np.float32))
+
+
+@pytest.mark.parametrize("views", [1, 2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("name", ["base", "many_per_pixel", "descending"])
+def test_fan_adjoint_of_few_views(ctx, oracle, name, views):
+    """Blocks of as many waves as views, and the first rounds of whole blocks."""
+    import ctr
+    d = geometry(name)
+    args = (33, 9, (33.0, 9.0), d["D"], 0.4 + 2 * np.pi / views * np.arange(views), d["p"])
+    g, og = ctr.FanGeom(*args), oracle.Fan(*args)
+    y = np.random.default_rng(views).random(g.nray).astype(np.float32)
+    print(f"[case] fan adjoint {name}, {views} views", flush=True)
+    e, m = errs(ctx.fan_bp_adjoint(g, y), oracle.fan_adjoint(og, y))
+    report(f"fan_adjoint[{name},{views} views]", rel_l2=e, max_rel=m)
+    assert e < 1e-5 and m < 1e-5
