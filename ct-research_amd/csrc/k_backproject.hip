@@ -168,7 +168,7 @@ __device__ __forceinline__ void dma_span(__amdgpu_buffer_rsrc_t rs, float *dst, 
 // the scalar cache (its own restrict argument), so no vector-memory wait in
 // the compute phase drains the prefetch.  Blocks of grid row s > 0 take the
 // s-th share of `share` views and the s-th of the partial volumes (bp_splits).
-template <int KIND, int TZ, int WP, int HMAX>
+template <int KIND, int TZ, int WP, int HMAX, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 5) void k_bp_tiled(const float *__restrict__ proj, float *__restrict__ vol,
                                                        BpParams P, const int4 *__restrict__ foot,
                                                        const BpView *__restrict__ views,
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(kThreads, 5) void k_bp_tiled(const float *__restric
     // largest float below vmax: 0 <= v < vmax  <=>  med3(v, 0, vlast) == v
     const float vlast = __builtin_bit_cast(float, __builtin_bit_cast(int, P.vmax) - 1);
     const int4 *ft = foot + (size_t)tile * P.nb;
-    const int b0 = blockIdx.y * share, b1 = min(b0 + share, P.nb);
+    const int b0 = SPLIT ? blockIdx.y * share : 0, b1 = SPLIT ? min(b0 + share, P.nb) : P.nb;
 
     float acc[TZ];
 #pragma unroll
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(kThreads, 5) void k_bp_tiled(const float *__restric
     }
 
     if (!col_in) return;
-    vol += blockIdx.y * ((size_t)P.nt * P.ns * P.nz);
+    if (SPLIT) vol += blockIdx.y * ((size_t)P.nt * P.ns * P.nz);
 #pragma unroll
     for (int k = 0; k < TZ; ++k) {
         if (k < nzt) {
@@ -844,21 +844,29 @@ hipError_t launch_bp_footprints(const BpParams &Pin, const BpPlan &L, int4 *foot
     return hipGetLastError();
 }
 
-template <int KIND>
-static hipError_t launch_bp_kind(const BpParams &P, const BpPlan &L, const int4 *foot, const float *proj, float *vol,
+template <int KIND, bool SPLIT>
+static hipError_t launch_bp_sets(const BpParams &P, const BpPlan &L, const int4 *foot, const float *proj, float *vol,
                                  int share, hipStream_t st)
 {
     const dim3 grid(L.tiles_t * L.tiles_s * L.tiles_z, (P.nb + share - 1) / share);
     if (L.wp == 64)
-        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 64, 64>), grid, dim3(kThreads), 0, st, proj, vol, P, foot,
+        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 64, 64, SPLIT>), grid, dim3(kThreads), 0, st, proj, vol, P, foot,
                            P.views, P.zq, share);
     else if (L.wp == 72)
-        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 72, 56>), grid, dim3(kThreads), 0, st, proj, vol, P, foot,
+        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 72, 56, SPLIT>), grid, dim3(kThreads), 0, st, proj, vol, P, foot,
                            P.views, P.zq, share);
     else
-        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 80, 50>), grid, dim3(kThreads), 0, st, proj, vol, P, foot,
+        hipLaunchKernelGGL((k_bp_tiled<KIND, kBpTZ, 80, 50, SPLIT>), grid, dim3(kThreads), 0, st, proj, vol, P, foot,
                            P.views, P.zq, share);
     return hipGetLastError();
+}
+
+template <int KIND>
+static hipError_t launch_bp_kind(const BpParams &P, const BpPlan &L, const int4 *foot, const float *proj, float *vol,
+                                 int share, hipStream_t st)
+{
+    return share < P.nb ? launch_bp_sets<KIND, true>(P, L, foot, proj, vol, share, st)
+                        : launch_bp_sets<KIND, false>(P, L, foot, proj, vol, share, st);
 }
 
 // Views per set of blocks.  A tile is one block of four wavefronts and the chip
