@@ -880,23 +880,45 @@ static hipError_t launch_bp_kind(const BpParams &P, const BpPlan &L, const int4 
 // 64^3, 360 views 516 -> 61 us; 128^3, 180 views 263 -> 174 us; 176^3, 180
 // views 497 -> 378 us (2 sets 414); 176^3, 60 views 169 -> 148 us; 256^3, 360
 // views 2616 -> 2498 us; 256^3, 90 views 581 -> 606 us in two sets, so one.
+// Volumes of less than a round of blocks gain what their views cost above their
+// share of a full chip, 1.22 us less 1.52 ns a tile and view (0.45 us at least,
+// for the last blocks' sake); that has to pay for a launch and for the partial
+// volumes at 3.9 TB/s: 128^3, 20 views 29 us in one set, 38 in three; 40 views
+// 53 and 56; 60 views 77 and 73; 136^3, 28 views 44 and 53; 150^3, 40 views 75
+// and 83.
 constexpr double kBpSetsScale = 160.0;
 constexpr size_t kBpPartsBytes = (size_t)384 << 20;
 constexpr int kBpMinShare = 4;
-constexpr long kBpBlocks = 2560;
+constexpr long kBpBlocks = 2560, kBpRound = 1280;
 int bp_share(long tiles, int nb, size_t nvox)
 {
     const double best = std::sqrt(kBpSetsScale * nb / tiles);
     if (best < 2.3) return nb;
     const long splits = std::min(std::min(std::lround(best), std::max(4L, kBpBlocks / tiles)),
                                  std::min((long)(nb / kBpMinShare), (long)(kBpPartsBytes / (sizeof(float) * nvox))));
-    return splits > 1 ? (int)((nb + splits - 1) / splits) : nb;
+    if (splits <= 1) return nb;
+    if (tiles < kBpRound) {
+        const double gain = nb * std::max(1.22 - 1.52e-3 * tiles, 0.45);
+        if (gain < 7.0 + splits * (2 * sizeof(float)) * nvox / 3.9e6) return nb;
+    }
+    return (int)((nb + splits - 1) / splits);
+}
+
+// Views per set of blocks of a plan.  Tiles whose footprints exceed LDS read memory
+// all the time and gain nothing from company: 128^3, 60 views of 64 x 700 (61 rows
+// a tile, 50 staged) 317 us in one set, 392 in four.
+static int bp_set_share(const BpParams &P, const BpPlan &L)
+{
+    const int staged = L.wp == 64 ? 64 : (L.wp == 72 ? 56 : 50);
+    if (kBpTZ * P.rz * std::fabs(P.v_scale) > staged || 16.0 * std::hypot(P.rt, P.rs) * std::fabs(P.u_scale) > L.wp)
+        return P.nb;
+    return bp_share((long)L.tiles_t * L.tiles_s * L.tiles_z, P.nb, (size_t)P.nt * P.ns * P.nz);
 }
 
 int bp_splits(int kind, const BpParams &P, const BpPlan &L)
 {
     if (kind == kBpFdk && P.quirks) return 1;
-    const int share = bp_share((long)L.tiles_t * L.tiles_s * L.tiles_z, P.nb, (size_t)P.nt * P.ns * P.nz);
+    const int share = bp_set_share(P, L);
     return (P.nb + share - 1) / share;
 }
 
@@ -917,7 +939,7 @@ hipError_t launch_bp_tiled(int kind, const BpParams &Pin, const BpPlan &L, const
     P.tiles_s = L.tiles_s;
     P.tiles_z = L.tiles_z;
     const int splits = parts ? bp_splits(kind, P, L) : 1;
-    const int share = splits > 1 ? bp_share((long)L.tiles_t * L.tiles_s * L.tiles_z, P.nb, (size_t)P.nt * P.ns * P.nz) : P.nb;
+    const int share = splits > 1 ? bp_set_share(P, L) : P.nb;
     float *dst = splits > 1 ? parts : vol;
     if (splits > 1) P.accumulate = 0;
     const hipError_t e = kind == kBpFdk ? launch_bp_kind<kBpFdk>(P, L, foot, proj, dst, share, st)
@@ -975,12 +997,13 @@ hipError_t launch_adjoint(const BpParams &P, const BpPlan &L, const int4 *foot, 
 // Views per set of blocks of the adjoint.  The chip holds 1536 blocks (tiles of
 // 16 x 16 x 4), so a volume of few of them leaves CUs idle, and one of a few
 // thousand most of them in its last round: up to 16384 blocks in up to ten
-// sets, or as many sets as make 2560 blocks, of at least 4 views, and of 16
-// (32) where one set has 1024 (4096) tiles and more to write.  One set
+// sets, or as many sets as make 2560 blocks, of at least 4 views, and of 6
+// (16, 32) where one set has 512 (1024, 4096) tiles and more to write.  One set
 // against split: 32^3, 60 views 114 -> 18 us; 64^3, 120 views 236 -> 88 us;
 // 128^3, 120 views 581 -> 519 us; 150 x 130 x 101, 120 views 671 -> 562 us (3
 // sets 581); 176^3, 120 views 1268 -> 1223 us; 192^3, 40 views 579 -> 589 us in
-// two sets, and 162 x 139 x 109, 24 views 161 -> 168 us in five, so one there.
+// two sets, and 162 x 139 x 109, 24 views 161 -> 168 us in five, so one there;
+// 88^3, 8 views 28 -> 32 us in two, so one.
 // 64^3 in 32 sets 92 us, 96^3 in 18 sets 245 us against
 // 234 in nine.
 constexpr long kAdjBlocks = 16384, kAdjSets = 10;
@@ -988,7 +1011,7 @@ static int adjoint_share(const BpPlan &L, int nb)
 {
     const long tiles = (long)L.tiles_t * L.tiles_s * L.tiles_z;
     const long sets = std::min(kAdjBlocks / tiles, std::max(kAdjSets, kBpBlocks / tiles));
-    const long splits = std::min(sets, (long)(nb / (tiles >= 4096 ? 32 : (tiles >= 1024 ? 16 : kBpMinShare))));
+    const long splits = std::min(sets, (long)(nb / (tiles >= 4096 ? 32 : (tiles >= 1024 ? 16 : (tiles >= 512 ? 6 : kBpMinShare)))));
     return splits > 1 ? (int)((nb + splits - 1) / splits) : nb;
 }
 

@@ -72,3 +72,22 @@ def test_adjoint_of_slices_far_off_the_rows(ctx, oracle, nz, pitch):
     e, m = errs(vol, ref)
     report(f"thick_slices[{nz},{pitch}]", rel_l2=e, max_rel=m)
     assert e < 1e-4 and m < 1e-3
+
+
+@pytest.mark.parametrize("rows,columns", [(400, 40), (40, 400)])
+def test_backprojection_of_tall_and_wide_footprints(ctx, oracle, rows, columns):
+    """Footprints larger than LDS holds: all views in one set, from memory."""
+    import ctr
+    beta = (2 * np.pi / 40 * np.arange(40) + 0.1).astype(np.float32)
+    p, xi = (np.linspace(-1, 1, n).astype(np.float32) * np.float32(26.0) for n in (columns, rows))
+    a = (24, 21, 33, (24.0, 23.1, 29.7), 60.0, beta, p, xi)
+    g, og = ctr.ConeGeom(*a), oracle.Cone(*a)
+    y = np.random.default_rng(rows).random(g.nray).astype(np.float32)
+    print(f"[case] backprojection, 40 views of {rows} x {columns}", flush=True)
+    img = ctx.fdk_bp(g, y)
+    with oracle.interp_mode(1):
+        e, m = errs(img, oracle.fdk_bp(og, y))
+        e2, m2 = errs(ctx.cone_bp_ref(g, y), oracle.cone_bp_ref(og, y))
+    report(f"bp_beyond_lds[{rows}x{columns}]", rel_l2=e, max_rel=m, ref_rel_l2=e2, ref_max_rel=m2)
+    assert e < 3e-5 and m < 1e-4 and e2 < 3e-5 and m2 < 1e-4
+    np.testing.assert_array_equal(ctx.fdk_bp(g, y, out=img.copy(), flags=ctr.ACCUMULATE), img + img)
