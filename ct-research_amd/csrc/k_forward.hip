@@ -624,19 +624,21 @@ __device__ __forceinline__ float trace_ray_flat(const RayParams &g, int ib, int 
     const float near_end = __builtin_bit_cast(float, max(__builtin_bit_cast(int, lend) - 8, 0));
     const float lcnt = one_tail ? lend : near_end, most = one_tail ? (float)aA.n : inf;
     const int last = one_tail ? nD : -1;   // the slab that ends at the exit, whatever its plane's float parameter
-    unsigned off = idx0 * 4u;
-    float pA = A0, cA = 0.0f, s = 0.0f, sum = 0.0f;
     const float ninf = opaque_ninf();
-    float w1[kFlatUnroll], w2[kFlatUnroll], v1[kFlatUnroll], v2[kFlatUnroll];
-    unsigned o1[kFlatUnroll];
     int ubegin = 0, ulast = uend;
-    if (parts > 1) {
-        // this part's blocks of slabs, and the ray's state where they begin
+    if (parts > 1) {   // this part's blocks of slabs
         const int blocks = uend / kFlatUnroll + 1;
         ubegin = blocks * part / parts * kFlatUnroll;
         ulast = min(uend, blocks * (part + 1) / parts * kFlatUnroll - 1);
+    }
+    unsigned off;
+    float pA, cA, s, sum = 0.0f;
+    auto begin = [&]() {   // the ray's state at slab ubegin
+        off = idx0 * 4u;
+        pA = A0;
+        cA = s = 0.0f;
         const int k = ubegin - o;
-        if (go && k > 0 && k <= nD) {
+        if (parts > 1 && go && k > 0 && k <= nD) {
             s = min_nc(fmaf((float)(k - 1), dD, D0), lend, ninf);
             if (pA < s) {   // crossings before s: a guess, and its neighbours by the walk's own comparison
                 cA = fminf(fmaxf(ceilf((s - A0) / dA), 0.0f), (float)aA.n);
@@ -646,7 +648,10 @@ __device__ __forceinline__ float trace_ray_flat(const RayParams &g, int ib, int 
             pA = fmaf(cA, dA, A0);
             off += (unsigned)(int)cA * sA + (unsigned)k * sD;
         }
-    }
+    };
+    begin();
+    float w1[kFlatUnroll], w2[kFlatUnroll], v1[kFlatUnroll], v2[kFlatUnroll];
+    unsigned o1[kFlatUnroll];
     for (int u = ubegin; u <= ulast; u += kFlatUnroll) {
         const int k0 = u - o;
         const float kf = (float)k0;
@@ -714,6 +719,30 @@ __device__ __forceinline__ float trace_ray_flat(const RayParams &g, int ib, int 
                 if (w3[q] != 0.0f) sum = fmaf(w3[q], load_vox(rs, o3[q]), sum);
             }
         }
+    }
+    // the walk multiplies the pixels beside a ray by 0, and an infinite or NaN one
+    // makes a NaN of it: such a ray is walked again, its own pixels only
+    const bool again = !(fabsf(sum) < inf);
+    if (__ballot(again) != 0) {
+        begin();
+        float own = 0.0f;
+        for (int u = ubegin; u <= ulast; ++u) {
+            const int k = u - o;
+            if (!again || (unsigned)k > (unsigned)nD) continue;
+            const float plane = min_nc(fmaf((float)k, dD, D0), lend, ninf);
+            const float e = k == last ? lend : plane, ec = min_nc(e, lcnt, ninf);
+            const bool hasA = pA < ec && cA < most;
+            const float p1 = hasA ? pA : ec;
+            const unsigned next = off + (hasA ? sA : 0u);
+            if (p1 != s) own = fmaf(p1 - s, load_vox(rs, off), own);
+            if (ec != p1) own = fmaf(ec - p1, load_vox(rs, off + sA), own);
+            if (e != ec) own = fmaf(e - ec, load_vox(rs, next), own);
+            cA = hasA ? cA + 1.0f : cA;
+            pA = fmaf(cA, dA, A0);
+            off = next + sD;
+            s = e;
+        }
+        sum = again ? own : sum;
     }
     return sum;
 }

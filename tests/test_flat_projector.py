@@ -75,3 +75,32 @@ def test_projector_of_an_image_beyond_the_pair(ctx):
                     lo, hi = max(lo, u), min(hi, v)
             # 33000 segments telescope to the chord: their rounding, 2^-24 of up to 5 mm each
             assert abs(got[a, b] - (hi - lo)) < 1e-3
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("views,bins", [(20, 110), (400, 1100)])
+def test_flat_projector_of_a_pixel_that_is_not_finite(ctx, bad, views, bins):
+    """It reaches the rays that cross it, and those alone: the others have the bits
+    of the projection with a 0 in its place.  Few rays (split over wavefronts, the
+    image as it is) and many; both beams."""
+    import ctr
+    ang = 2 * np.pi / views * np.arange(1, views + 1) + 0.01
+    pos = 77.0 / bins * (np.arange(bins) - (bins - 1) / 2)
+    for n in ((48, 40), (150, 141)):
+        size = (48.0, 40.0)
+        for name, g, run in (("fan", ctr.FanGeom(*n, size, 80.0, ang, pos), ctx.fan_fp),
+                             ("parallel", ctr.ParGeom(*n, size, ang, pos), ctx.par_fp)):
+            img = np.random.default_rng(2).random(g.nvox).astype(np.float32)
+            for at in (0, 17 * n[0] + 22, n[0] * n[1] - 1):
+                print(f"[case] {name} {n} {views} x {bins}, {bad} at {at}", flush=True)
+                one = np.zeros(g.nvox, np.float32)
+                one[at] = 1.0
+                meets = run(g, one)
+                keep, img[at] = img[at], 0.0
+                clean = run(g, img)
+                img[at] = bad
+                got = run(g, img)
+                img[at] = keep
+                assert np.array_equal(got[meets == 0], clean[meets == 0])
+                hit = meets > 1e-3 * size[0] / n[0]
+                assert hit.any() and np.array_equal(got[hit], np.full(hit.sum(), bad, np.float32), equal_nan=True)
