@@ -770,12 +770,13 @@ __global__ __launch_bounds__(64 * kFlatWaves) void k_ray_fp_flat(float *__restri
 // same 64 rays each, and the shares are added in order.  A ray's walk is a chain
 // of gathers' latencies that nothing hides below a few wavefronts per SIMD.
 // Whole calls, a ray to one lane / split by 2 / 4 / 8 (pixels, views x bins):
-//    64^2,  90 x   96   17.8 / 11.0 / 10.2 / 10.4 us
-//   128^2, 180 x  192   29.1 / 20.8 / 17.6 / 16.3 us
-//   256^2, 360 x  512   50.2 / 50.2 / 47.1 / 57.4 us
-//   512^2, 360 x  730  125.6 / 105.8 / 99.7 / 113.3 us (4320 wavefronts of rays)
-//   512^2, 720 x 1024    156 / 191 / 231 / 285 us (11520)
-// 3 us of the first line are the image's transpose, left out up to 128^2 pixels.
+//    64^2,  90 x   96   15.8 /  9.2 /  9.1 /  9.2 us
+//   128^2, 180 x  192   24.5 / 16.8 / 14.6 / 14.1 us
+//   256^2, 360 x  512   41.3 / 51.0 / 48.7 / 58.8 us (2880 wavefronts of rays)
+//   512^2, 360 x  730  113.9 / 97.9 / 91.1 / 99.9 us (4320)
+//   512^2, 720 x 1024    267 /  263 /  267 /  297 us (11520)
+// 3 us of the first column's first line are the image's transpose, left out up
+// to 128^2 pixels.
 __global__ __launch_bounds__(64 * kFlatWaves) void k_ray_fp_flat_split(float *__restrict__ proj, RayParams g)
 {
     __shared__ float part[kFlatWaves][64];
